@@ -70,7 +70,7 @@ def listed():
         # a chunk of a prompt, or many sequences decoded together: too few rows to fill the chip
         dict(_linear(128, 8192, 8192, "fp8", "bf16", "kn"), name="linear_fp8_m128"),
         # a long prompt through the widest projection, one scale per token: the largest
-        dict(_linear(4096, 4096, 28672, "fp8", "bf16", "kn", "row"), name="linear_fp8_m4096"),
+        dict(_linear(2048, 8192, 28672, "fp8", "bf16", "kn", "row"), name="linear_fp8_m2048"),
         # decode of one sequence: streams the packed weights
         dict(_w4(1, 4096, 14336), name="w4_m1"),
         # decode of a batch of sequences
@@ -274,10 +274,35 @@ def _prepare_codec(case, g):
     return s
 
 
+def _encoder_weights(case, g):
+    """Float weights as int8 codes with a scale per column, biases, and the token ids."""
+    batch, seq, hidden, vocab = case["batch"], case["seq"], case["hidden"], 30522
+
+    def linear(n_in, n_out):
+        w = _normal(g, n_in, n_out, std=0.02)
+        sw = w.abs().amax(0) / 127.0
+        return _codes(w, "int8", sw), sw, _normal(g, n_out, std=0.02)
+
+    def norm():
+        return torch.rand(hidden, generator=g, device="cuda") * 0.2 + 0.9, _normal(g, hidden, std=0.02)
+
+    return {"words": _normal(g, vocab, hidden, std=0.02), "positions": _normal(g, seq, hidden, std=0.02),
+            "norm": norm(),
+            "layers": [{"q": linear(hidden, hidden), "k": linear(hidden, hidden), "v": linear(hidden, hidden),
+                        "o": linear(hidden, hidden), "norm1": norm(), "up": linear(hidden, 4 * hidden),
+                        "down": linear(4 * hidden, hidden), "norm2": norm()} for _ in range(case["layers"])],
+            "ids": torch.randint(0, vocab, (batch * seq,), generator=g, dtype=torch.int32, device="cuda")}
+
+
+# largest activation in front of each of an encoder layer's linears, as calibration leaves them
+_AMAX = {"x": 4.5, "context": 0.5, "up": 2.5}
+
+
 def _prepare_encoder(case, g):
-    batch, seq, hidden, heads, ffn, vocab = (case["batch"], case["seq"], case["hidden"], case["hidden"] // 64,
-                                             case["hidden"] * 4, 30522)
-    tokens, d = batch * seq, 64
+    batch, seq, hidden, heads, ffn, d = (case["batch"], case["seq"], case["hidden"], case["hidden"] // 64,
+                                         case["hidden"] * 4, 64)
+    tokens = batch * seq
+    weights = _encoder_weights(case, g)
     p = mgx.program()
     mm = p.get_main_module()
 
@@ -299,15 +324,14 @@ def _prepare_encoder(case, g):
     def scalar(v, lens):
         return over(lit(np.float32([v])), lens)
 
-    def layer_norm(x):
+    def layer_norm(x, norm):
         lens = [tokens, hidden]
         mean = over(op("reduce_mean", x, axes=[-1]), lens)
         xc = op("sub", x, mean)
         var = op("reduce_mean", op("mul", xc, xc), axes=[-1])
         rs = op("rsqrt", op("add", var, scalar(1e-5, [tokens, 1])))
         y = op("mul", xc, over(rs, lens))
-        y = op("mul", y, row(lit(host(torch.rand(hidden, generator=g, device="cuda") * 0.2 + 0.9)), lens))
-        return op("add", y, row(lit(host(_normal(g, hidden, std=0.02))), lens))
+        return op("add", op("mul", y, row(lit(host(norm[0])), lens)), row(lit(host(norm[1])), lens))
 
     def quantized(x, width, amax):
         s, z = lit(np.float32([amax / 127.0])), lit(np.int8([0]))
@@ -315,45 +339,43 @@ def _prepare_encoder(case, g):
         q = op("quantizelinear", x, over(s, lens), over(z, lens))
         return op("dequantizelinear", q, over(s, lens), over(z, lens))
 
-    def linear(x, n_in, n_out):
-        w = _normal(g, n_in, n_out, std=0.02)
-        sw = w.abs().amax(0) / 127.0
-        lens = [n_in, n_out]
-        w = op("dequantizelinear", lit(host(_codes(w, "int8", sw))), row(lit(host(sw)), lens),
-               row(lit(np.zeros(n_out, np.int8)), lens))
-        return op("add", op("dot", x, w), row(lit(host(_normal(g, n_out, std=0.02))), [tokens, n_out]))
+    def linear(x, wsb):
+        w, sw, bias = wsb
+        lens = list(w.shape)
+        w = op("dequantizelinear", lit(host(w)), row(lit(host(sw)), lens), row(lit(np.zeros(lens[1], np.int8)), lens))
+        return op("add", op("dot", x, w), row(lit(host(bias)), [tokens, lens[1]]))
 
     def split(x):
-        return op("contiguous", op("transpose", op("reshape", x, dims=[batch, seq, heads, d]), permutation=[0, 2, 1, 3]))
+        x = op("reshape", x, dims=[batch, seq, heads, d])
+        return op("contiguous", op("transpose", x, permutation=[0, 2, 1, 3]))
 
     def gelu(x, lens):
         e = op("erf", op("mul", x, scalar(math.sqrt(0.5), lens)))
         return op("mul", op("mul", x, scalar(0.5, lens)), op("add", e, scalar(1.0, lens)))
 
-    def layer(x):
+    def layer(x, w):
         lens = [tokens, hidden]
-        xin = quantized(x, hidden, 4.5)
-        q, k, v = (split(linear(xin, hidden, hidden)) for _ in range(3))
+        xin = quantized(x, hidden, _AMAX["x"])
+        q, k, v = (split(linear(xin, w[name])) for name in "qkv")
         scores = op("dot", q, op("transpose", k, permutation=[0, 1, 3, 2]))
         scores = op("mul", scores, scalar(1.0 / math.sqrt(d), [batch, heads, seq, seq]))
         ctx = op("dot", op("softmax", scores, axis=3), v)
         ctx = op("contiguous", op("transpose", ctx, permutation=[0, 2, 1, 3]))
-        att = linear(quantized(op("reshape", ctx, dims=lens), hidden, 0.5), hidden, hidden)
-        x = layer_norm(op("add", x, att))
-        h = gelu(linear(quantized(x, hidden, 4.5), hidden, ffn), [tokens, ffn])
-        return layer_norm(op("add", x, linear(quantized(h, ffn, 2.5), ffn, hidden)))
+        att = linear(quantized(op("reshape", ctx, dims=lens), hidden, _AMAX["context"]), w["o"])
+        x = layer_norm(op("add", x, att), w["norm1"])
+        h = gelu(linear(quantized(x, hidden, _AMAX["x"]), w["up"]), [tokens, ffn])
+        return layer_norm(op("add", x, linear(quantized(h, ffn, _AMAX["up"]), w["down"])), w["norm2"])
 
     ids = mm.add_parameter("ids", mgx.shape(type="int32_type", lens=[tokens]))
-    x = op("gather", lit(host(_normal(g, vocab, hidden, std=0.02))), ids, axis=0)
-    pos = over(lit(host(_normal(g, seq, hidden, std=0.02))), [batch, seq, hidden])
+    x = op("gather", lit(host(weights["words"])), ids, axis=0)
+    pos = over(lit(host(weights["positions"])), [batch, seq, hidden])
     x = op("reshape", op("add", op("reshape", x, dims=[batch, seq, hidden]), pos), dims=[tokens, hidden])
-    x = layer_norm(x)
-    for _ in range(case["layers"]):
-        x = layer(x)
+    x = layer_norm(x, weights["norm"])
+    for w in weights["layers"]:
+        x = layer(x, w)
     mm.add_return([x])
     p.compile(mgx.get_target("gpu"), offload_copy=False)
-    words = torch.randint(0, vocab, (tokens,), generator=g, dtype=torch.int32, device="cuda")
-    return {"case": case, "program": p, "parameters": {"ids": mgx.to_gpu(mgx.argument(host(words)))}}
+    return {"case": case, "program": p, "parameters": {"ids": mgx.to_gpu(mgx.argument(host(weights["ids"])))}}
 
 
 _PREPARE = {"linear": _prepare_linear, "w4": _prepare_w4, "attention": _prepare_attention, "conv": _prepare_conv,
@@ -428,6 +450,130 @@ def _run_encoder(s, case):
 
 _RUN = {"linear": _run_linear, "w4": _run_w4, "attention": _run_attention, "conv": _run_conv, "mx": _run_mx,
         "codec": _run_codec, "encoder": _run_encoder}
+
+
+# ---- the same in 64 bits ---------------------------------------------------------------------------------
+
+
+def exact(case, seed):
+    """What run() returns for these inputs, from plain torch in float64: the operands are the codes the operators
+    are defined by (a quantized activation is rounded where its operator rounds it), all sums and scales double."""
+    return _EXACT[case["kind"]](case, _generator(seed))
+
+
+def _toward_zero(x, dtype):
+    """float32 values cut to a 16-bit type's mantissa, as a quotient in that type is."""
+    cut = {torch.float32: 0, torch.float16: 13, torch.bfloat16: 16}[dtype]
+    return (x.view(torch.int32) >> cut << cut).view(torch.float32)
+
+
+def _quantize(x, scale, code, zp=0):
+    """quantizelinear's values (not their codes): of x's own type's quotient, and of a double one for fp8"""
+    v = x.double() / scale.double()
+    if code == "fp8":
+        return v.clamp_(-448, 448).float().to(torch.float8_e4m3fn).double()
+    lo, hi = {"int8": (-128, 127), "int4": (0, 15)}[code]
+    return _toward_zero(v.float(), x.dtype).double().round_().add_(zp).clamp_(lo, hi)
+
+
+def _values(codes, dtype):
+    """int8 or fp8 codes as doubles"""
+    return codes.double() if dtype == "int8" else codes.contiguous().view(torch.float8_e4m3fn).double()
+
+
+def _exact_linear(case, g):
+    s = _prepare_linear(case, g)
+    sx = s["sx"][:, None] if case["scale"] == "row" else s["sx"]
+    q = _quantize(s["x"], sx, case["dtype"], s["zp"]) - s["zp"]
+    w = _values(s["w"].t(), case["dtype"])
+    return torch.matmul(q, w.t()) * sx.double() * s["sw"].double() + s["bias"].double()
+
+
+def _exact_w4(case, g):
+    s = _prepare_w4(case, g)
+    w = torch.stack([s["w"] & 15, s["w"] >> 4], dim=2).reshape(case["n"], -1, case["group"]).double()
+    zp = s["zp"][:, :, None].double() if case["zero_points"] else 8
+    w = (w - zp).mul_(s["scales"][:, :, None].double()).reshape(case["n"], case["k"])
+    return torch.matmul(s["x"].double(), w.t())
+
+
+def _exact_attention(case, g):
+    s = _prepare_attention(case, g)
+    q, k, p, v = (_values(c, case["dtype"]) * sc.double() for c, sc in zip(s["codes"], s["scales"]))
+    return {"scores": torch.bmm(q, k.transpose(1, 2).contiguous()), "context": torch.bmm(p, v)}
+
+
+def _exact_conv(case, g):
+    s = _prepare_conv(case, g)
+    pad, st, out = case["window"] // 2, case["stride"], (case["hw"] + 2 * (case["window"] // 2) - case["window"]) // \
+        case["stride"] + 1
+    x = torch.nn.functional.pad(_values(s["x"], case["dtype"]), (pad,) * 4)
+    w = _values(s["w"], case["dtype"])
+    total = 0
+    for i in range(case["window"]):
+        for j in range(case["window"]):
+            tap = x[:, :, i:i + (out - 1) * st + 1:st, j:j + (out - 1) * st + 1:st]
+            if case["group"] > 1:  # depthwise
+                total = total + tap * w[:, 0, i, j][:, None, None]
+            else:
+                total = total + torch.matmul(w[:, :, i, j].contiguous(), tap.reshape(case["n"], case["c"], -1))
+    return total.reshape(case["n"], case["o"], out, out) * (s["sx"].double() * s["sw"].double())[:, None, None]
+
+
+def _exact_mx(case, g):
+    s = _prepare_mx(case, g)
+    fp4 = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6], dtype=torch.float64, device="cuda")
+    fp4 = torch.cat([fp4, -fp4])
+
+    def operand(codes, scales):
+        if case["dtype"] == "fp4":
+            v = fp4[torch.stack([codes & 15, codes >> 4], dim=2).long()].reshape(len(codes), -1)
+        else:
+            v = _values(codes, "fp8")
+        return v * scales.double().repeat_interleave(32, dim=1)
+
+    return torch.matmul(operand(s["a"], s["sa"]), operand(s["b"], s["sb"]).t())
+
+
+def _exact_codec(case, g):
+    s = _prepare_codec(case, g)
+    scale = s["scale"][:, None] if case["scale"] == "row" else s["scale"]
+    zp = 8 if case["code"] == "int4" else 0
+    return {"stored": None, "read": (_quantize(s["x"], scale, case["code"], zp) - zp) * scale.double()}
+
+
+def _exact_encoder(case, g):
+    batch, seq, hidden, heads = case["batch"], case["seq"], case["hidden"], case["hidden"] // 64
+    weights = _encoder_weights(case, g)
+
+    def layer_norm(x, norm):
+        x = x - x.mean(1, keepdim=True)
+        x = x * torch.rsqrt((x * x).mean(1, keepdim=True) + float(np.float32(1e-5)))
+        return x * norm[0].double() + norm[1].double()
+
+    def linear(x, amax, wsb):
+        scale = float(np.float32(amax / 127.0))
+        w, sw, bias = (t.double() for t in wsb)
+        return torch.matmul((x / scale).round().clamp(-128, 127), w) * (sw * scale) + bias
+
+    def split(x):
+        return x.reshape(batch, seq, heads, 64).transpose(1, 2).reshape(batch * heads, seq, 64)
+
+    x = weights["words"].double()[weights["ids"].long()].reshape(batch, seq, hidden) + weights["positions"].double()
+    x = layer_norm(x.reshape(batch * seq, hidden), weights["norm"])
+    for w in weights["layers"]:
+        q, k, v = (split(linear(x, _AMAX["x"], w[name])) for name in "qkv")
+        p = torch.softmax(torch.bmm(q, k.transpose(1, 2).contiguous()) / 8.0, dim=2)
+        context = torch.bmm(p, v).reshape(batch, heads, seq, 64).transpose(1, 2).reshape(batch * seq, hidden)
+        x = layer_norm(x + linear(context, _AMAX["context"], w["o"]), w["norm1"])
+        h = linear(x, _AMAX["x"], w["up"])
+        h = h * 0.5 * (torch.erf(h * math.sqrt(0.5)) + 1.0)
+        x = layer_norm(x + linear(h, _AMAX["up"], w["down"]), w["norm2"])
+    return x
+
+
+_EXACT = {"linear": _exact_linear, "w4": _exact_w4, "attention": _exact_attention, "conv": _exact_conv, "mx": _exact_mx,
+          "codec": _exact_codec, "encoder": _exact_encoder}
 
 
 # ---- what a pass cannot do without ---------------------------------------------------------------------------
