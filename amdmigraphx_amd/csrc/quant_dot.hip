@@ -1,6 +1,6 @@
 // mi355_quant_dot: argument checking, kernel selection, and the any-stride
-// kernel that serves the shapes the MFMA kernel's load pattern does not fit
-// (transposed A, K not a multiple of 16, odd leading dimensions, tiny cases).
+// kernel that serves what no matrix-core kernel takes (transposed A, uint8,
+// unaligned e5m2, K below 16 and the like).
 #include "common.h"
 #include <atomic>
 #include <mutex>
@@ -16,6 +16,18 @@ int mi355_mfma_gemm_launch(const mi355_quant_dot_desc*,
                            const int32_t*,
                            const float*,
                            hipStream_t);
+bool mi355_ragged_gemm_supported(const mi355_quant_dot_desc*);
+int mi355_ragged_gemm_launch(const mi355_quant_dot_desc*,
+                             const void*,
+                             const void*,
+                             void*,
+                             const float*,
+                             const float*,
+                             const int32_t*,
+                             const int32_t*,
+                             const float*,
+                             bool,
+                             hipStream_t);
 bool mi355_dma_gemm_supported(const mi355_quant_dot_desc*, const void*, const void*);
 int mi355_dma_gemm_launch(const mi355_quant_dot_desc*,
                           const void*,
@@ -318,6 +330,9 @@ extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
         return MI355_ERR_UNSUPPORTED;
     if(!u8 && d->k > 0 && mi355_mfma_gemm_supported(d, a, b, c))
         return mi355_mfma_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, s);
+    // rows aligned to nothing; fp8 sums stay exact there, as in the kernel below
+    if(mi355_ragged_gemm_supported(d))
+        return mi355_ragged_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, false, s);
 
     generic_params p;
     p.a            = static_cast<const uint8_t*>(a);
