@@ -19,17 +19,22 @@ MI355_DEVINL float load_x(const void* x, int64_t i)
         return bf16_to_f32(static_cast<const uint16_t*>(x)[i]);
 }
 
-// x / s evaluated in x's own type (generic_float's operator/ converts the float
+// a quotient in x's own type (generic_float's operator/ converts the float
 // quotient back to the narrow type, generic_float.hpp:318-326)
 template <int XT>
-MI355_DEVINL float div_in_type(float x, float s)
+MI355_DEVINL float in_type(float d)
 {
-    float d = x / s;
     if constexpr(XT == MI355_F16)
         d = half_to_f32(f32_to_half_rtz(d));
     else if constexpr(XT == MI355_BF16)
         d = bf16_to_f32(f32_to_bf16_rtz(d));
     return d;
+}
+
+template <int XT>
+MI355_DEVINL float div_in_type(float x, float s)
+{
+    return in_type<XT>(x / s);
 }
 
 struct qparams
@@ -100,36 +105,283 @@ __global__ __launch_bounds__(PW_THREADS) void quantizelinear_kernel(
             o[e] = res[e];
 }
 
-// fp32 -> int8 with one scale and one zero point for the whole tensor (activations): 16 elements
-// per thread as four 16-byte loads and one 16-byte store, the same arithmetic as above.  n16 is
-// the element count / 16; x and out are 16-byte aligned.
-__global__ __launch_bounds__(PW_THREADS) void quantize_f32_i8_tensor_kernel(
-    const v4f* x, const float* scale, const int8_t* zp, uint4* out, int64_t n16)
+// ---- runs of 16 elements -------------------------------------------------------------------------
+// What bounds both operators is memory: the kernels below move 16 consecutive elements of one row
+// per thread, 16 bytes a load or store, at whatever address the row has (a global load of 16 bytes
+// takes any).  Everything an element used to pay for by itself is gone:
+// the 64-bit division that finds its row (a multiplication by the reciprocal here, once per run), the
+// loads of scale and zero point (once per run where they don't vary along the row, else as a vector),
+// and arithmetic in double where float provably gives the same bits:
+//   x / s       rounding the double quotient of two floats to float is the float quotient (53 bits are
+//               more than twice 24 and two), and what overflows saturates on both ways;
+//   rint + zp   whole numbers below 2^24, or saturated;
+//   (x - zp) s  the difference of two 8-bit values, fp8 e4m3fn's 2^-9 ... 896 included, is exact in
+//               float, so is the double product: one rounding to float either way.
+// Left to the kernels of any strides: strides along the row other than 0 and 1, e5m2 (whose zero
+// points cost more than 24 bits), fp8 quantization with a zero point (the sum is rounded as a
+// double there), int32 and float32 inputs of dequantizelinear, 2^31 runs and beyond.
+// Measured, [8192, 1024] bfloat16 with a scale per row: to uint8 14.3 -> 7.5 us, back
+// from uint8 with zero points 28 -> 7.0 us; [2048, 8192] bfloat16 to fp8
+// 30 -> 13 us (50 MB).
+
+constexpr int RUN = 16;
+
+struct run_params
 {
-    const float sv = scale[0];
-    const double z = zp != nullptr ? (double)zp[0] : 0.0;
-    const int64_t step = (int64_t)gridDim.x * PW_THREADS;
-    for(int64_t i = (int64_t)blockIdx.x * PW_THREADS + threadIdx.x; i < n16; i += step)
+    const void* x;
+    void* out;
+    qparams q;
+    int64_t cols;
+    uint32_t runs;     // in all
+    uint32_t per_row;  // runs of a row, the last of which may be short
+    uint32_t magic;    // run / per_row = (run * magic) >> shift for run < 2^31
+    uint32_t shift;
+};
+
+// consecutive elements at any address
+template <class T, int N = RUN>
+struct __attribute__((packed, aligned(1))) run_of
+{
+    T v[N];
+};
+
+template <int N = RUN, class T>
+MI355_DEVINL run_of<T, N> load_run(const T* p)
+{
+    return *reinterpret_cast<const run_of<T, N>*>(p);
+}
+
+template <class T, int N>
+MI355_DEVINL void store_run(T* p, const run_of<T, N>& r)
+{
+    *reinterpret_cast<run_of<T, N>*>(p) = r;
+}
+
+// N float32 / float16 / bfloat16 values, or 8-bit codes, as floats
+template <int T, int N>
+MI355_DEVINL void load_f32(float (&f)[N], const void* p, int64_t i)
+{
+    if constexpr(T == MI355_F32)
     {
-        v4f v[4];
+        const auto r = load_run<N>(static_cast<const float*>(p) + i);
 #pragma unroll
-        for(int j = 0; j < 4; j++)
-            v[j] = x[4 * i + j];
-        uint32_t w[4];
+        for(int e = 0; e < N; e++)
+            f[e] = r.v[e];
+    }
+    else if constexpr(T == MI355_F16 || T == MI355_BF16)
+    {
+        const auto r = load_run<N>(static_cast<const uint16_t*>(p) + i);
 #pragma unroll
-        for(int j = 0; j < 4; j++)
+        for(int e = 0; e < N; e++)
+            f[e] = T == MI355_F16 ? half_to_f32(r.v[e]) : bf16_to_f32(r.v[e]);
+    }
+    else
+    {
+        const auto r = load_run<N>(static_cast<const uint8_t*>(p) + i);
+#pragma unroll
+        for(int e = 0; e < N; e++)
+            f[e] = T == MI355_I8 ? (float)(int8_t)r.v[e] : T == MI355_U8 ? (float)r.v[e] : fp8_to_f32(r.v[e]);
+    }
+}
+
+// the scales (or zero points) of N elements: one for all of them, or their own
+template <int T, int N>
+MI355_DEVINL void load_param(float (&f)[N], const void* p, int64_t i, int64_t stride)
+{
+    if(stride == 0)
+    {
+        float one[1];
+        load_f32<T>(one, p, i);
+#pragma unroll
+        for(int e = 0; e < N; e++)
+            f[e] = one[0];
+    }
+    else
+        load_f32<T>(f, p, i);
+}
+
+MI355_DEVINL float clamp_like_ref_f32(float q, float lo, float hi)
+{
+    const float v = (q < hi) ? q : hi;
+    return (lo < v) ? v : lo;
+}
+
+// The correctly rounded quotient of x by one s from its correctly rounded reciprocal: each of the
+// two steps adds what the exact remainder says is missing, the first leaves a quotient within one
+// unit of its last place, the second the nearest (P. Markstein, "Computation of elementary functions
+// on the IBM RISC System/6000 processor", 1990).  Five instructions in place of a division's eleven.
+// No step overflows for 2^-60 <= |s| <= 2^60 and |x| <= 2^60.  Bits lost below the normal range
+// belong to quotients under 2^-40: the 8-bit code is zero with or without them, with the quotient's
+// sign (of x = 0 alone the sign may be lost).
+MI355_DEVINL bool reciprocal_serves(float s)
+{
+    return __builtin_fabsf(s) >= 0x1p-60f && __builtin_fabsf(s) <= 0x1p60f;
+}
+
+MI355_DEVINL float div_by_reciprocal(float x, float s, float rs)
+{
+    float q = x * rs;
+    q       = __builtin_fmaf(__builtin_fmaf(-q, s, x), rs, q);
+    return __builtin_fmaf(__builtin_fmaf(-q, s, x), rs, q);
+}
+
+template <int XT, int OT, int N>
+MI355_DEVINL void quantize_elements(const run_params& p, int64_t r, int64_t c)
+{
+    float x[N], s[N], z[N] = {};
+    load_param<XT>(s, p.q.scale, r * p.q.s_sr + c * p.q.s_sc, p.q.s_sc);
+    if constexpr(OT != MI355_FP8)
+        if(p.q.zp != nullptr)
+            load_param<OT>(z, p.q.zp, r * p.q.z_sr + c * p.q.z_sc, p.q.z_sc);
+    load_f32<XT>(x, p.x, r * p.cols + c);
+    // the quotients: where one scale serves all, so does its reciprocal
+    float q[N];
+    uint32_t most = 0; // of the magnitudes' bits, which order like the magnitudes, NaN on top
+#pragma unroll
+    for(int e = 0; e < N; e++)
+        most = max(most, __builtin_bit_cast(uint32_t, x[e]) & 0x7fffffffu);
+    const bool serves = p.q.s_sc == 0 && reciprocal_serves(s[0]) && most <= 0x5d800000u; // 2^60
+    if(N > 1 && serves)
+    {
+        const float rs = 1.f / s[0];
+#pragma unroll
+        for(int e = 0; e < N; e++)
+            q[e] = div_by_reciprocal(x[e], s[0], rs);
+    }
+    else
+    {
+#pragma unroll
+        for(int e = 0; e < N; e++)
+            q[e] = x[e] / s[e];
+    }
+#pragma unroll
+    for(int e = 0; e < N; e++)
+    {
+        if constexpr(OT == MI355_FP8)
         {
-            w[j] = 0;
+            // the double sum with no zero point turns an exact -0 into +0, but no tiny negative quotient
+            const float zero = x[e] == 0.f || __builtin_isinf(s[e]) ? 0.f : -0.f;
+            q[e]             = clamp_like_ref_f32(q[e] + zero, -448.f, 448.f);
+        }
+        else
+        {
+            const float lo = OT == MI355_I8 ? -128.f : 0.f;
+            q[e]           = clamp_like_ref_f32(rintf(in_type<XT>(q[e])) + z[e], lo, lo + 255.f);
+        }
+    }
+    uint8_t* out = static_cast<uint8_t*>(p.out) + r * p.cols + c;
+    if constexpr(N % 4 == 0)
+    {
+        uint32_t w[N / 4];
 #pragma unroll
-            for(int e = 0; e < 4; e++)
+        for(int h = 0; h < N / 4; h++)
+        {
+            if constexpr(OT == MI355_FP8)
             {
-                const double qv = (double)rintf(v[j][e] / sv) + z;
-                const uint32_t b = (uint8_t)(int8_t)(int)clamp_like_ref(qv, -128.0, 127.0);
-                w[j] |= b << (8 * e);
+                w[h] = __builtin_amdgcn_cvt_pk_fp8_f32(q[4 * h], q[4 * h + 1], 0, false);
+                w[h] = __builtin_amdgcn_cvt_pk_fp8_f32(q[4 * h + 2], q[4 * h + 3], w[h], true);
+            }
+            else
+            {
+                // an int8 code is its value + 128 with the top bit flipped
+                w[h] = 0;
+#pragma unroll
+                for(int e = 0; e < 4; e++)
+                    w[h] = __builtin_amdgcn_cvt_pk_u8_f32(OT == MI355_I8 ? q[4 * h + e] + 128.f : q[4 * h + e], e, w[h]);
+                if constexpr(OT == MI355_I8)
+                    w[h] ^= 0x80808080u;
             }
         }
-        out[i] = make_uint4(w[0], w[1], w[2], w[3]);
+        store_run(out, __builtin_bit_cast(run_of<uint8_t, N>, w));
     }
+    else
+    {
+#pragma unroll
+        for(int e = 0; e < N; e++)
+            out[e] = OT == MI355_FP8 ? f32_to_fp8_rne(q[e]) : (uint8_t)(int)q[e];
+    }
+}
+
+template <int XT, int ST, int N>
+MI355_DEVINL void dequantize_elements(const run_params& p, int64_t r, int64_t c)
+{
+    float x[N], s[N], z[N] = {};
+    load_param<ST>(s, p.q.scale, r * p.q.s_sr + c * p.q.s_sc, p.q.s_sc);
+    if(p.q.zp != nullptr)
+        load_param<XT>(z, p.q.zp, r * p.q.z_sr + c * p.q.z_sc, p.q.z_sc);
+    const int64_t i = r * p.cols + c;
+    load_f32<XT>(x, p.x, i);
+#pragma unroll
+    for(int e = 0; e < N; e++)
+        x[e] = (x[e] - z[e]) * s[e];
+    if constexpr(ST == MI355_F32)
+        store_run(static_cast<float*>(p.out) + i, __builtin_bit_cast(run_of<float, N>, x));
+    else
+    {
+        run_of<uint16_t, N> res;
+#pragma unroll
+        for(int e = 0; e < N; e++)
+            res.v[e] = ST == MI355_F16 ? f32_to_half_rtz(x[e]) : f32_to_bf16_rtz(x[e]);
+        store_run(static_cast<uint16_t*>(p.out) + i, res);
+    }
+}
+
+// QUANTIZE: IN a float type, OUT a code's; else the other way
+template <bool QUANTIZE, int IN, int OUT>
+__global__ __launch_bounds__(PW_THREADS) void run_kernel(run_params p)
+{
+    const uint32_t run = blockIdx.x * PW_THREADS + threadIdx.x;
+    if(run >= p.runs)
+        return;
+    const uint32_t r = (uint32_t)(((uint64_t)run * p.magic) >> p.shift);
+    int64_t c        = (int64_t)(run - r * p.per_row) * RUN;
+    if(p.cols - c >= RUN)
+    {
+        if constexpr(QUANTIZE)
+            quantize_elements<IN, OUT, RUN>(p, r, c);
+        else
+            dequantize_elements<IN, OUT, RUN>(p, r, c);
+    }
+    else
+        for(; c < p.cols; c++) // the end of a row
+        {
+            if constexpr(QUANTIZE)
+                quantize_elements<IN, OUT, 1>(p, r, c);
+            else
+                dequantize_elements<IN, OUT, 1>(p, r, c);
+        }
+}
+
+// Strides along the row of 0 and 1 only; rows that are one vector for the parameters as well become
+// one long row.  False where the kernels of any strides have to take the call.
+bool run_plan(run_params& p, const void* x, const qparams& q, void* out, int64_t rows, int64_t cols)
+{
+    const bool has_zp = q.zp != nullptr;
+    if(q.s_sc < 0 || q.s_sc > 1 || (has_zp && (q.z_sc < 0 || q.z_sc > 1)))
+        return false;
+    // element i of the tensor has parameter i (a full tensor of them), or the one there is
+    auto flat = [&](int64_t sr, int64_t sc) { return sr == sc * cols; };
+    if(flat(q.s_sr, q.s_sc) && (!has_zp || flat(q.z_sr, q.z_sc)))
+    {
+        cols *= rows;
+        rows = 1;
+    }
+    const int64_t per_row = (cols + RUN - 1) / RUN;
+    if(per_row > 0x7fffffff || rows > 0x7fffffff / per_row)
+        return false;
+    p.x       = x;
+    p.out     = out;
+    p.q       = q;
+    p.cols    = cols;
+    p.per_row = (uint32_t)per_row;
+    p.runs    = (uint32_t)(rows * per_row);
+    // ceil(2^(31 + l) / d) with 2^l >= d is exact for every numerator below 2^31; it fits 32 bits
+    uint32_t l = 0;
+    while(((uint64_t)1 << l) < p.per_row)
+        l++;
+    p.shift = 31 + l;
+    p.magic = (uint32_t)((((uint64_t)1 << p.shift) + p.per_row - 1) / p.per_row);
+    return true;
 }
 
 __global__ __launch_bounds__(PW_THREADS) void dequantizelinear_kernel(const void* x,
@@ -161,7 +413,8 @@ __global__ __launch_bounds__(PW_THREADS) void dequantizelinear_kernel(const void
         static_cast<uint16_t*>(out)[i] = f32_to_bf16_rtz(f);
 }
 
-// one packed byte -> two bytes; 8 packed bytes per thread where aligned
+// one packed byte -> two bytes: 8 packed bytes per thread, one load and one 16-byte store at any
+// address, four codes a register ([8192, 512] packed: 10.9 -> 3.7 us)
 __global__ __launch_bounds__(PW_THREADS) void unpack_int4_kernel(
     const uint8_t* in, uint8_t* out, int is_signed, int64_t total)
 {
@@ -169,22 +422,36 @@ __global__ __launch_bounds__(PW_THREADS) void unpack_int4_kernel(
     if(i0 >= total)
         return;
     const int cnt = (int)min((int64_t)8, total - i0);
-    for(int e = 0; e < cnt; e++)
+    uint64_t v = 0;
+    if(cnt == 8)
+        v = __builtin_bit_cast(uint64_t, load_run<8>(in + i0));
+    else
+        for(int e = 0; e < cnt; e++)
+            v |= (uint64_t)in[i0 + e] << (8 * e);
+    uint32_t w[4];
+#pragma unroll
+    for(int h = 0; h < 2; h++)
     {
-        uint8_t v = in[i0 + e];
-        uint8_t lo, hi;
+        const uint32_t b = (uint32_t)(v >> (32 * h));
+        uint32_t lo = b & 0x0f0f0f0fu, hi = (b >> 4) & 0x0f0f0f0fu;
         if(is_signed)
         {
-            lo = (uint8_t)((int8_t)(uint8_t)(v << 4) >> 4);
-            hi = (uint8_t)((int8_t)v >> 4);
+            // bit 3 of a code into the four above it: 8 * 30 = 0xf0, no carry leaves its byte
+            lo |= (lo & 0x08080808u) * 30u;
+            hi |= (hi & 0x08080808u) * 30u;
         }
-        else
-        {
-            lo = v & 0xf;
-            hi = v >> 4;
-        }
-        out[2 * (i0 + e)]     = lo;
-        out[2 * (i0 + e) + 1] = hi;
+        // low nibble first: bytes 0 to 3 of a selector are lo's, 4 to 7 hi's
+        w[2 * h]     = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
+        w[2 * h + 1] = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
+    }
+    if(cnt == 8)
+        store_run(out + 2 * i0, __builtin_bit_cast(run_of<uint8_t, 16>, w));
+    else
+    {
+#pragma unroll
+        for(int e = 0; e < 16; e++)
+            if(e < 2 * cnt)
+                out[2 * i0 + e] = (uint8_t)(w[e >> 2] >> (8 * (e & 3)));
     }
 }
 
@@ -243,27 +510,40 @@ __global__ __launch_bounds__(PW_THREADS) void pack_fp4_kernel(const float* in, u
     out[i] = (uint8_t)((f32_to_fp4(in[2 * i + 1]) << 4) | f32_to_fp4(in[2 * i]));
 }
 
+// two bytes -> one packed byte: 16 bytes per thread, one load and one 8-byte store at any address
+// ([8192, 1024] bytes: 7.9 -> 3.4 us)
 __global__ __launch_bounds__(PW_THREADS) void pack_int4_kernel(
     const uint8_t* in, uint8_t* out, int is_signed, int64_t total_out)
 {
-    const int64_t i = (int64_t)blockIdx.x * PW_THREADS + threadIdx.x;
-    if(i >= total_out)
+    const int64_t i0 = ((int64_t)blockIdx.x * PW_THREADS + threadIdx.x) * 8;
+    if(i0 >= total_out)
         return;
-    uint8_t u1, u2;
-    if(is_signed)
+    auto packed = [&](uint32_t two) {
+        int u1 = (int)(two & 0xff), u2 = (int)(two >> 8);
+        if(is_signed)
+        {
+            u1 = max(-8, min(7, (int)(int8_t)u1));
+            u2 = max(-8, min(7, (int)(int8_t)u2));
+        }
+        else
+        {
+            u1 = min(u1, 15);
+            u2 = min(u2, 15);
+        }
+        return (uint8_t)((u2 << 4) | (u1 & 0xf));
+    };
+    if(total_out - i0 >= 8)
     {
-        int v1 = (int8_t)in[2 * i], v2 = (int8_t)in[2 * i + 1];
-        v1 = max(-8, min(7, v1));
-        v2 = max(-8, min(7, v2));
-        u1 = (uint8_t)v1;
-        u2 = (uint8_t)v2;
+        const auto v = load_run<8>(reinterpret_cast<const uint16_t*>(in) + i0);
+        run_of<uint8_t, 8> res;
+#pragma unroll
+        for(int e = 0; e < 8; e++)
+            res.v[e] = packed(v.v[e]);
+        store_run(out + i0, res);
     }
     else
-    {
-        u1 = min((int)in[2 * i], 15);
-        u2 = min((int)in[2 * i + 1], 15);
-    }
-    out[i] = (uint8_t)((u2 << 4) | (u1 & 0xf));
+        for(int64_t i = i0; i < total_out; i++)
+            out[i] = packed(in[2 * i] | ((uint32_t)in[2 * i + 1] << 8));
 }
 
 __global__ __launch_bounds__(PW_THREADS) void convert_kernel(
@@ -323,6 +603,19 @@ int launch_quantize(int out_type,
                     int64_t cols,
                     hipStream_t s)
 {
+    run_params p;
+    if((out_type == MI355_I8 || out_type == MI355_U8 || (out_type == MI355_FP8 && q.zp == nullptr)) &&
+       run_plan(p, x, q, out, rows, cols))
+    {
+        const dim3 grid(blocks_for(p.runs));
+        if(out_type == MI355_I8)
+            hipLaunchKernelGGL((run_kernel<true, XT, MI355_I8>), grid, dim3(PW_THREADS), 0, s, p);
+        else if(out_type == MI355_U8)
+            hipLaunchKernelGGL((run_kernel<true, XT, MI355_U8>), grid, dim3(PW_THREADS), 0, s, p);
+        else
+            hipLaunchKernelGGL((run_kernel<true, XT, MI355_FP8>), grid, dim3(PW_THREADS), 0, s, p);
+        return mi355_launch_status();
+    }
     const int64_t work = rows * ((cols + 3) / 4);
     switch(out_type)
     {
@@ -345,6 +638,18 @@ int launch_quantize(int out_type,
     default: return MI355_ERR_UNSUPPORTED;
     }
     return mi355_launch_status();
+}
+
+template <int XT>
+void launch_dequantize_runs(int s_type, const run_params& p, hipStream_t s)
+{
+    const dim3 grid(blocks_for(p.runs));
+    if(s_type == MI355_F32)
+        hipLaunchKernelGGL((run_kernel<false, XT, MI355_F32>), grid, dim3(PW_THREADS), 0, s, p);
+    else if(s_type == MI355_F16)
+        hipLaunchKernelGGL((run_kernel<false, XT, MI355_F16>), grid, dim3(PW_THREADS), 0, s, p);
+    else
+        hipLaunchKernelGGL((run_kernel<false, XT, MI355_BF16>), grid, dim3(PW_THREADS), 0, s, p);
 }
 
 } // namespace
@@ -371,20 +676,6 @@ extern "C" int mi355_quantizelinear(const void* x,
         return MI355_ERR_UNSUPPORTED;
     qparams q{scale, scale_stride_r, scale_stride_c, zp, zp_stride_r, zp_stride_c};
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int64_t total = rows * cols;
-    if(x_type == MI355_F32 && out_type == MI355_I8 && scale_stride_r == 0 && scale_stride_c == 0 &&
-       (zp == nullptr || (zp_stride_r == 0 && zp_stride_c == 0)) && total % 16 == 0 &&
-       reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0)
-    {
-        const int64_t n16 = total / 16;
-        int64_t blocks    = (n16 + PW_THREADS - 1) / PW_THREADS;
-        if(blocks > 256 * 32)
-            blocks = 256 * 32;
-        hipLaunchKernelGGL(quantize_f32_i8_tensor_kernel, dim3((unsigned)blocks), dim3(PW_THREADS), 0, s,
-                           static_cast<const v4f*>(x), static_cast<const float*>(scale),
-                           static_cast<const int8_t*>(zp), static_cast<uint4*>(out), n16);
-        return mi355_launch_status();
-    }
     switch(x_type)
     {
     case MI355_F32: return launch_quantize<MI355_F32>(out_type, x, q, out, rows, cols, s);
@@ -418,6 +709,18 @@ extern "C" int mi355_dequantizelinear(const void* x,
     if(rows == 0 || cols == 0)
         return MI355_OK;
     qparams q{scale, scale_stride_r, scale_stride_c, zp, zp_stride_r, zp_stride_c};
+    run_params p;
+    if((x_type == MI355_I8 || x_type == MI355_U8 || x_type == MI355_FP8) && run_plan(p, x, q, out, rows, cols))
+    {
+        hipStream_t s = static_cast<hipStream_t>(stream);
+        if(x_type == MI355_I8)
+            launch_dequantize_runs<MI355_I8>(scale_type, p, s);
+        else if(x_type == MI355_U8)
+            launch_dequantize_runs<MI355_U8>(scale_type, p, s);
+        else
+            launch_dequantize_runs<MI355_FP8>(scale_type, p, s);
+        return mi355_launch_status();
+    }
     hipLaunchKernelGGL(dequantizelinear_kernel, dim3(blocks_for(rows * cols)), dim3(PW_THREADS), 0,
                        static_cast<hipStream_t>(stream), x, x_type, q, scale_type, out, rows, cols);
     return mi355_launch_status();
@@ -447,7 +750,7 @@ extern "C" int mi355_pack_int4(
     const int64_t total_out = rows * (cols / 2);
     if(total_out == 0)
         return MI355_OK;
-    hipLaunchKernelGGL(pack_int4_kernel, dim3(blocks_for(total_out)), dim3(PW_THREADS), 0,
+    hipLaunchKernelGGL(pack_int4_kernel, dim3(blocks_for((total_out + 7) / 8)), dim3(PW_THREADS), 0,
                        static_cast<hipStream_t>(stream), static_cast<const uint8_t*>(in),
                        static_cast<uint8_t*>(out), is_signed, total_out);
     return mi355_launch_status();
