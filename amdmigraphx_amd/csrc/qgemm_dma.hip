@@ -2456,9 +2456,15 @@ int launch_i8_out(const dma_params& p, int batch, bool deq, int out, hipStream_t
 // p.vec_store); VEC8: 16-bit outputs in groups of 8 (p.vec8_store).  The way C is stored is fixed at
 // compile time: with both ways behind a run-time branch the compiler keeps the accumulators in
 // scratch memory across the epilogue.
-template <bool TRANS_B, bool DEQ, int OUT, bool VEC8>
+// HALF: operands of float16, B as [N, K], K counted in bytes.  A half product of a slab costs the matrix
+// cores what an fp8 one does (32 halves at half the rate of 64 codes), so loads, stages and waits stay
+// as they are: the 32 bytes of a lane are two chunks of 8 halves, one v_mfma_f32_32x32x16_f16 of 32
+// cycles each.  The two MFMAs of a tile are four apart, behind the first halves of a row's four tiles.
+template <bool TRANS_B, bool DEQ, int OUT, bool VEC8, bool HALF = false>
 __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_f8_kernel(dma_params p)
 {
+    static_assert(!HALF || (TRANS_B && (DEQ ? OUT == MI355_F16 && VEC8 : OUT == MI355_F32)),
+                  "half operands: half results or bare float sums, B as [N, K]");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
     const int tid    = threadIdx.x;
@@ -2624,10 +2630,23 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_f8_kernel(dma_params p)
     // loop nothing reads an accumulator.  In the last slabs, whose loads and reads are conditional,
     // the compiler keeps copies of the accumulators in scratch memory and stores them right behind
     // the MFMA, so there the statement carries the wait states itself.
+// (HALF: chunk X of the operands)
+#define CHUNK(frag, X) __builtin_shufflevector(frag, frag, 4 * (X), 4 * (X) + 1, 4 * (X) + 2, 4 * (X) + 3)
+#define MFH(Q, I, J, X)                                                                    \
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0"                                  \
+                 : "+a"(acc[I][J])                                                         \
+                 : "v"(CHUNK(fb[Q][J], X)), "v"(CHUNK(fa[Q][I], X)))
 #define MF(Q, I, J)                                                                        \
     do                                                                                     \
     {                                                                                      \
-        if constexpr(fast_)                                                                \
+        if constexpr(HALF)                                                                 \
+        {                                                                                  \
+            MFH(Q, I, J, 0);                                                               \
+            MFH(Q, I, J, 1);                                                               \
+            if constexpr(!fast_)                                                           \
+                asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+a"(acc[I][J]));           \
+        }                                                                                  \
+        else if constexpr(fast_)                                                           \
             asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0"                       \
                          : "+a"(acc[I][J])                                                 \
                          : "v"(fb[Q][J]), "v"(fa[Q][I]));                                  \
@@ -2760,6 +2779,49 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_f8_kernel(dma_params p)
     asm volatile("v_mfma_f32_32x32x64_f8f6f4 %0, %1, %2, %0"                                    \
                  : "+a"(acc[I][J])                                                              \
                  : "v"(fb[Q][J]), "v"(fa[Q][I]))
+    // HALF: 8 MFMAs in a row of tiles, a read behind each (8 of the slab's 16)
+#define ROWH12_READS(U, Q, I, N0)                                                               \
+    do                                                                                          \
+    {                                                                                           \
+        SB(); MFH(Q, I, 0, 0); SB(); READ12(U, Q, (N0) + 0);                                    \
+        SB(); MFH(Q, I, 1, 0); SB(); READ12(U, Q, (N0) + 1);                                    \
+        SB(); MFH(Q, I, 2, 0); SB(); READ12(U, Q, (N0) + 2);                                    \
+        SB(); MFH(Q, I, 3, 0); SB(); READ12(U, Q, (N0) + 3);                                    \
+        SB(); MFH(Q, I, 0, 1); SB(); READ12(U, Q, (N0) + 4);                                    \
+        SB(); MFH(Q, I, 1, 1); SB(); READ12(U, Q, (N0) + 5);                                    \
+        SB(); MFH(Q, I, 2, 1); SB(); READ12(U, Q, (N0) + 6);                                    \
+        SB(); MFH(Q, I, 3, 1); SB(); READ12(U, Q, (N0) + 7);                                    \
+    } while(0)
+#define MFH8_LOAD4(Q, I, LDS_CONST, OFF0, OFF1, OFF2, OFF3, BASE)                               \
+    asm volatile("s_add_i32 m0, %[wl], %[lc0]\n\t"                                              \
+                 "v_mfma_f32_32x32x16_f16 %[c0], %[b0], %[a0], %[c0]\n\t"                       \
+                 "global_load_lds_dwordx4 %[o0], %[base]\n\t"                                   \
+                 "v_mfma_f32_32x32x16_f16 %[c1], %[b1], %[a0], %[c1]\n\t"                       \
+                 "s_add_i32 m0, %[wl], %[lc1]\n\t"                                              \
+                 "v_mfma_f32_32x32x16_f16 %[c2], %[b2], %[a0], %[c2]\n\t"                       \
+                 "global_load_lds_dwordx4 %[o1], %[base]\n\t"                                   \
+                 "v_mfma_f32_32x32x16_f16 %[c3], %[b3], %[a0], %[c3]\n\t"                       \
+                 "s_add_i32 m0, %[wl], %[lc2]\n\t"                                              \
+                 "v_mfma_f32_32x32x16_f16 %[c0], %[d0], %[a1], %[c0]\n\t"                       \
+                 "global_load_lds_dwordx4 %[o2], %[base]\n\t"                                   \
+                 "v_mfma_f32_32x32x16_f16 %[c1], %[d1], %[a1], %[c1]\n\t"                       \
+                 "s_add_i32 m0, %[wl], %[lc3]\n\t"                                              \
+                 "v_mfma_f32_32x32x16_f16 %[c2], %[d2], %[a1], %[c2]\n\t"                       \
+                 "global_load_lds_dwordx4 %[o3], %[base]\n\t"                                   \
+                 "v_mfma_f32_32x32x16_f16 %[c3], %[d3], %[a1], %[c3]"                           \
+                 : [c0] "+a"(acc[I][0]), [c1] "+a"(acc[I][1]), [c2] "+a"(acc[I][2]),            \
+                   [c3] "+a"(acc[I][3])                                                         \
+                 : [b0] "v"(CHUNK(fb[Q][0], 0)), [b1] "v"(CHUNK(fb[Q][1], 0)),                  \
+                   [b2] "v"(CHUNK(fb[Q][2], 0)), [b3] "v"(CHUNK(fb[Q][3], 0)),                  \
+                   [d0] "v"(CHUNK(fb[Q][0], 1)), [d1] "v"(CHUNK(fb[Q][1], 1)),                  \
+                   [d2] "v"(CHUNK(fb[Q][2], 1)), [d3] "v"(CHUNK(fb[Q][3], 1)),                  \
+                   [a0] "v"(CHUNK(fa[Q][I], 0)), [a1] "v"(CHUNK(fa[Q][I], 1)),                  \
+                   [wl] "s"(wave_lds),                                                          \
+                   [lc0] "n"((LDS_CONST) + 0 * 4096), [lc1] "n"((LDS_CONST) + 1 * 4096),        \
+                   [lc2] "n"((LDS_CONST) + 2 * 4096), [lc3] "n"((LDS_CONST) + 3 * 4096),        \
+                   [o0] "v"(OFF0), [o1] "v"(OFF1), [o2] "v"(OFF2), [o3] "v"(OFF3),              \
+                   [base] "s"(BASE)                                                             \
+                 : "memory", "scc")
 #define ROW12_READS(U, Q, I, N0)                                                                \
     do                                                                                          \
     {                                                                                           \
@@ -2803,14 +2865,28 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_f8_kernel(dma_params p)
                      : "+v"(fa[q_][0]), "+v"(fa[q_][1]), "+v"(fa[q_][2]), "+v"(fa[q_][3]),      \
                        "+v"(fb[q_][0]), "+v"(fb[q_][1]), "+v"(fb[q_][2]), "+v"(fb[q_][3])::"memory"); \
         block_barrier();                                                                        \
-        ROW12_READS(U, q_, 0, 0);                                                               \
-        ROW12_READS(U, q_, 1, 12);                                                              \
-        SB();                                                                                   \
-        MF4_LOAD4(q_, 2, W4_B_BASE + (((U) + 4) & (STAGES - 1)) * B_BYTES,                      \
-                  b_off[0], b_off[1], b_off[2], b_off[3], b_ptr);                               \
-        MF4_LOAD4(q_, 3, A_LOAD_STAGE12(U) * A2_BYTES + A_LOAD_BLOCK12(U) * 4096,               \
-                  a_off[A_LOAD_BLOCK12(U) + 0], a_off[A_LOAD_BLOCK12(U) + 1],                   \
-                  a_off[A_LOAD_BLOCK12(U) + 2], a_off[A_LOAD_BLOCK12(U) + 3], a_ptr);           \
+        if constexpr(HALF)                                                                      \
+        {                                                                                       \
+            ROWH12_READS(U, q_, 0, 0);                                                          \
+            ROWH12_READS(U, q_, 1, 8);                                                          \
+            SB();                                                                               \
+            MFH8_LOAD4(q_, 2, W4_B_BASE + (((U) + 4) & (STAGES - 1)) * B_BYTES,                 \
+                       b_off[0], b_off[1], b_off[2], b_off[3], b_ptr);                          \
+            MFH8_LOAD4(q_, 3, A_LOAD_STAGE12(U) * A2_BYTES + A_LOAD_BLOCK12(U) * 4096,          \
+                       a_off[A_LOAD_BLOCK12(U) + 0], a_off[A_LOAD_BLOCK12(U) + 1],              \
+                       a_off[A_LOAD_BLOCK12(U) + 2], a_off[A_LOAD_BLOCK12(U) + 3], a_ptr);      \
+        }                                                                                       \
+        else                                                                                    \
+        {                                                                                       \
+            ROW12_READS(U, q_, 0, 0);                                                           \
+            ROW12_READS(U, q_, 1, 12);                                                          \
+            SB();                                                                               \
+            MF4_LOAD4(q_, 2, W4_B_BASE + (((U) + 4) & (STAGES - 1)) * B_BYTES,                  \
+                      b_off[0], b_off[1], b_off[2], b_off[3], b_ptr);                           \
+            MF4_LOAD4(q_, 3, A_LOAD_STAGE12(U) * A2_BYTES + A_LOAD_BLOCK12(U) * 4096,           \
+                      a_off[A_LOAD_BLOCK12(U) + 0], a_off[A_LOAD_BLOCK12(U) + 1],               \
+                      a_off[A_LOAD_BLOCK12(U) + 2], a_off[A_LOAD_BLOCK12(U) + 3], a_ptr);       \
+        }                                                                                       \
         SB();                                                                                   \
         b_ptr += b_step;                                                                        \
         if constexpr(((U) & 1) == 0)                                                            \
@@ -2894,6 +2970,8 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_f8_kernel(dma_params p)
         SLAB(kt, 0, false);
 #undef SLAB12
 #undef MF4_LOAD4
+#undef MFH8_LOAD4
+#undef ROWH12_READS
 #undef ROW12_READS
 #undef MF12
 #undef READ12
@@ -2904,6 +2982,8 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_f8_kernel(dma_params p)
 #undef ROW
 #undef OTHER
 #undef MF
+#undef MFH
+#undef CHUNK
 #undef WAIT_FRAGS
 #undef RB
 #undef RA
@@ -3024,6 +3104,13 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_f8_kernel(dma_params p)
         constexpr int ESZ  = OUT == MI355_F32 ? 4 : 2;
         constexpr int JP   = OUT == MI355_F32 ? 2 : 4; // 32-column blocks per round
         uint8_t* mine      = lds + wave * 40960;
+        // a product of halves is rounded by the operator itself, dequantized codes by `convert`
+        auto pack = [](float lo, float hi) -> uint32_t {
+            if constexpr(HALF)
+                return f32_to_half_rtz(lo) | ((uint32_t)f32_to_half_rtz(hi) << 16);
+            else
+                return pack16<OUT>(lo, hi);
+        };
 #pragma unroll
         for(int round = 0; round < 4 / JP; round++)
         {
@@ -3050,8 +3137,7 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_f8_kernel(dma_params p)
                         if constexpr(OUT == MI355_F32)
                             *reinterpret_cast<v4f*>(dst) = v4f{v[0], v[1], v[2], v[3]};
                         else
-                            *reinterpret_cast<uint2*>(dst) =
-                                make_uint2(pack16<OUT>(v[0], v[1]), pack16<OUT>(v[2], v[3]));
+                            *reinterpret_cast<uint2*>(dst) = make_uint2(pack(v[0], v[1]), pack(v[2], v[3]));
                     }
                 }
                 if(j + 1 < 4)
@@ -4357,6 +4443,65 @@ int launch_out(const dma_params& p, int batch, bool deq, int out, hipStream_t s)
 }
 
 } // namespace
+
+// half A [M, K] times half B [N, K] (dense rows), half result rounded toward zero, or with shares > 1
+// float sums of K / shares each in partial[share][M][N] (the split goes through the kernel's batch
+// index); offsets inside an operand are kept in 32 bits, a slab is 32 halves, results leave in groups
+// of 8
+bool mi355_dma_half_supported(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldc, const void* a, const void* out)
+{
+    const int64_t lim = (int64_t)1 << 31;
+    return m > 0 && n > 0 && k >= 1536 && k % 32 == 0 && n % 8 == 0 && lda % 8 == 0 && ldc % 8 == 0 &&
+           m * lda * 2 < lim && n * k * 2 < lim && reinterpret_cast<uintptr_t>(a) % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(out) % 16 == 0;
+}
+
+int mi355_dma_half_launch(const uint16_t* a, int64_t lda, const uint16_t* b, uint16_t* out, int64_t ldc, int64_t m,
+                          int64_t n, int64_t k, int shares, float* partial, hipStream_t stream)
+{
+    dma_params p{};
+    p.a            = reinterpret_cast<const uint8_t*>(a);
+    p.b            = reinterpret_cast<const uint8_t*>(b);
+    p.c            = out;
+    p.m            = (int)m;
+    p.n            = (int)n;
+    p.k            = (int)(2 * k);
+    p.lda          = 2 * lda;
+    p.ldb          = 2 * k;
+    p.ldc          = ldc;
+    p.tiles_m      = (p.m + BM - 1) / BM;
+    p.tiles_n      = (p.n + BN - 1) / BN;
+    p.scale_a_mode = MI355_QP_NONE;
+    p.scale_b_mode = MI355_QP_NONE;
+    p.ksplit       = 1;
+    p.vec_store    = 1;
+    p.vec8_store   = 1;
+    p.vec_cols     = 1;
+    p.stream_c     = (double)m * (double)n * 2.0 >= 128.0 * 1048576.0;
+    if(shares > 1)
+    {
+        p.k        = (int)(2 * k / shares);
+        p.stride_a = p.k;
+        p.stride_b = p.k;
+        p.c        = partial;
+        p.ldc      = n;
+        p.stride_c = m * n;
+        p.stream_c = 0;
+    }
+    using kernel_t        = void (*)(dma_params);
+    const kernel_t whole  = qgemm_w4_f8_kernel<true, true, MI355_F16, true, true>;
+    const kernel_t shared = qgemm_w4_f8_kernel<true, false, MI355_F32, false, true>;
+    static const bool attrs_ok =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(whole), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            W4_LDS_BYTES) == hipSuccess &&
+        hipFuncSetAttribute(reinterpret_cast<const void*>(shared), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            W4_LDS_BYTES) == hipSuccess;
+    if(!attrs_ok)
+        return MI355_ERR_LAUNCH;
+    hipLaunchKernelGGL(shares > 1 ? shared : whole, dim3(p.tiles_m * p.tiles_n, shares), dim3(W4_THREADS), W4_LDS_BYTES,
+                       stream, p);
+    return mi355_launch_status();
+}
 
 // Block-scaled fp4 x fp4 or fp8 x fp8 (see qgemm_dma_kernel<.., MX>): kbytes = bytes per row of A
 // [M, kbytes] and of B [N, kbytes] (K / 2 or K), a multiple of the 64-byte slab; bits = 4 or 8;

@@ -16,6 +16,11 @@
 #include <utility>
 #include "common.h"
 
+// the 256 x 256 matrix-core kernel for half operands (qgemm_dma.hip)
+bool mi355_dma_half_supported(int64_t m, int64_t n, int64_t k, int64_t lda, int64_t ldc, const void* a, const void* out);
+int mi355_dma_half_launch(const uint16_t* a, int64_t lda, const uint16_t* b, uint16_t* out, int64_t ldc, int64_t m,
+                          int64_t n, int64_t k, int shares, float* partial, hipStream_t stream);
+
 namespace {
 
 constexpr int W4_THREADS = 256;
@@ -396,6 +401,7 @@ int launch_gemv_m1(const w4_params& p, hipStream_t s)
 
 #include "w4a16_mfma.h"
 #include "w4a16_tile.h"
+#include "w4a16_expand.h"
 
 } // namespace
 
@@ -423,6 +429,8 @@ extern "C" size_t mi355_w4a16_gemm_workspace_size(int64_t m, int64_t n, int64_t 
     if(m < 2 || n <= 0 || k <= 0 || group <= 0 || k % 128 != 0 || n % 16 != 0 || k > (1 << 30) || n > (1 << 30) ||
        m > (1 << 30))
         return 0;
+    if(const int shares = expand_gemm_shares(m, n, k); shares > 0)
+        return expand_gemm_bytes(m, n, k, shares);
     if(m > 32 && n % TL_BN == 0)
     {
         const int shares = tile_gemm_shares((int)m, (int)n, (int)k);
@@ -498,6 +506,8 @@ extern "C" int mi355_w4a16_gemm_ws(const void* a,
     if(m == 1 && zp_mode == MI355_W4_ZP_SCALAR && k % 2048 == 0 && k <= GV_MAX_K &&
        (group & (group - 1)) == 0 && group <= 2048)
         return launch_gemv_m1(p, s);
+    if(expand_gemm_supported(p))
+        return launch_expand_gemm(p, s);
     if(m >= 2 && mfma_gemm_supported(p))
         return launch_mfma_gemm(p, s);
     dim3 grid((unsigned)((n + 3) / 4));

@@ -1,0 +1,122 @@
+// int4 weight-only GEMM for many rows of A (included by w4a16.hip inside its anonymous namespace, after
+// w4a16_tile.h): the weights are dequantized once into the caller's workspace, then multiplied as
+// halves by the 256 x 256 kernel of qgemm_dma.hip.
+//
+// The tile kernel next door dequantizes the weights anew for every 64 rows of A, in the waves that
+// feed the matrix cores: 14 packed instructions per 16 x 16 x 32 product of 4 row tiles bound it at
+// 660 TFLOP/s.  From about a thousand rows on, writing the operator's own intermediate (the
+// dequantized half weights, rounded toward zero as dequantizelinear rounds them) costs less than
+// that: 2.5 bytes per weight at the memory's rate, once.
+// Measured: 2048 x 14336 x 4096 362 -> 259 us, of which the expansion is 23 (147 MB) and the product 233
+// (1030 TFLOP/s in two waves of workgroups, the second 3/4 full; a 8192^3 bf16 library product
+// reaches 1210 here); 4096 x 28672 x 8192 2724 -> 1612; 2048 x 4096 x 14336 in two shares of K 324 -> 237.
+
+// 8 consecutive weights of one row per thread and turn: 4 packed bytes in, one 16-byte store, so that
+// a wave reads 256 and writes 1024 bytes in one piece each.  blockIdx.y is the row, a block walks
+// EX_TURNS * 256 pieces of it.  group_magic = ceil(2^32 / (group / 8)) divides a piece's index
+// exactly while the product of both stays below 2^32.
+constexpr int EX_TURNS = 4;
+
+__global__ __launch_bounds__(256) void w4a16_expand_kernel(w4_params p, v4u* out, uint32_t group_magic)
+{
+    const uint32_t per_row = (uint32_t)p.k / 8;
+    const uint32_t n       = blockIdx.y + gridDim.y * blockIdx.z;
+    if(n >= (uint32_t)p.n)
+        return;
+    const uint32_t groups  = (uint32_t)p.k / (uint32_t)p.group;
+    const uint16_t* scales = p.scales + (int64_t)n * groups;
+    const uint32_t* packed = reinterpret_cast<const uint32_t*>(p.w) + (int64_t)n * per_row;
+    v4u* row               = out + (int64_t)n * per_row;
+#pragma unroll
+    for(int t = 0; t < EX_TURNS; t++)
+    {
+        const uint32_t i = (blockIdx.x * EX_TURNS + t) * 256 + threadIdx.x;
+        if(i >= per_row)
+            return;
+        const uint32_t g = __umulhi(i, group_magic);
+        const uint32_t q = packed[i];
+        const float sc   = half_to_f32(scales[g]);
+        int z            = p.zp_scalar;
+        if(p.zp_mode == MI355_W4_ZP_GROUP)
+            z = p.zp[(int64_t)n * groups + g];
+        else if(p.zp_mode == MI355_W4_ZP_PACKED)
+        {
+            const uint8_t zb = p.zp[(int64_t)n * ((groups + 1) / 2) + (g >> 1)];
+            z                = (g & 1) ? (zb >> 4) : (zb & 0xf);
+        }
+        const float zf = (float)z;
+        v4u w;
+#pragma unroll
+        for(int e = 0; e < 4; e++)
+        {
+            // (q - zp) * scale is exact in float; one rounding toward zero, to the largest finite
+            // half where it leaves the range, as the packed half multiplication of the tile kernel
+            const float lo = ((float)((q >> (8 * e)) & 0xf) - zf) * sc;
+            const float hi = ((float)((q >> (8 * e + 4)) & 0xf) - zf) * sc;
+            w[e]           = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
+        }
+        row[i] = w;
+    }
+}
+
+// Shares of K for the two passes, or 0 where the tile kernel is the faster one, from what each was
+// measured to take (us) on one MI355X: a full wave of 256 workgroups of the 256 x 256 kernel 29 per
+// 1024 of K, the expansion 0.42 per 2^20 weights, the sum of the shares 0.4 per MB of partial
+// sums and 3, a full wave of the tile kernel 6.8 per 1024 of K.  A tenth stays with the tile
+// kernel, which needs no workspace for weights.
+int expand_gemm_shares(int64_t m, int64_t n, int64_t k)
+{
+    if(m <= 256 || n % TL_BN != 0 || k < 1536 || k > (1 << 18))
+        return 0;
+    const int64_t big   = ((m + 255) / 256) * ((n + 255) / 256);
+    const int64_t small = ((m + 63) / 64) * (n / TL_BN);
+    const double k1024  = (double)k / 1024.0;
+    const double expand = (double)n * (double)k / 1048576.0 * 0.42;
+    double best         = 0.9 * (double)((small + 255) / 256) * 6.8 * k1024;
+    int shares          = 0;
+    for(int s = 1; s <= 4 && (s == 1 || big * (s - 1) < 256); s++)
+    {
+        if(k % (32 * s) != 0 || k / s < 1536)
+            continue;
+        double us = expand + (double)((big * s + 255) / 256) * 29.0 * k1024 / s;
+        if(s > 1)
+            us += 3.0 + (double)s * (double)m * (double)n * 4e-6 * 0.4;
+        if(us < best)
+        {
+            best   = us;
+            shares = s;
+        }
+    }
+    return shares;
+}
+
+size_t expand_gemm_bytes(int64_t m, int64_t n, int64_t k, int shares)
+{
+    return (size_t)n * k * 2 + (shares > 1 ? (size_t)shares * m * n * 4 : 0);
+}
+
+bool expand_gemm_supported(const w4_params& p)
+{
+    const int shares = expand_gemm_shares(p.m, p.n, p.k);
+    return shares > 0 && p.partial != nullptr && tile_gemm_supported(p) &&
+           p.partial_bytes >= expand_gemm_bytes(p.m, p.n, p.k, shares) &&
+           mi355_dma_half_supported(p.m, p.n, p.k, p.lda, p.ldc, p.a, p.out);
+}
+
+int launch_expand_gemm(const w4_params& p0, hipStream_t s)
+{
+    w4_params p              = p0;
+    const int shares         = expand_gemm_shares(p.m, p.n, p.k);
+    uint16_t* weights        = reinterpret_cast<uint16_t*>(p.partial);
+    const uint32_t per_piece = (uint32_t)p.group / 8; // pieces of a group, at least 4
+    const uint32_t magic     = (uint32_t)(((1ull << 32) + per_piece - 1) / per_piece);
+    const unsigned rows_y    = (unsigned)(p.n < 32768 ? p.n : 32768);
+    const dim3 grid((unsigned)((p.k / 8 + 256 * EX_TURNS - 1) / (256 * EX_TURNS)), rows_y,
+                    (unsigned)((p.n + rows_y - 1) / rows_y));
+    hipLaunchKernelGGL(w4a16_expand_kernel, grid, dim3(256), 0, s, p, reinterpret_cast<v4u*>(weights), magic);
+    p.partial    = reinterpret_cast<float*>(weights + (size_t)p.n * p.k);
+    const int st = mi355_dma_half_launch(p.a, p.lda, weights, p.out, p.ldc, p.m, p.n, p.k, shares, p.partial, s);
+    if(st != MI355_OK || shares == 1)
+        return st;
+    return launch_w4a16_reduce(p, shares, s);
+}

@@ -1,0 +1,51 @@
+"""int4 weight-only GEMM of many rows: weights dequantized into the workspace, then the 256 x 256
+half kernel.  Against a float64 product of the dequantized half weights."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from amdmigraphx_amd import ops
+    return ops
+
+
+# rows and columns that fill no 256 x 256 tile, K of 12 * 4 slabs, one more trip of slabs and a remainder
+@pytest.mark.parametrize("m,n,k,pad", [(1999, 7296, 1536, 0), (970, 15744, 1664, 8), (2048, 8192, 2688, 0),
+                                       (1000, 3968, 9216, 8)])
+@pytest.mark.parametrize("group,zeros", [(128, "scalar"), (64, "group"), (32, "packed")])
+def test_many_rows(ops, m, n, k, pad, group, zeros):
+    need = ops.w4a16_gemm_workspace_size(m, n, k, group)
+    assert need >= 2 * n * k  # the shapes of this test take the two passes
+    assert (need > 2 * n * k) == (k > 4096)  # the last one with K in shares
+    rng = np.random.default_rng(m + group)
+    x = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float16)).cuda()
+    packed = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    scales = orc.half_from_f32(rng.uniform(0.005, 0.02, (n, k // group)).astype(np.float32))
+    scales[::17, 0] = 0x0001  # a subnormal scale
+    groups = k // group
+    z = rng.integers(0, 16, (n, groups), dtype=np.uint8)
+    if zeros == "scalar":
+        z[:] = 8
+        zp, mode = 8, None
+    elif zeros == "group":
+        zp, mode = torch.from_numpy(z).cuda(), ops.W4ZP.GROUP
+    else:
+        both = np.concatenate([z, np.zeros((n, groups % 2), np.uint8)], axis=1)
+        zp, mode = torch.from_numpy(both[:, ::2] | (both[:, 1::2] << 4)).cuda().contiguous(), ops.W4ZP.PACKED
+    q = np.stack([packed & 15, packed >> 4], axis=2).reshape(n, groups, group).astype(np.float32)
+    w = (q - z[:, :, None].astype(np.float32)) * orc.half_to_f32(scales)[:, :, None]
+    w = torch.from_numpy(orc.half_from_f32(w.reshape(n, k)).view(np.float16)).cuda().double()
+    out = torch.full((m, n + pad), -1.0, dtype=torch.float16, device="cuda")
+    got = ops.w4a16_gemm(x, torch.from_numpy(packed).cuda(), torch.from_numpy(scales.view(np.float16)).cuda(), group,
+                         zp, zp_mode=mode, out=out[:, :n], workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))
+    want = x.double() @ w.t()
+    # k float32 additions round to nearest, the result is cut to 11 bits (subnormal steps of 2^-24 below)
+    bound = (x.double().abs() @ w.t().abs()) * (k * 2.0**-24) + want.abs() * 2.0**-10 + 2.0**-24
+    assert bool(((got.double() - want).abs() <= bound).all())
+    assert pad == 0 or bool((out[:, n:] == -1).all())
