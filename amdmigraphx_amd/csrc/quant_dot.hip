@@ -207,6 +207,63 @@ __global__ __launch_bounds__(256) void colsum_rowmajor_kernel(
     atomicAdd(out + col, s);
 }
 
+// What a product takes (us) in the kernels that compete for it, fitted to measurements on one MI355X of
+// 1 to 384 batches, M and N of 16 to 16384, K of 64 to 8208, both types and both orders of B.
+//
+// The register-staged kernel (qgemm_ragged.hip) has tiles of 64 x 64, or 128 x 128 where those fill
+// the chip; a workgroup of it starts sooner and several share a CU, so it wins wherever the 256 x 256
+// tiles of the other two leave CUs idle or are mostly padding, and where K is short:
+//   96 batches of 197 x 197 x 64 int8 -> float   23.7 -> 11.3 us     384 of 64 x 64 x 64   19.7 -> 8.2
+//   1024 x 1024 x 1024 int8 -> bfloat16          23.5 -> 6.5         512 x 4096 x 4096 (split)   30.9 -> 21.3
+//   48 x 1024 x 1024 x 128                       49.8 against 53.7 (stays)
+double ragged_us(const mi355_quant_dot_desc* d)
+{
+    auto tiles = [&](int64_t t) { return (double)d->batch * (double)((d->m + t - 1) / t) * (double)((d->n + t - 1) / t); };
+    const double small = tiles(64), big = tiles(128);
+    double per_k;
+    if(big < 256) // (the kernel's own choice of the tile)
+        per_k = d->trans_b ? 0.0021 * __builtin_fmax(1.0, small / 256.0 * 0.95)
+                           : 0.0031 * __builtin_fmax(1.0, small / 256.0 * 0.8);
+    else if(big <= 256)
+        per_k = d->trans_b ? 0.0083 : 0.0088;
+    else
+        per_k = (d->trans_b ? 0.0095 : 0.0115) * __builtin_ceil(big / 512.0);
+    const double out = (double)d->batch * (double)d->m * (double)d->n *
+                       (double)(d->dequant ? mi355_dtype_size(d->out_type) : 4);
+    return 3.4 + per_k * (double)d->k + out / 4.0e6;
+}
+
+double waves_of_256(const mi355_quant_dot_desc* d)
+{
+    return __builtin_ceil((double)d->batch * (double)((d->m + 255) / 256) * (double)((d->n + 255) / 256) / 256.0);
+}
+
+// direct-to-LDS kernels; `shares` of K through a workspace
+double dma_us(const mi355_quant_dot_desc* d, double shares)
+{
+    const double k = (double)d->k;
+    if(shares > 1.0)
+        return 7.8 + 0.0093 * k / shares +
+               shares * (double)d->batch * (double)d->m * (double)d->n * 8.0 / 5.0e6;
+    if(d->in_type == MI355_FP8)
+        return waves_of_256(d) * (d->k < 3072 ? 8.8 + 0.0093 * k : 14.0 + 0.0081 * k);
+    return waves_of_256(d) * (d->k < 3072 ? 12.8 + 0.0112 * k : 16.0 + 0.0089 * k);
+}
+
+// the matrix-core kernel for K that is no multiple of 64
+double mfma_us(const mi355_quant_dot_desc* d)
+{
+    return waves_of_256(d) * (13.0 + (d->trans_b ? 0.0145 : 0.0165) * (double)d->k);
+}
+
+// a vector of column scales per batch entry exists in the direct-to-LDS kernels only; a fourteenth
+// of the time is left to the fit's error
+bool ragged_is_faster(const mi355_quant_dot_desc* d, double other_us)
+{
+    return d->k > 0 && mi355_ragged_gemm_supported(d) &&
+           !(d->dequant && d->scale_b_mode == MI355_QP_PER_COL_BATCH) && ragged_us(d) < 0.93 * other_us;
+}
+
 __global__ void zero_i32_kernel(int32_t* p, int64_t n)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -324,12 +381,24 @@ extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
     // int8 with N % 4 != 0 would take the DMA path's 32 x 32 kernel, which applies no bias
     const bool dma_has_bias = bias == nullptr || fp8 || d->n % 4 == 0;
     if(!u8 && !bf8 && d->k > 0 && dma_has_bias && mi355_dma_gemm_supported(d, a, b))
+    {
+        // fp8: the sums of both are float
+        const size_t split = mi355_dma_gemm_workspace(d);
+        const bool room    = workspace != nullptr && split > 0 && split <= workspace_bytes;
+        const double shares = room ? (double)split / (4.0 * (double)d->batch * (double)d->m * (double)d->n) : 1.0;
+        if(ragged_is_faster(d, dma_us(d, shares)))
+            return mi355_ragged_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, true, s);
         return mi355_dma_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace, workspace_bytes, s);
+    }
     // a vector of column scales per batch entry exists in the kernels above only
     if(d->dequant && d->scale_b_mode == MI355_QP_PER_COL_BATCH)
         return MI355_ERR_UNSUPPORTED;
     if(!u8 && d->k > 0 && mi355_mfma_gemm_supported(d, a, b, c))
+    {
+        if(!bf8 && ragged_is_faster(d, mfma_us(d)))
+            return mi355_ragged_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, true, s);
         return mi355_mfma_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, s);
+    }
     // rows aligned to nothing; fp8 sums stay exact there, as in the kernel below
     if(mi355_ragged_gemm_supported(d))
         return mi355_ragged_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, false, s);

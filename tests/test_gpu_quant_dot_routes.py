@@ -1,0 +1,67 @@
+"""quant_dot on both sides of the line between the kernels with 256 x 256 tiles and the register-staged
+one: the shapes that stay with the large tiles, and those beside them that do not, against the same
+product in float64 (exact for int8; the fp8 sums are float)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from amdmigraphx_amd import ops
+    return ops
+
+
+def _codes(g, shape, fp8):
+    if fp8:
+        return (torch.randn(shape, generator=g, device="cuda") * 16).to(torch.float8_e4m3fn)
+    return torch.randint(-128, 128, shape, generator=g, device="cuda", dtype=torch.int8)
+
+
+def _check(ops, batch, m, n, k, trans_b, fp8, workspace=None):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = _codes(g, (batch, m, k), fp8)
+    b = _codes(g, (batch, n, k) if trans_b else (batch, k, n), fp8)
+    b = b.transpose(1, 2) if trans_b else b
+    sa = torch.rand(1, generator=g, device="cuda") * 0.01
+    sb = torch.rand(n, generator=g, device="cuda") * 0.01
+    bits = (lambda t: t.view(torch.uint8)) if fp8 else (lambda t: t)
+    bd = bits(b.transpose(1, 2)).transpose(1, 2) if trans_b else bits(b)
+    print("route", batch, m, n, k, trans_b, fp8, flush=True)
+    got = [ops.quant_dot(bits(a), bd, fp8=fp8), ops.quant_dot(bits(a), bd, fp8=fp8, scale_a=sa, scale_b=sb)]
+    if batch == 1:
+        need = ops.quant_dot_workspace_size(m, n, k, trans_b=trans_b, fp8=fp8)
+        if need:
+            got.append(ops.quant_dot(bits(a)[0], bd[0], fp8=fp8, scale_a=sa, scale_b=sb,
+                                     workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))[None])
+    for i in range(batch):
+        acc = a[i].double() @ b[i].double().contiguous()
+        s = (sa * sb).double()
+        for t, want in zip(got, [acc, acc * s, acc * s]):
+            if not fp8:
+                assert torch.equal(t[i].double(), want.float().double() if t.is_floating_point() else want)
+                continue
+            # the contract of the fp8 sums: 1e-3 relative, or, where a sum cancels, 2^-15 of the sum of the
+            # magnitudes (the instruction cuts its products at a distance below the largest of them; both
+            # kernels are 1.46e-5 from the exact sums as a whole)
+            most = (a[i].double().abs() @ b[i].double().abs().contiguous()) * (s if want is not acc else 1.0)
+            assert bool(((t[i].double() - want).abs() <= torch.maximum(want.abs() * 1e-3, most * 2.0**-15)).all())
+
+
+# K on both sides of the four-wave kernels' first length; edges of the 256 tiles
+@pytest.mark.parametrize("batch,m,n,k", [(1, 4100, 4112, 1600), (1, 2050, 8208, 3136), (1, 16, 512, 8192),
+                                         (1, 2050, 8208, 784), (1, 300, 8208, 3136)])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_large_tiles(ops, batch, m, n, k, trans_b, fp8):
+    _check(ops, batch, m, n, k, trans_b, fp8)
+
+
+@pytest.mark.parametrize("batch,m,n,k", [(5, 64, 64, 64), (3, 197, 208, 128), (2, 130, 80, 272), (40, 384, 64, 384),
+                                         (1, 1030, 1040, 1024), (1, 16, 16, 3072)])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_small_tiles(ops, batch, m, n, k, trans_b, fp8):
+    _check(ops, batch, m, n, k, trans_b, fp8)
