@@ -280,6 +280,263 @@ __global__ __launch_bounds__(256) void mx_gemm_kernel(mx_params p)
         }
 }
 
+// ---- small tiles, scales read as they are ----------------------------------------------------------
+// The 256 x 256 staged kernels need a grid of them: 512 x 4096 x 4096 is 32 workgroups on 256 CUs.  This
+// kernel has tiles of 64 x 64 (a wave 32 x 32), register-staged through two LDS stages with the loads
+// of the next two slabs in flight, and reads the float scales of one value per block itself: the exponent is a shift, and a lane that meets anything but a normal power of two
+// raises the call's flag as mx_prepare_kernel does (the exact kernel behind it then computes the
+// result), so the prepare launch and its pass over the scales are gone.
+// What bounds it is the latency of a slab and the rate at which a workgroup pulls its operands in.
+// Measured, all launches of a call, fp4 / fp8: 512 x 4096 x 4096 40.0 -> 27.6 / 59.5 -> 44.6 us, 16 x 4096 x 4096
+// 35.6 -> 13.3 / 51.2 -> 18.3, 128 x 4096 x 14336 101 -> 41 / 154 -> 71.  (Slabs of 256 bytes need more
+// registers than two workgroups on a CU have and spill: 44 us; 128 x 128 tiles as well.)
+//
+// Both operands have one type, K bytes are K / 2 (fp4) or K (fp8).  The product does not care which K
+// positions meet as long as A and B agree, so the blocks of a slab are dealt to the instruction's
+// four lane groups in runs: group g holds the slab's blocks NB g .. NB g + NB - 1 (NB = blocks of a
+// slab / 4), block NB g + h in step h, and its scales are consecutive floats.
+//   fp4: a block is 16 bytes, a lane's operand of one step.
+//   fp8: the instruction's K is two halves of 64, lane group g holds 16 bytes of either; block b of
+//        the four is half b / 2, lane groups 2 (b % 2) and 2 (b % 2) + 1.
+template <int N>
+struct __attribute__((packed, aligned(4))) scale_run
+{
+    uint32_t v[N];
+};
+
+template <bool FP4>
+__global__ __launch_bounds__(256, 2) void mx_tile_kernel(mx_params p, int tiles_m, int tiles_n)
+{
+    constexpr int BT     = 64;
+    constexpr int SLAB   = 128; // bytes of a row
+    constexpr int T      = BT / 32;         // 16 x 16 tiles of a wave along either side
+    constexpr int PITCH  = SLAB + 16;
+    constexpr int BLOCK  = FP4 ? 16 : 32; // bytes of a scale block
+    constexpr int NB     = SLAB / BLOCK / 4; // steps of a slab = blocks of a lane group
+    constexpr int PIECES = BT * SLAB / 16 / 256;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2][2][BT * PITCH];
+
+    const int tid    = threadIdx.x;
+    const int lane   = tid & 63;
+    const int wave   = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_m = wave >> 1, wave_n = wave & 1;
+    const int r = lane & 15, g = lane >> 4;
+
+    // a contiguous run of tiles per XCD, the rows that share a panel of B one after the other
+    int v           = blockIdx.x;
+    const int tiles = tiles_m * tiles_n;
+    if(tiles % 8 == 0)
+        v = (v % 8) * (tiles / 8) + v / 8;
+    const int m0 = (v % tiles_m) * BT;
+    const int n0 = (v / tiles_m) * BT;
+    const int kb = FP4 ? p.k / 2 : p.k;
+
+    const uint8_t* __restrict__ ga = p.a + (int64_t)blockIdx.y * p.stride_a;
+    const uint8_t* __restrict__ gb = p.b + (int64_t)blockIdx.y * p.stride_b;
+
+    constexpr int KC = SLAB / 16;
+    const int ld_kc  = (tid % KC) * 16;
+    uint32_t a_off[PIECES], b_off[PIECES];
+#pragma unroll
+    for(int s = 0; s < PIECES; s++)
+    {
+        const int row = (tid + 256 * s) / KC;
+        a_off[s]      = (uint32_t)min(m0 + row, p.m - 1) * (uint32_t)p.lda;
+        b_off[s]      = (uint32_t)min(n0 + row, p.n - 1) * (uint32_t)p.ldb;
+    }
+    const float* sa_row[T];
+    const float* sb_row[T];
+#pragma unroll
+    for(int i = 0; i < T; i++)
+    {
+        sa_row[i] = p.scale_a + (int64_t)blockIdx.y * p.sa_batch +
+                    (int64_t)min(m0 + wave_m * 16 * T + 16 * i + r, p.m - 1) * p.sa_row;
+        sb_row[i] = p.scale_b + (int64_t)blockIdx.y * p.sb_batch +
+                    (int64_t)min(n0 + wave_n * 16 * T + 16 * i + r, p.n - 1) * p.sb_row;
+    }
+
+    // The scales of a slab are needed before its successor's operands: they are requested in front of
+    // them, so that waiting for the former leaves the latter in flight.
+    constexpr int AHEAD = 2;
+    v4u ra[AHEAD][PIECES], rb[AHEAD][PIECES];
+    uint32_t sa_next[AHEAD][T][NB], sb_next[AHEAD][T][NB];
+    uint32_t sa[T], sb[T]; // exponent bytes of the slab in hand, step h in byte h
+    auto load_slab = [&](int k0, int u) {
+        const int at = min(k0 + ld_kc, kb - 16);
+#pragma unroll
+        for(int s = 0; s < PIECES; s++)
+        {
+            ra[u][s] = *reinterpret_cast<const v4u*>(ga + a_off[s] + at);
+            rb[u][s] = *reinterpret_cast<const v4u*>(gb + b_off[s] + at);
+        }
+    };
+    auto store_slab = [&](int k0, int stage, int u) {
+        // pieces past the end of K: zeros, which add nothing whatever their scale
+        const bool past = k0 + ld_kc >= kb;
+#pragma unroll
+        for(int s = 0; s < PIECES; s++)
+        {
+            const int at = (tid + 256 * s) / KC * PITCH + ld_kc;
+            *reinterpret_cast<v4u*>(lds[stage][0] + at) = past ? v4u{0, 0, 0, 0} : ra[u][s];
+            *reinterpret_cast<v4u*>(lds[stage][1] + at) = past ? v4u{0, 0, 0, 0} : rb[u][s];
+        }
+    };
+    // K is whole runs of 4 blocks: a lane's run lies inside K or behind it (the last run again: a scale
+    // of zeros)
+    auto load_scales = [&](int kt, int u) {
+        const int blk = min(kt * 4 * NB + NB * g, p.nblk - NB);
+#pragma unroll
+        for(int i = 0; i < T; i++)
+        {
+            const scale_run<NB> ar = *reinterpret_cast<const scale_run<NB>*>(sa_row[i] + blk);
+            const scale_run<NB> br = *reinterpret_cast<const scale_run<NB>*>(sb_row[i] + blk);
+#pragma unroll
+            for(int h = 0; h < NB; h++)
+            {
+                sa_next[u][i][h] = ar.v[h];
+                sb_next[u][i][h] = br.v[h];
+            }
+        }
+    };
+    // a positive normal power of two has neither sign nor mantissa, and an exponent of 1 .. 254
+    uint32_t bad     = 0;
+    auto exponents = [&](const uint32_t (&bits)[NB]) {
+        uint32_t packed = 0;
+#pragma unroll
+        for(int h = 0; h < NB; h++)
+        {
+            bad |= (bits[h] & 0x807fffffu) | (bits[h] - 0x00800000u >= 0x7f000000u ? 1u : 0u);
+            packed |= ((bits[h] >> 23) & 0xffu) << (8 * h);
+        }
+        return packed;
+    };
+    auto take_scales = [&](int u) {
+#pragma unroll
+        for(int i = 0; i < T; i++)
+        {
+            sa[i] = exponents(sa_next[u][i]);
+            sb[i] = exponents(sb_next[u][i]);
+        }
+    };
+
+    v4f32 acc[T][T];
+#pragma unroll
+    for(int i = 0; i < T; i++)
+#pragma unroll
+        for(int j = 0; j < T; j++)
+            acc[i][j] = v4f32{0.f, 0.f, 0.f, 0.f};
+
+    auto multiply = [&](int stage) {
+        const uint8_t* as = lds[stage][0] + (wave_m * 16 * T + r) * PITCH;
+        const uint8_t* bs = lds[stage][1] + (wave_n * 16 * T + r) * PITCH;
+        auto fragment = [&](const uint8_t* row, int h) -> v8i {
+            if constexpr(FP4)
+            {
+                const v4i lo = *reinterpret_cast<const v4i*>(row + (NB * g + h) * 16);
+                return v8i{lo.x, lo.y, lo.z, lo.w, 0, 0, 0, 0};
+            }
+            else
+            {
+                const v4i lo = *reinterpret_cast<const v4i*>(row + (NB * (g >> 1) + h) * 32 + 16 * (g & 1));
+                const v4i hi = *reinterpret_cast<const v4i*>(row + (NB * (2 + (g >> 1)) + h) * 32 + 16 * (g & 1));
+                return v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+            }
+        };
+auto one = [&](auto step) {
+            constexpr int h = decltype(step)::value;
+            if constexpr(h < NB)
+            {
+                v8i fa[T], fb[T];
+#pragma unroll
+                for(int i = 0; i < T; i++)
+                {
+                    fa[i] = fragment(as + 16 * i * PITCH, h);
+                    fb[i] = fragment(bs + 16 * i * PITCH, h);
+                }
+#pragma unroll
+                for(int i = 0; i < T; i++)
+#pragma unroll
+                    for(int j = 0; j < T; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
+                            fa[i], fb[j], acc[i][j], FP4 ? 4 : 0, FP4 ? 4 : 0, h, (int)sa[i], h, (int)sb[j]);
+                // the operands of all steps at once would not fit the registers
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        one(std::integral_constant<int, 0>{});
+        one(std::integral_constant<int, 1>{});
+    };
+
+    // slab kt sits in stage kt & 1; while it is multiplied, the next ones are loaded
+    const int nk = (kb + SLAB - 1) / SLAB;
+    load_scales(0, 0);
+    load_slab(0, 0);
+    load_scales(1, 1);
+    load_slab(SLAB, 1);
+    store_slab(0, 0, 0);
+    __syncthreads();
+    auto step = [&](int kt, int u) {
+        take_scales(u);
+        load_scales(kt + AHEAD, u);
+        load_slab((kt + AHEAD) * SLAB, u);
+        multiply(u);
+        // the other stage was last read before the barrier that ended the step before
+        if(kt + 1 < nk)
+            store_slab((kt + 1) * SLAB, u ^ 1, u ^ 1);
+        // the LDS accesses of all waves done; the loads stay in flight
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    int kt = 0;
+    for(; kt + 1 < nk; kt += 2)
+    {
+        step(kt, 0);
+        step(kt + 1, 1);
+    }
+    if(kt < nk)
+    {
+        take_scales(0);
+        multiply(0);
+    }
+    if(bad != 0)
+        *p.flag = p.ticket;
+
+    // element e of lane (r, g) of tile (i, j): row 16 i + 4 g + e, column 16 j + r
+    float* c = p.c + (int64_t)blockIdx.y * p.stride_c;
+#pragma unroll
+    for(int i = 0; i < T; i++)
+#pragma unroll
+        for(int e = 0; e < 4; e++)
+        {
+            const int row = m0 + wave_m * 16 * T + i * 16 + 4 * g + e;
+            if(row >= p.m)
+                continue;
+#pragma unroll
+            for(int j = 0; j < T; j++)
+            {
+                const int col = n0 + wave_n * 16 * T + j * 16 + r;
+                if(col < p.n)
+                    c[(int64_t)row * p.ldc + col] = acc[i][j][e];
+            }
+        }
+}
+
+int64_t mx_small_tiles(const mx_params& p, int64_t batch)
+{
+    return batch * ((p.m + 63) / 64) * ((p.n + 63) / 64);
+}
+
+// Up to two workgroups a CU: the last size at which the small tiles are the faster ones whatever K is
+// (512 of them: 512 x 4096 fp4 with K = 512 / 4096 / 14336 16.2 -> 8.3, 40.0 -> 27.6, 104 -> 76 us; at
+// 1024 a second wave of them costs what the 256 x 256 kernels' whole call does).  One type, scales of one
+// float per block side by side, whole runs of 4 blocks.
+bool mx_tiles_pay(const mx_params& p, int64_t batch)
+{
+    const bool compact = p.sa_elem == 0 && p.sb_elem == 0 && p.sa_block == 1 && p.sb_block == 1;
+    const int64_t lim  = (int64_t)1 << 31;
+    return p.a4 == p.b4 && compact && p.nblk % 4 == 0 && p.m * p.lda < lim && p.n * p.ldb < lim &&
+           mx_small_tiles(p, batch) <= 512;
+}
+
 size_t align16(size_t x) { return (x + 15) / 16 * 16; }
 
 // The flag word of the workspace is never cleared: a call raises it by writing its own number, and
@@ -380,6 +637,19 @@ extern "C" int mi355_quant_dot_mx(const mi355_mx_dot_desc* d,
                mi355_dma_mx_supported(d->m, d->n, a_row, d->lda, d->ldb, d->ldc, d->stride_a, d->stride_b, a, b);
     p.group = p.staged && !a4 ? 2 : 4;
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const int64_t etiles = (int64_t)d->batch * ((d->n + 15) / 16) * ((d->m + 15) / 16);
+    const dim3 exact_grid((unsigned)(etiles < 2048 ? etiles : 2048));
+    if(mx_tiles_pay(p, d->batch))
+    {
+        const int tm = (p.m + 63) / 64, tn = (p.n + 63) / 64;
+        const dim3 tile_grid((unsigned)(tm * tn), (unsigned)d->batch);
+        if(a4)
+            hipLaunchKernelGGL(mx_tile_kernel<true>, tile_grid, dim3(256), 0, s, p, tm, tn);
+        else
+            hipLaunchKernelGGL(mx_tile_kernel<false>, tile_grid, dim3(256), 0, s, p, tm, tn);
+        hipLaunchKernelGGL(mx_exact_kernel, exact_grid, dim3(256), 0, s, p, (int)d->batch);
+        return mi355_launch_status();
+    }
     const int64_t most = (int64_t)d->batch * (d->m > d->n ? d->m : d->n) * ((p.nblk + p.group - 1) / p.group);
     hipLaunchKernelGGL(mx_prepare_kernel, dim3((unsigned)((most + 255) / 256), 2), dim3(256), 0, s, p, (int)d->batch);
     const dim3 grid((unsigned)((d->n + 127) / 128), (unsigned)((d->m + 127) / 128), (unsigned)d->batch);
@@ -398,8 +668,6 @@ extern "C" int mi355_quant_dot_mx(const mi355_mx_dot_desc* d,
         hipLaunchKernelGGL((mx_gemm_kernel<false, true>), grid, dim3(256), 0, s, p);
     else
         hipLaunchKernelGGL((mx_gemm_kernel<false, false>), grid, dim3(256), 0, s, p);
-    const int64_t etiles = (int64_t)d->batch * ((d->n + 15) / 16) * ((d->m + 15) / 16);
-    hipLaunchKernelGGL(mx_exact_kernel, dim3((unsigned)(etiles < 2048 ? etiles : 2048)), dim3(256), 0, s, p,
-                       (int)d->batch);
+    hipLaunchKernelGGL(mx_exact_kernel, exact_grid, dim3(256), 0, s, p, (int)d->batch);
     return mi355_launch_status();
 }
