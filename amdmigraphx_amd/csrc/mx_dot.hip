@@ -283,9 +283,10 @@ __global__ __launch_bounds__(256) void mx_gemm_kernel(mx_params p)
 // ---- small tiles, scales read as they are ----------------------------------------------------------
 // The 256 x 256 staged kernels need a grid of them: 512 x 4096 x 4096 is 32 workgroups on 256 CUs.  This
 // kernel has tiles of 64 x 64 (a wave 32 x 32), register-staged through two LDS stages with the loads
-// of the next two slabs in flight, and reads the float scales of one value per block itself: the exponent is a shift, and a lane that meets anything but a normal power of two
-// raises the call's flag as mx_prepare_kernel does (the exact kernel behind it then computes the
-// result), so the prepare launch and its pass over the scales are gone.
+// of the next two slabs in flight, and reads the float scales of one value per block itself: the
+// exponent is a shift, and a lane that meets anything but a normal power of two raises the call's flag
+// as mx_prepare_kernel does (the exact kernel behind it then computes the result), so the prepare
+// launch and its pass over the scales are gone.
 // What bounds it is the latency of a slab and the rate at which a workgroup pulls its operands in.
 // Measured, all launches of a call, fp4 / fp8: 512 x 4096 x 4096 40.0 -> 27.6 / 59.5 -> 44.6 us, 16 x 4096 x 4096
 // 35.6 -> 13.3 / 51.2 -> 18.3, 128 x 4096 x 14336 101 -> 41 / 154 -> 71.  (Slabs of 256 bytes need more
@@ -399,7 +400,7 @@ __global__ __launch_bounds__(256, 2) void mx_tile_kernel(mx_params p, int tiles_
         }
     };
     // a positive normal power of two has neither sign nor mantissa, and an exponent of 1 .. 254
-    uint32_t bad     = 0;
+    uint32_t bad   = 0;
     auto exponents = [&](const uint32_t (&bits)[NB]) {
         uint32_t packed = 0;
 #pragma unroll
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(256, 2) void mx_tile_kernel(mx_params p, int tiles_
                 return v8i{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
             }
         };
-auto one = [&](auto step) {
+        auto one = [&](auto step) {
             constexpr int h = decltype(step)::value;
             if constexpr(h < NB)
             {
