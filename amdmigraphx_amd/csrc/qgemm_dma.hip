@@ -4644,6 +4644,41 @@ size_t mi355_dma_gemm_workspace(const mi355_quant_dot_desc* d)
     return s > 1 ? (size_t)s * d->batch * d->m * ((d->n + 3) / 4 * 4) * 4 : 0;
 }
 
+// Shares of K in which mi355_dma_gemm_launch works on this call, 1 for one pass; *atomic: they are added
+// into C with integer atomics (the bare int8 product), else they go through the workspace.
+int mi355_dma_gemm_shares(const mi355_quant_dot_desc* d,
+                          const void* c,
+                          const void* workspace,
+                          size_t workspace_bytes,
+                          bool* atomic)
+{
+    *atomic          = false;
+    const size_t esz = d->dequant ? mi355_dtype_size(d->out_type) : 4;
+    const bool vec   = d->n % 4 == 0 && d->ldc % 4 == 0 && d->stride_c % 4 == 0 &&
+                     reinterpret_cast<uintptr_t>(c) % (4 * esz) == 0;
+    const bool room  = workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % 16 == 0;
+    if(d->in_type == MI355_FP8)
+    {
+        const int s = room && vec ? fp8_shares(d) : 1;
+        return s > 1 && (size_t)s * d->m * d->n * 4 <= workspace_bytes ? s : 1;
+    }
+    const int tiles = (int)(((d->m + BM - 1) / BM) * ((d->n + BN - 1) / BN));
+    const int nk    = (int)(d->k / BK);
+    if(room && d->scale_b_mode != MI355_QP_PER_COL_BATCH)
+    {
+        const int s = choose_ksplit_ws(tiles, (int)d->batch, nk, d->m, d->n, d->k);
+        if(s > 1 && (size_t)s * d->batch * d->m * ((d->n + 3) / 4 * 4) * 4 <= workspace_bytes)
+            return s;
+    }
+    if(vec && !d->dequant)
+    {
+        const int s = choose_ksplit(tiles, (int)d->batch, nk, d->m, d->n, d->k);
+        *atomic     = s > 1;
+        return s;
+    }
+    return 1;
+}
+
 int mi355_dma_gemm_launch(const mi355_quant_dot_desc* d,
                           const void* a,
                           const void* b,
@@ -4706,34 +4741,31 @@ int mi355_dma_gemm_launch(const mi355_quant_dot_desc* d,
         p.vec_cols = d->n % 4 == 0 && (p.scale_b_mode != MI355_QP_PER_COL || aligned16(scale_b)) &&
                      (d->zp_a == 0 || aligned16(colsum_b)) && (bias == nullptr || aligned16(bias));
     }
-    p.ksplit = 1;
-    if(fp8 && workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && p.vec_store &&
-       d->n % 4 == 0)
+    bool atomic      = false;
+    const int shares = mi355_dma_gemm_shares(d, c, workspace, workspace_bytes, &atomic);
+    p.ksplit         = 1;
+    if(fp8 && shares > 1)
     {
         // Split K through the batch index: share z is the bare product of A[:, z*kz : (z+1)*kz]
         // and the matching rows of B, written to partial[z] (the kernel itself is unchanged);
         // the second kernel adds the shares and applies the epilogue.
-        const int s = fp8_shares(d);
-        if(s > 1 && (size_t)s * d->m * d->n * 4 <= workspace_bytes)
-        {
-            dma_params q = p;
-            q.k          = p.k / s;
-            q.c          = workspace;
-            q.ldc        = d->n;
-            q.stride_c   = d->m * d->n;
-            q.stride_a   = q.k;
-            q.stride_b   = d->trans_b ? (int64_t)q.k : (int64_t)q.k * d->ldb;
-            q.vec_store  = 1;
-            q.vec8_store = 0;
-            q.bias       = nullptr;
-            const int st = d->trans_b ? launch_out<true, true>(q, s, false, MI355_F32, stream)
-                                      : launch_out<true, false>(q, s, false, MI355_F32, stream);
-            if(st != MI355_OK)
-                return st;
-            p.ksplit  = s;
-            p.partial = static_cast<int32_t*>(workspace);
-            return launch_reduce<true>(p, 1, s, deq, d->out_type, stream);
-        }
+        dma_params q = p;
+        q.k          = p.k / shares;
+        q.c          = workspace;
+        q.ldc        = d->n;
+        q.stride_c   = d->m * d->n;
+        q.stride_a   = q.k;
+        q.stride_b   = d->trans_b ? (int64_t)q.k : (int64_t)q.k * d->ldb;
+        q.vec_store  = 1;
+        q.vec8_store = 0;
+        q.bias       = nullptr;
+        const int st = d->trans_b ? launch_out<true, true>(q, shares, false, MI355_F32, stream)
+                                  : launch_out<true, false>(q, shares, false, MI355_F32, stream);
+        if(st != MI355_OK)
+            return st;
+        p.ksplit  = shares;
+        p.partial = static_cast<int32_t*>(workspace);
+        return launch_reduce<true>(p, 1, shares, deq, d->out_type, stream);
     }
     if(fp8)
         return d->trans_b ? launch_out<true, true>(p, (int)d->batch, deq, d->out_type, stream)
@@ -4744,30 +4776,17 @@ int mi355_dma_gemm_launch(const mi355_quant_dot_desc* d,
     const size_t osz = deq ? mi355_dtype_size(d->out_type) : 4;
     const bool vec   = d->n % 4 == 0 && d->ldc % 4 == 0 && d->stride_c % 4 == 0 &&
                      reinterpret_cast<uintptr_t>(c) % (4 * osz) == 0;
-    if(workspace != nullptr && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && !cols_per_batch &&
-       (!deq || d->out_type == MI355_F32 || d->out_type == MI355_F16 || d->out_type == MI355_BF16))
+    if(shares > 1)
     {
-        const int s = choose_ksplit_ws(p.tiles_m * p.tiles_n, (int)d->batch, p.k / BK, d->m, d->n, d->k);
-        if(s > 1 && (size_t)s * d->batch * d->m * p.partial_ld * 4 <= workspace_bytes)
-        {
-            p.ksplit  = s;
-            p.partial = static_cast<int32_t*>(workspace);
-            return d->trans_b ? launch_i8_splitk<true>(p, (int)d->batch, stream, deq, d->out_type)
-                              : launch_i8_splitk<false>(p, (int)d->batch, stream, deq, d->out_type);
-        }
+        p.ksplit  = shares;
+        p.partial = atomic ? nullptr : static_cast<int32_t*>(workspace);
+        return d->trans_b ? launch_i8_splitk<true>(p, (int)d->batch, stream, deq, d->out_type)
+                          : launch_i8_splitk<false>(p, (int)d->batch, stream, deq, d->out_type);
     }
     if(d->n % 4 != 0)
         // the 16 x 16 kernel drops or keeps 4 columns together
         return d->trans_b ? launch_out<false, true>(p, (int)d->batch, deq, d->out_type, stream)
                           : launch_out<false, false>(p, (int)d->batch, deq, d->out_type, stream);
-    p.ksplit = 1;
-    if(vec && !deq)
-    {
-        p.ksplit = choose_ksplit(p.tiles_m * p.tiles_n, (int)d->batch, p.k / BK, d->m, d->n, d->k);
-        if(p.ksplit > 1)
-            return d->trans_b ? launch_i8_splitk<true>(p, (int)d->batch, stream)
-                              : launch_i8_splitk<false>(p, (int)d->batch, stream);
-    }
     if(vec)
         return d->trans_b ? launch_i8_out<true, true>(p, (int)d->batch, deq, d->out_type, stream)
                           : launch_i8_out<false, true>(p, (int)d->batch, deq, d->out_type, stream);

@@ -614,7 +614,8 @@ bool mi355_ragged_gemm_supported(const mi355_quant_dot_desc* d)
     if(d->in_type == MI355_FP8 && d->k > 32768)
         return false;
     const int64_t lim = (int64_t)1 << 31;
-    if(d->m >= lim / 256 || d->n >= lim / 256 || d->lda >= lim || d->ldb >= lim || d->k >= lim - 256)
+    // positions along K are ints and run up to two slabs of 256 and a row of pieces past the end
+    if(d->m >= lim / 256 || d->n >= lim / 256 || d->lda >= lim || d->ldb >= lim || d->k >= lim - 1024)
         return false;
     return d->m * d->lda < lim && (d->trans_b ? d->n * d->ldb : d->k * d->ldb) < lim &&
            ((d->m + 63) / 64) * ((d->n + 63) / 64) < lim;

@@ -42,6 +42,7 @@ int mi355_dma_gemm_launch(const mi355_quant_dot_desc*,
                           size_t,
                           hipStream_t);
 size_t mi355_dma_gemm_workspace(const mi355_quant_dot_desc*);
+int mi355_dma_gemm_shares(const mi355_quant_dot_desc*, const void*, const void*, size_t, bool*);
 
 namespace {
 
@@ -305,18 +306,34 @@ extern "C" size_t mi355_quant_dot_workspace_size(const mi355_quant_dot_desc* d)
     return d == nullptr ? 0 : mi355_dma_gemm_workspace(d);
 }
 
-extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
-                                  const void* a,
-                                  const void* b,
-                                  void* c,
-                                  const float* scale_a,
-                                  const float* scale_b,
-                                  const int32_t* colsum_b,
-                                  const int32_t* rowsum_a,
-                                  const float* bias,
-                                  void* workspace,
-                                  size_t workspace_bytes,
-                                  void* stream)
+namespace {
+
+// which kernel a call runs
+enum class kernel_id : int
+{
+    none         = 0, // nothing to compute
+    generic      = 1,
+    ragged       = 2, // register-staged; fp8 sums in float
+    ragged_exact = 3, // fp8 sums exact
+    mfma         = 4,
+    dma          = 5, // direct-to-LDS, one pass over K
+    dma_shares   = 6, // K in shares through the workspace
+    dma_atomic   = 7  // K in shares added into C
+};
+
+// argument checks and the choice of the kernel; the pointers are looked at, not through
+int choose_kernel(const mi355_quant_dot_desc* d,
+                  const void* a,
+                  const void* b,
+                  const void* c,
+                  const float* scale_a,
+                  const float* scale_b,
+                  const int32_t* colsum_b,
+                  const int32_t* rowsum_a,
+                  const float* bias,
+                  const void* workspace,
+                  size_t workspace_bytes,
+                  kernel_id* kernel)
 {
     if(d == nullptr)
         return MI355_ERR_BAD_ARG;
@@ -368,6 +385,7 @@ extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
         if(d->out_type != (fp8 ? MI355_F32 : MI355_I32))
             return MI355_ERR_BAD_ARG;
     }
+    *kernel = kernel_id::none;
     if(empty)
         return MI355_OK;
     if(d->ldc < d->n)
@@ -377,7 +395,6 @@ extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
     if(d->batch > 65535)
         return MI355_ERR_UNSUPPORTED;
 
-    hipStream_t s = static_cast<hipStream_t>(stream);
     // int8 with N % 4 != 0 would take the DMA path's 32 x 32 kernel, which applies no bias
     const bool dma_has_bias = bias == nullptr || fp8 || d->n % 4 == 0;
     if(!u8 && !bf8 && d->k > 0 && dma_has_bias && mi355_dma_gemm_supported(d, a, b))
@@ -386,22 +403,90 @@ extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
         const size_t split = mi355_dma_gemm_workspace(d);
         const bool room    = workspace != nullptr && split > 0 && split <= workspace_bytes;
         const double shares = room ? (double)split / (4.0 * (double)d->batch * (double)d->m * (double)d->n) : 1.0;
+        bool atomic         = false;
         if(ragged_is_faster(d, dma_us(d, shares)))
-            return mi355_ragged_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, true, s);
-        return mi355_dma_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace, workspace_bytes, s);
+            *kernel = kernel_id::ragged;
+        else if(mi355_dma_gemm_shares(d, c, workspace, workspace_bytes, &atomic) > 1)
+            *kernel = atomic ? kernel_id::dma_atomic : kernel_id::dma_shares;
+        else
+            *kernel = kernel_id::dma;
+        return MI355_OK;
     }
     // a vector of column scales per batch entry exists in the kernels above only
     if(d->dequant && d->scale_b_mode == MI355_QP_PER_COL_BATCH)
         return MI355_ERR_UNSUPPORTED;
     if(!u8 && d->k > 0 && mi355_mfma_gemm_supported(d, a, b, c))
     {
-        if(!bf8 && ragged_is_faster(d, mfma_us(d)))
-            return mi355_ragged_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, true, s);
-        return mi355_mfma_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, s);
+        *kernel = !bf8 && ragged_is_faster(d, mfma_us(d)) ? kernel_id::ragged : kernel_id::mfma;
+        return MI355_OK;
     }
-    // rows aligned to nothing; fp8 sums stay exact there, as in the kernel below
+    // rows aligned to nothing; fp8 sums stay exact there, as in the generic kernel
     if(mi355_ragged_gemm_supported(d))
-        return mi355_ragged_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, false, s);
+    {
+        *kernel = kernel_id::ragged_exact;
+        return MI355_OK;
+    }
+    *kernel = kernel_id::generic;
+    return (d->m + 15) / 16 > 65535 ? MI355_ERR_UNSUPPORTED : MI355_OK;
+}
+
+} // namespace
+
+// The kernel_id of a call, or its (negative) status.  Not part of the public interface: tests ask it,
+// without a GPU, which kernel their shapes reach.
+extern "C" int mi355_internal_quant_dot_kernel(const mi355_quant_dot_desc* d,
+                                               const void* a,
+                                               const void* b,
+                                               const void* c,
+                                               const float* scale_a,
+                                               const float* scale_b,
+                                               const int32_t* colsum_b,
+                                               const int32_t* rowsum_a,
+                                               const float* bias,
+                                               const void* workspace,
+                                               size_t workspace_bytes)
+{
+    kernel_id kernel = kernel_id::none;
+    const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
+                                     workspace_bytes, &kernel);
+    return status == MI355_OK ? (int)kernel : status;
+}
+
+extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
+                                  const void* a,
+                                  const void* b,
+                                  void* c,
+                                  const float* scale_a,
+                                  const float* scale_b,
+                                  const int32_t* colsum_b,
+                                  const int32_t* rowsum_a,
+                                  const float* bias,
+                                  void* workspace,
+                                  size_t workspace_bytes,
+                                  void* stream)
+{
+    kernel_id kernel = kernel_id::none;
+    const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
+                                     workspace_bytes, &kernel);
+    if(status != MI355_OK)
+        return status;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    switch(kernel)
+    {
+    case kernel_id::none: return MI355_OK;
+    case kernel_id::ragged:
+    case kernel_id::ragged_exact:
+        return mi355_ragged_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias,
+                                        kernel == kernel_id::ragged, s);
+    case kernel_id::mfma:
+        return mi355_mfma_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, s);
+    case kernel_id::dma:
+    case kernel_id::dma_shares:
+    case kernel_id::dma_atomic:
+        return mi355_dma_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
+                                     workspace_bytes, s);
+    case kernel_id::generic: break;
+    }
 
     generic_params p;
     p.a            = static_cast<const uint8_t*>(a);
@@ -427,13 +512,11 @@ extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
     p.scale_b_mode = d->scale_b_mode;
     p.zp_a         = d->zp_a;
     p.zp_b         = d->zp_b;
-    p.fp8          = bf8 ? 2 : (fp8 ? 1 : 0);
-    p.is_unsigned  = u8;
+    p.fp8          = d->in_type == MI355_BF8 ? 2 : d->in_type == MI355_FP8 ? 1 : 0;
+    p.is_unsigned  = d->in_type == MI355_U8;
     p.dequant      = d->dequant;
     p.out_type     = d->out_type;
     const int64_t gx = (d->n + 15) / 16, gy = (d->m + 15) / 16;
-    if(gy > 65535)
-        return MI355_ERR_UNSUPPORTED;
     dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)d->batch);
     hipLaunchKernelGGL(quant_dot_generic_kernel, grid, dim3(256), 0, s, p);
     return mi355_launch_status();
