@@ -617,8 +617,11 @@ bool mi355_ragged_gemm_supported(const mi355_quant_dot_desc* d)
     // positions along K are ints and run up to two slabs of 256 and a row of pieces past the end
     if(d->m >= lim / 256 || d->n >= lim / 256 || d->lda >= lim || d->ldb >= lim || d->k >= lim - 1024)
         return false;
+    // a grid holds less than 2^32 threads along x; int8 results that large take tiles of 128 x 128
+    const int64_t side  = d->in_type == MI355_I8 ? 128 : 64;
+    const int64_t tiles = ((d->m + side - 1) / side) * ((d->n + side - 1) / side);
     return d->m * d->lda < lim && (d->trans_b ? d->n * d->ldb : d->k * d->ldb) < lim &&
-           ((d->m + 63) / 64) * ((d->n + 63) / 64) < lim;
+           tiles < ((int64_t)1 << 32) / THREADS;
 }
 
 int mi355_ragged_gemm_launch(const mi355_quant_dot_desc* d,

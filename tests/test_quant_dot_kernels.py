@@ -18,3 +18,13 @@ def test_register_staged_kernel_keeps_room_for_its_read_ahead():
     furthest = ((last + 255) // 256 + 1) * 256 + 240
     assert furthest < 2**31
     assert kernel_of(1, 1, last, trans_b=True) == "ragged_exact"
+
+
+def test_register_staged_kernel_keeps_to_the_largest_grid():
+    """2^24 workgroups of 256 threads are more than one launch takes; 180 GB of bfloat16 results still fit the card."""
+    m = 300001
+    assert (m + 63) // 64 * ((m + 63) // 64) * 256 >= 2**32
+    assert kernel_of(m, m, 17, fp8=True, out="bf16") == "generic"
+    assert kernel_of(250001, 250001, 17, fp8=True, out="bf16") == "ragged_exact"
+    assert (m + 127) // 128 * ((m + 127) // 128) * 256 < 2**32
+    assert kernel_of(m, m, 17, out="bf16") == "ragged_exact"
