@@ -420,8 +420,9 @@ def quantizelinear(x, scale, zp=None, out_type=DT.I8):
     out = torch.empty(x.shape, dtype=_DT2TORCH[out_type], device=x.device)
     ssr, ssc = _qparam_strides(scale, rows, cols)
     zsr, zsc = _qparam_strides(zp, rows, cols)
-    st = lib().mi355_quantizelinear(_ptr(x), _TORCH2DT[x.dtype], _ptr(scale.contiguous()), ssr, ssc,
-                                    _ptr(None if zp is None else zp.contiguous()), zsr, zsc,
+    # named: a dense copy of a strided parameter has to live until the launch
+    scale, zp = scale.contiguous(), None if zp is None else zp.contiguous()
+    st = lib().mi355_quantizelinear(_ptr(x), _TORCH2DT[x.dtype], _ptr(scale), ssr, ssc, _ptr(zp), zsr, zsc,
                                     _ptr(out), out_type, rows, cols, _stream())
     check(st, "mi355_quantizelinear")
     return out
@@ -436,9 +437,9 @@ def dequantizelinear(x, scale, zp=None, x_type=None):
     out = torch.empty(x.shape, dtype=scale.dtype, device=x.device)
     ssr, ssc = _qparam_strides(scale, rows, cols)
     zsr, zsc = _qparam_strides(zp, rows, cols)
-    st = lib().mi355_dequantizelinear(_ptr(x), xt, _ptr(scale.contiguous()), _TORCH2DT[scale.dtype],
-                                      ssr, ssc, _ptr(None if zp is None else zp.contiguous()),
-                                      zsr, zsc, _ptr(out), rows, cols, _stream())
+    scale, zp = scale.contiguous(), None if zp is None else zp.contiguous()
+    st = lib().mi355_dequantizelinear(_ptr(x), xt, _ptr(scale), _TORCH2DT[scale.dtype], ssr, ssc, _ptr(zp), zsr, zsc,
+                                      _ptr(out), rows, cols, _stream())
     check(st, "mi355_dequantizelinear")
     return out
 

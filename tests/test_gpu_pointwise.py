@@ -226,3 +226,18 @@ def test_fp4_unpack_and_pack_match_oracle(ops):
     from amdmigraphx_amd import Mi355Error
     with pytest.raises(Mi355Error):
         ops.pack_fp4(dev(np.zeros((2, 3), np.float32)))
+
+
+@pytest.mark.parametrize("rows,cols", [(100, 7), (128, 64)])
+def test_strided_scales_and_zero_points(ops, rows, cols):
+    """Both parameters are views with a stride: each is made dense for the call, and the copy of the scales has to
+    live until the kernel is launched (the allocator hands a block that is given back to the next copy)."""
+    rng = np.random.default_rng(rows)
+    x = rng.standard_normal((rows, cols)).astype(np.float32) * 10
+    scale = rng.uniform(0.1, 0.5, (rows, 3)).astype(np.float32)
+    zp = rng.integers(-100, 100, (rows, 5), dtype=np.int8)
+    ds, dz = dev(scale)[:, 1], dev(zp)[:, 2]
+    codes = orc.quantizelinear(x, scale[:, 1:2], zp[:, 2:3], orc.F32, orc.I8)
+    assert np.array_equal(ops.quantizelinear(dev(x), ds, dz).cpu().numpy(), codes)
+    want = orc.dequantizelinear(codes, scale[:, 1:2], zp[:, 2:3], orc.I8, orc.F32)
+    assert np.array_equal(ops.dequantizelinear(dev(codes), ds, dz).cpu().numpy(), want)
