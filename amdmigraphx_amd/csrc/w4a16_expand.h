@@ -66,7 +66,8 @@ __global__ __launch_bounds__(256) void w4a16_expand_kernel(w4_params p, v4u* out
 // kernel, which needs no workspace for weights.
 int expand_gemm_shares(int64_t m, int64_t n, int64_t k)
 {
-    if(m <= 256 || n % TL_BN != 0 || k < 1536 || k > (1 << 18))
+    // (dense rows at aligned addresses: what a caller that asks for the size alone is taken to have)
+    if(m <= 256 || n % TL_BN != 0 || k > (1 << 18) || !mi355_dma_half_supported(m, n, k, k, n, nullptr, nullptr))
         return 0;
     const int64_t big   = ((m + 255) / 256) * ((n + 255) / 256);
     const int64_t small = ((m + 63) / 64) * (n / TL_BN);

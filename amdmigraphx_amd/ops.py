@@ -527,8 +527,8 @@ def convert(x, out_type, in_type=None):
 def w4a16_gemm(a, w_packed, scales, group, zp=8, zp_mode=None, out=None, workspace=None):
     """fp16 activations [M, K] times int4 weights packed [N, K/2] with fp16
     group scales [N, K/group]; zp is an int (per tensor) or a uint8 tensor.
-    ``workspace`` (a dense device tensor, see w4a16_gemm_workspace_size) lets shapes whose
-    column tiles do not fill the chip split K."""
+    ``workspace`` (a dense device tensor, see w4a16_gemm_workspace_size) lets many rows multiply
+    weights dequantized once, and shapes whose column tiles do not fill the chip split K."""
     _require_cuda(a, w_packed, scales, workspace)
     m, k = a.shape
     n = w_packed.shape[0]
@@ -584,5 +584,6 @@ def w4a16_gemm_prepacked(a, prepacked, n, out=None):
 
 
 def w4a16_gemm_workspace_size(m, n, k, group):
-    """Bytes of workspace w4a16_gemm can use for that shape (0: none)."""
+    """Bytes of workspace w4a16_gemm can use for that shape (0: none): room for the sums of a split K, or for
+    many rows 2 bytes a weight."""
     return int(lib().mi355_w4a16_gemm_workspace_size(m, n, k, group))

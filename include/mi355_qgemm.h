@@ -394,13 +394,16 @@ int mi355_w4a16_gemm(const void* a, int64_t lda,
                      int64_t m, int64_t n, int64_t k, int64_t group,
                      void* stream);
 
-/* The same with a workspace.  Where the column tiles alone do not fill the chip (more than 32
- * rows against N / 128 tiles; 2..64 rows against few 64-column tiles and K >= 8192) the kernels
- * split K over more workgroups when they have room for the float partial sums; a second kernel
- * adds them in a fixed order and converts to half.  Deterministic, within the path's fp tolerance
- * of the unsplit result (another order of fp32 additions).  mi355_w4a16_gemm_workspace_size gives
- * the bytes the shape can use (0: none); a NULL or smaller workspace is not an error.  16-byte
- * aligned device memory, free again when the call's work is done. */
+/* The same with a workspace, which serves one of two ends.  Many rows (about a thousand and more): the weights
+ * are written into it once, as the half values the operator's dequantizelinear gives (2 bytes a
+ * weight, and float partial sums where K is split), and multiplied as halves.  Otherwise, where the column
+ * tiles alone do not fill the chip (more than 32 rows against N / 128 tiles; 2..64 rows against few
+ * 64-column tiles and K >= 8192), the kernels split K over more workgroups when they have room for
+ * the float partial sums; a second kernel adds them in a fixed order and converts to half.
+ * Deterministic, within the path's fp tolerance of the result without a workspace (another order of
+ * fp32 additions).  mi355_w4a16_gemm_workspace_size gives the bytes the shape can use (0: none); a
+ * NULL or smaller workspace is not an error, the call then runs without.  16-byte aligned device
+ * memory, free again when the call's work is done. */
 size_t mi355_w4a16_gemm_workspace_size(int64_t m, int64_t n, int64_t k, int64_t group);
 int mi355_w4a16_gemm_ws(const void* a, int64_t lda,
                         const void* w_packed,

@@ -49,3 +49,24 @@ def test_many_rows(ops, m, n, k, pad, group, zeros):
     bound = (x.double().abs() @ w.t().abs()) * (k * 2.0**-24) + want.abs() * 2.0**-10 + 2.0**-24
     assert bool(((got.double() - want).abs() <= bound).all())
     assert pad == 0 or bool((out[:, n:] == -1).all())
+
+
+def test_a_workspace_one_byte_short_is_left_alone(ops):
+    """the call falls back to the tiles that dequantize for themselves, with the same result up to the order of sums"""
+    m, n, k, group = 1000, 3968, 9216, 128
+    need = ops.w4a16_gemm_workspace_size(m, n, k, group)
+    assert need > 2 * n * k
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(m, k, generator=g, device="cuda").half()
+    w = torch.randint(0, 256, (n, k // 2), generator=g, dtype=torch.uint8, device="cuda")
+    scales = (torch.rand(n, k // group, generator=g, device="cuda") * 0.015 + 0.005).half()
+    room = torch.full((need,), 0x5a, dtype=torch.uint8, device="cuda")
+    short = ops.w4a16_gemm(x, w, scales, group, workspace=room[:-1])
+    assert bool((room == 0x5a).all())
+    whole = ops.w4a16_gemm(x, w, scales, group, workspace=room)
+    assert not bool((room[:2 * n * k] == 0x5a).all())
+    # k float32 additions in either order, and the cut to 11 bits twice
+    dense = torch.stack([w & 15, w >> 4], dim=2).reshape(n, -1, group).float() - 8
+    dense = (dense * scales.float()[:, :, None]).reshape(n, k).abs().double()
+    bound = 2 * (x.double().abs() @ dense.t()) * (k * 2.0**-24) + whole.double().abs() * 2.0**-9 + 2.0**-23
+    assert bool(((short.double() - whole.double()).abs() <= bound).all())
