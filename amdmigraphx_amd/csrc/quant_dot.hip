@@ -208,61 +208,109 @@ __global__ __launch_bounds__(256) void colsum_rowmajor_kernel(
     atomicAdd(out + col, s);
 }
 
-// What a product takes (us) in the kernels that compete for it, fitted to measurements on one MI355X of
-// 1 to 384 batches, M and N of 16 to 16384, K of 64 to 8208, both types and both orders of B.
-//
-// The register-staged kernel (qgemm_ragged.hip) has tiles of 64 x 64, or 128 x 128 where those fill
-// the chip; a workgroup of it starts sooner and several share a CU, so it wins wherever the 256 x 256
-// tiles of the other two leave CUs idle or are mostly padding, and where K is short:
+// What a product takes (us) in the kernels that compete for it, fitted to 11800 products on one MI355X: M
+// of 1 to 4096, N of 16 to 28672, K of 16 to 28672 over weights that no cache holds, and 2 to 384
+// batches that one may hold; both types, both orders of B, with and without epilogue and workspace.
+// Nine products in ten take 0.9 to 1.15 times their fit (shares added into C: 0.8 to 1.3).
+//   fixed       launch, and the first loads' way
+//   wave        a round of workgroups over the chip: a tile's prologue and epilogue, and `rows` for the part
+//               of the epilogue that a tile's rows and columns fill
+//   k_wave      per step of K in every round; k_fill: and in proportion to the workgroups, not the rounds
+//   b_mb, out_m per MB of B from memory, per million outputs
+struct fit
+{
+    double fixed, wave, rows, k_wave, k_fill, b_mb, out_m;
+};
+
+double fitted_us(const fit& f, const mi355_quant_dot_desc* d, double fill, double rows, double k)
+{
+    const double waves = __builtin_ceil(fill);
+    return f.fixed + waves * (f.wave + rows * f.rows + k * f.k_wave) + fill * k * f.k_fill +
+           (double)d->batch * (double)d->n * (double)d->k * 1e-6 * f.b_mb +
+           (double)d->batch * (double)d->m * (double)d->n * 1e-6 * f.out_m;
+}
+
+// tiles of a product; the share of a tile's or wave's `side` that a dimension fills
+double tiles_of(const mi355_quant_dot_desc* d, int64_t side)
+{
+    return (double)d->batch * (double)((d->m + side - 1) / side) * (double)((d->n + side - 1) / side);
+}
+
+double part(int64_t dim, double side) { return __builtin_fmin((double)dim, side) / side; }
+
+// The register-staged kernel (qgemm_ragged.hip), tiles of 64 x 64, or 128 x 128 where those fill the chip.  A
+// workgroup of it starts sooner and several share a CU, so it wins wherever the 256 x 256 tiles of
+// the other two leave CUs idle or are mostly padding, and where K is short:
 //   96 batches of 197 x 197 x 64 int8 -> float   23.7 -> 11.3 us     384 of 64 x 64 x 64   19.7 -> 8.2
 //   1024 x 1024 x 1024 int8 -> bfloat16          23.5 -> 6.5         512 x 4096 x 4096 (split)   30.9 -> 21.3
 //   48 x 1024 x 1024 x 128                       49.8 against 53.7 (stays)
+// It never splits K: few tiles of a long K stay with shares (5 x 192 x 25472 int8: 79.9 against 16.4 us).
 double ragged_us(const mi355_quant_dot_desc* d)
 {
-    auto tiles = [&](int64_t t) { return (double)d->batch * (double)((d->m + t - 1) / t) * (double)((d->n + t - 1) / t); };
-    const double small = tiles(64), big = tiles(128);
-    double per_k;
-    if(big < 256) // (the kernel's own choice of the tile)
-        per_k = d->trans_b ? 0.0021 * __builtin_fmax(1.0, small / 256.0 * 0.95)
-                           : 0.0031 * __builtin_fmax(1.0, small / 256.0 * 0.8);
-    else if(big <= 256)
-        per_k = d->trans_b ? 0.0083 : 0.0088;
-    else
-        per_k = (d->trans_b ? 0.0095 : 0.0115) * __builtin_ceil(big / 512.0);
-    const double out = (double)d->batch * (double)d->m * (double)d->n *
-                       (double)(d->dequant ? mi355_dtype_size(d->out_type) : 4);
-    return 3.4 + per_k * (double)d->k + out / 4.0e6;
-}
-
-double waves_of_256(const mi355_quant_dot_desc* d)
-{
-    return __builtin_ceil((double)d->batch * (double)((d->m + 255) / 256) * (double)((d->n + 255) / 256) / 256.0);
-}
-
-// direct-to-LDS kernels; `shares` of K through a workspace
-double dma_us(const mi355_quant_dot_desc* d, double shares)
-{
+    const int deq = d->dequant != 0, tb = d->trans_b != 0;
     const double k = (double)d->k;
-    if(shares > 1.0)
-        return 7.8 + 0.0093 * k / shares +
-               shares * (double)d->batch * (double)d->m * (double)d->n * 8.0 / 5.0e6;
-    if(d->in_type == MI355_FP8)
-        return waves_of_256(d) * (d->k < 3072 ? 8.8 + 0.0093 * k : 14.0 + 0.0081 * k);
-    return waves_of_256(d) * (d->k < 3072 ? 12.8 + 0.0112 * k : 16.0 + 0.0089 * k);
+    // (the kernel's own choice of the tile; two of the large ones share a CU)
+    if(const double big = tiles_of(d, 128); big >= 256)
+    {
+        // [epilogue][B as [N, K]]
+        static const fit large[2][2] = {
+            {{3.8, 0.15, 1.4, 0.0099, 0.0030, 0.120, 0.61}, {3.8, 0.25, 1.3, 0.0082, 0.0027, 0.110, 0.62}},
+            {{3.4, 2.1, 1.8, 0.0080, 0.0052, 0.130, 0.29}, {3.5, 2.2, 1.8, 0.0083, 0.0028, 0.083, 0.33}}};
+        return fitted_us(large[deq][tb], d, big / 512.0, part(d->m, 128.0), k);
+    }
+    // A second workgroup on a CU costs less of K than the first.  Rows of a row-major B that lie a
+    // multiple of 1 KiB apart meet in few of the memory's channels: 16 x 2048 x 8192 34.8 us, where other
+    // N of that size take 29.
+    static const fit small[2][2] = {{{3.4, 0.1, 0.2, 0, 0, 0, 1.04}, {3.4, 0.2, 0.2, 0, 0, 0, 0.90}},
+                                    {{3.95, 0.2, 0.6, 0, 0, 0, 0.63}, {3.95, 0.3, 0.45, 0, 0, 0, 0.68}}};
+    const bool pitched = !tb && d->ldb % 1024 == 0;
+    const double fill  = tiles_of(d, 64) / 256.0;
+    fit f              = small[deq][tb];
+    f.k_wave           = tb ? 0.0016 : pitched ? 0.0018 : 0.0026;
+    f.b_mb             = tb ? 0.080 : fill > 1.0 ? 0.170 : 0.100;
+    const double first = tb ? 0.0020 : pitched ? 0.0036 : 0.0030;
+    return fitted_us(f, d, fill, part(d->m, 64.0), k) + (first - f.k_wave) * k;
+}
+
+// direct-to-LDS kernels; `shares` of K through a workspace, or added into C
+double dma_us(const mi355_quant_dot_desc* d, int shares, bool atomic)
+{
+    // [epilogue]: one pass with eight waves, and with four from K = 3072 on
+    static const fit i8[2]   = {{2.0, 3.5, 0.6, 0.0113, 0.0010, 0.060, 0.49}, {3.2, 2.5, 6.7, 0.0106, 0, 0.120, 0.48}};
+    static const fit i8_4[2] = {{3.8, 0, 11.8, 0.0089, 0.0025, 0.030, 0}, {4.1, 13.2, 2.0, 0.0081, 0.0040, 0.020, 0.05}};
+    static const fit f8[2]   = {{3.9, 0, 2.0, 0.0100, 0, 0.090, 0.92}, {2.7, 3.2, 2.6, 0.0098, 0.0017, 0.070, 0.41}};
+    static const fit f8_4[2] = {{4.7, 8.2, 7.0, 0.0071, 0.0038, 0.073, 0}, {2.0, 11.8, 6.5, 0.0074, 0.0030, 0.073, 0}};
+    static const fit i8_shares = {0, 8.0, 2.7, 0.0098, 0, 0.074, 0.7}, f8_shares = {0, 7.5, 3.1, 0.0087, 0, 0.095, 1.1};
+    const bool fp8     = d->in_type == MI355_FP8;
+    const double fill  = tiles_of(d, 256) * shares / 256.0;
+    const double rows  = part(d->m, 128.0);
+    const double k     = (double)d->k / shares;
+    const double sums  = (double)shares * (double)d->batch * (double)d->m * (double)d->n * 1e-6;
+    if(atomic) // at most two rounds; clearing C, then the slower of the shares and of B's way through so few CUs
+        return __builtin_fmax((double)d->batch * (double)d->n * (double)d->k * 1e-6 * 0.37,
+                              5.3 + 11.3 * rows + k * (0.0129 + 0.003 * fill) + 0.76 * sums + 5.7 * fill);
+    if(shares > 1)
+        return fitted_us(fp8 ? f8_shares : i8_shares, d, fill, rows, k) + (fp8 ? 1.75 : 1.51) * sums;
+    const fit* one = d->k >= 3072 && d->n % 4 == 0 ? (fp8 ? f8_4 : i8_4) : (fp8 ? f8 : i8);
+    return fitted_us(one[d->dequant != 0], d, fill, rows * part(d->n, 64.0), k);
 }
 
 // the matrix-core kernel for K that is no multiple of 64
 double mfma_us(const mi355_quant_dot_desc* d)
 {
-    return waves_of_256(d) * (13.0 + (d->trans_b ? 0.0145 : 0.0165) * (double)d->k);
+    static const fit i8[2] = {{3.2, 1.6, 2.7, 0.0152, 0.0023, 0.080, 0.41}, {3.2, 2.0, 8.7, 0.0153, 0.0015, 0.090, 0.37}};
+    static const fit f8[2] = {{2.1, 2.2, 1.0, 0.0145, 0.0022, 0.120, 0.55}, {3.4, 1.7, 6.7, 0.0149, 0.0010, 0.120, 0.36}};
+    return fitted_us((d->in_type == MI355_FP8 ? f8 : i8)[d->dequant != 0], d, tiles_of(d, 256) / 256.0,
+                     part(d->m, 128.0), (double)d->k);
 }
 
-// a vector of column scales per batch entry exists in the direct-to-LDS kernels only; a fourteenth
-// of the time is left to the fit's error
-bool ragged_is_faster(const mi355_quant_dot_desc* d, double other_us)
+// A vector of column scales per batch entry exists in the direct-to-LDS kernels only.  `left` of the time is
+// left to the fits' errors, a fourteenth, against shares of K a tenth: so 28 of the 11800 products take
+// over 1.05 times what the other kernel does (1.27 at most), and 141 miss a tenth and more.
+bool ragged_is_faster(const mi355_quant_dot_desc* d, double other_us, double left)
 {
     return d->k > 0 && mi355_ragged_gemm_supported(d) &&
-           !(d->dequant && d->scale_b_mode == MI355_QP_PER_COL_BATCH) && ragged_us(d) < 0.93 * other_us;
+           !(d->dequant && d->scale_b_mode == MI355_QP_PER_COL_BATCH) && ragged_us(d) < (1.0 - left) * other_us;
 }
 
 __global__ void zero_i32_kernel(int32_t* p, int64_t n)
@@ -400,16 +448,12 @@ int choose_kernel(const mi355_quant_dot_desc* d,
     if(!u8 && !bf8 && d->k > 0 && dma_has_bias && mi355_dma_gemm_supported(d, a, b))
     {
         // fp8: the sums of both are float
-        const size_t split = mi355_dma_gemm_workspace(d);
-        const bool room    = workspace != nullptr && split > 0 && split <= workspace_bytes;
-        const double shares = room ? (double)split / (4.0 * (double)d->batch * (double)d->m * (double)d->n) : 1.0;
-        bool atomic         = false;
-        if(ragged_is_faster(d, dma_us(d, shares)))
-            *kernel = kernel_id::ragged;
-        else if(mi355_dma_gemm_shares(d, c, workspace, workspace_bytes, &atomic) > 1)
-            *kernel = atomic ? kernel_id::dma_atomic : kernel_id::dma_shares;
-        else
-            *kernel = kernel_id::dma;
+        bool atomic      = false;
+        const int shares = mi355_dma_gemm_shares(d, c, workspace, workspace_bytes, &atomic);
+        *kernel          = ragged_is_faster(d, dma_us(d, shares, atomic), shares > 1 ? 0.1 : 0.07) ? kernel_id::ragged
+                           : shares == 1                                  ? kernel_id::dma
+                           : atomic                                       ? kernel_id::dma_atomic
+                                                                          : kernel_id::dma_shares;
         return MI355_OK;
     }
     // a vector of column scales per batch entry exists in the kernels above only
@@ -417,7 +461,7 @@ int choose_kernel(const mi355_quant_dot_desc* d,
         return MI355_ERR_UNSUPPORTED;
     if(!u8 && d->k > 0 && mi355_mfma_gemm_supported(d, a, b, c))
     {
-        *kernel = !bf8 && ragged_is_faster(d, mfma_us(d)) ? kernel_id::ragged : kernel_id::mfma;
+        *kernel = !bf8 && ragged_is_faster(d, mfma_us(d), 0.07) ? kernel_id::ragged : kernel_id::mfma;
         return MI355_OK;
     }
     // rows aligned to nothing; fp8 sums stay exact there, as in the generic kernel

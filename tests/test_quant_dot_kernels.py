@@ -28,3 +28,43 @@ def test_register_staged_kernel_keeps_to_the_largest_grid():
     assert kernel_of(250001, 250001, 17, fp8=True, out="bf16") == "ragged_exact"
     assert (m + 127) // 128 * ((m + 127) // 128) * 256 < 2**32
     assert kernel_of(m, m, 17, out="bf16") == "ragged_exact"
+
+
+@pytest.mark.parametrize("m,n,k,trans_b,kernel", [
+    # bare int8 without a workspace: few tiles of a long K are split over the chip with atomic adds ...
+    (16, 8192, 8192, False, "dma_atomic"), (16, 2048, 8192, True, "dma_atomic"), (16, 256, 25600, False, "dma_atomic"),
+    (16, 256, 25600, True, "dma_atomic"), (1, 64, 26688, True, "dma_atomic"), (5, 192, 25472, False, "dma_atomic"),
+    (264, 128, 19968, False, "dma_atomic"),
+    # ... but not where the adds or the long way of B cost more than they gain, or K is short
+    (16, 8192, 8192, True, "ragged"), (128, 8192, 8192, False, "ragged"), (128, 8192, 8192, True, "ragged"),
+    (16, 1024, 1024, False, "ragged"), (256, 512, 2048, True, "ragged")])
+def test_bare_int8_product_is_compared_with_the_split_it_would_run(m, n, k, trans_b, kernel):
+    """Measured, split against register-staged: 5 x 192 x 25472 16.4 / 79.9 us, 16 x 8192 x 8192 30.1 / 36.7 and with B
+    as [N, K] 30.7 / 23.6, 128 x 8192 x 8192 71.0 / 39.3 and 74.6 / 26.0."""
+    assert kernel_of(m, n, k, trans_b=trans_b) == kernel
+
+
+@pytest.mark.parametrize("m,n,k,trans_b,kernel", [
+    (16, 8192, 8192, False, "dma_shares"), (128, 8192, 8192, False, "dma_shares"), (16, 2048, 8192, True, "dma_shares"),
+    (128, 14336, 4096, False, "dma_shares"), (128, 8192, 8192, True, "ragged"), (512, 2048, 8192, True, "ragged"),
+    (512, 4096, 4096, False, "ragged"), (512, 4096, 4096, True, "ragged")])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("out", [None, "bf16"])
+def test_a_workspace_is_used_where_the_shares_are_faster(m, n, k, trans_b, kernel, fp8, out):
+    """Measured, shares against register-staged: 128 x 8192 x 8192 fp8 34.5 / 39.3 us, with B as [N, K] 34.5 / 25.3;
+    512 x 4096 x 4096 33.5 / 28.0."""
+    assert kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, out=out, workspace=64 << 20) == kernel
+    # one that is too small is none
+    assert kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, out=out, workspace=1 << 10) in ("ragged", "dma_atomic")
+
+
+def test_large_and_small_grids():
+    for fp8 in (False, True):
+        for out in (None, "bf16", "f32"):
+            assert kernel_of(8192, 8192, 8192, fp8=fp8, out=out) == "dma"
+            assert kernel_of(4096, 4096, 4096, fp8=fp8, out=out) == "dma"
+            assert kernel_of(1024, 1024, 1024, fp8=fp8, out=out) == "ragged"
+            assert kernel_of(4096, 4096, 4112, fp8=fp8, out=out) == "mfma"
+            assert kernel_of(197, 64, 208, batch=96, fp8=fp8, out=out) == "ragged"
+    # a vector of column scales per batch entry: only the direct-to-LDS kernels have it
+    assert kernel_of(128, 768, 768, batch=3, out="f32", scale_b_mode=capi.QP.PER_COL_BATCH) == "dma"
