@@ -1,6 +1,6 @@
 // mi355_quant_dot: argument checking, kernel selection, and the any-stride
 // kernel that serves what no matrix-core kernel takes (transposed A, uint8,
-// unaligned e5m2, K below 16 and the like).
+// unaligned e5m2, K below 16 and the like) and short unaligned K.
 #include "common.h"
 #include <atomic>
 #include <mutex>
@@ -313,6 +313,25 @@ bool ragged_is_faster(const mi355_quant_dot_desc* d, double other_us, double lef
            !(d->dequant && d->scale_b_mode == MI355_QP_PER_COL_BATCH) && ragged_us(d) < (1.0 - left) * other_us;
 }
 
+// Matrices aligned to nothing: the any-stride kernel, whose blocks of 16 x 16 outputs start at once, against
+// the register-staged one, whose first barrier stands behind a slab that a short K hardly fills (fitted
+// to 500 products of K below 128; the results are the same bits).  44 x 87 x 16 fp8 with the epilogue 5.7
+// against 3.5 us, 74 x 7 x 31 int8 6.0 against 4.0; from K = 80 on the register-staged kernel is the faster
+// one at any size.
+bool short_k_is_faster(const mi355_quant_dot_desc* d)
+{
+    if(d->k >= 128 || (d->m + 15) / 16 > 65535)
+        return false;
+    const bool fp8   = d->in_type == MI355_FP8;
+    const double k   = (double)d->k;
+    const double out = (double)d->batch * (double)d->m * (double)d->n * 1e-6;
+    const double any = 3.0 + 0.036 * k + tiles_of(d, 16) / 2048.0 * (1.8 + 0.06 * k);
+    const double staged =
+        fp8 ? (d->dequant ? 5.7 : 5.0) + 0.0015 * k + tiles_of(d, 64) / 256.0 * (0.7 + 0.013 * k) + 1.4 * out
+            : (d->dequant ? 5.3 : 4.25) + 0.0007 * k + 1.9 * out;
+    return any < staged;
+}
+
 __global__ void zero_i32_kernel(int32_t* p, int64_t n)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -465,7 +484,7 @@ int choose_kernel(const mi355_quant_dot_desc* d,
         return MI355_OK;
     }
     // rows aligned to nothing; fp8 sums stay exact there, as in the generic kernel
-    if(mi355_ragged_gemm_supported(d))
+    if(mi355_ragged_gemm_supported(d) && !short_k_is_faster(d))
     {
         *kernel = kernel_id::ragged_exact;
         return MI355_OK;

@@ -7,6 +7,7 @@ import torch
 
 from oracle import oracle as orc
 from tests.gpu_util import bf16_bits, dev, half_bits
+from tests.quant_dot_kernel import kernel_of
 
 pytestmark = pytest.mark.gpu
 
@@ -108,3 +109,22 @@ def test_fp8_largest_digit_sums(ops):
     b[:, 1] = 0x01
     got = ops.quant_dot(dev(a), dev(b), fp8=True).cpu().numpy()
     assert np.array_equal(got, orc.quant_dot(a, b, orc.FP8).reshape(3, 5))
+
+
+# the smallest M, N and K of the kernel, and slabs filled in part: short K reaches it in batches (alone it is
+# left to the any-stride kernel)
+@pytest.mark.parametrize("batch,m,n,k", [(1, 1, 5, 131), (1, 3, 4, 129), (500, 64, 67, 16), (500, 33, 35, 17),
+                                         (500, 65, 66, 33), (300, 130, 65, 61)])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_short_k_in_batches(ops, batch, m, n, k, trans_b, fp8):
+    rng = np.random.default_rng(batch + n)
+    assert kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, batch=batch) == "ragged_exact"
+    if fp8:
+        a, b = _fp8(rng, (batch, m, k), False), _fp8(rng, (batch, k, n), False)
+    else:
+        a, b = (rng.integers(-128, 128, s, dtype=np.int8) for s in ((batch, m, k), (batch, k, n)))
+    db = dev(np.ascontiguousarray(b.transpose(0, 2, 1))).transpose(1, 2) if trans_b else dev(b)
+    print("short", batch, m, n, k, trans_b, fp8, flush=True)
+    got = ops.quant_dot(dev(a), db, fp8=fp8).cpu().numpy()
+    assert np.array_equal(got, orc.quant_dot(a, b, orc.FP8 if fp8 else orc.I8))

@@ -68,3 +68,14 @@ def test_large_and_small_grids():
             assert kernel_of(197, 64, 208, batch=96, fp8=fp8, out=out) == "ragged"
     # a vector of column scales per batch entry: only the direct-to-LDS kernels have it
     assert kernel_of(128, 768, 768, batch=3, out="f32", scale_b_mode=capi.QP.PER_COL_BATCH) == "dma"
+
+
+@pytest.mark.parametrize("m,n,k,batch,kernel", [
+    (44, 87, 17, 1, "generic"), (356, 45, 17, 1, "generic"), (1, 5, 16, 1, "generic"), (74, 7, 31, 1, "generic"),
+    # many outputs, or more of K than a few blocks are done with at once
+    (2049, 2051, 17, 1, "ragged_exact"), (33, 35, 17, 500, "ragged_exact"), (65, 63, 93, 1, "ragged_exact"),
+    (500, 30522, 768, 1, "ragged_exact"), (197, 197, 61, 96, "ragged_exact")])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("out", [None, "bf16"])
+def test_short_unaligned_k(m, n, k, batch, kernel, fp8, out):
+    assert kernel_of(m, n, k, batch=batch, fp8=fp8, out=out) == kernel
