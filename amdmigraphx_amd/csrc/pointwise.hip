@@ -105,10 +105,10 @@ __global__ __launch_bounds__(PW_THREADS) void quantizelinear_kernel(
             o[e] = res[e];
 }
 
-// ---- runs of 16 elements -------------------------------------------------------------------------
-// What bounds both operators is memory: the kernels below move 16 consecutive elements of one row
-// per thread, 16 bytes a load or store, at whatever address the row has (a global load of 16 bytes
-// takes any).  Everything an element used to pay for by itself is gone:
+// ---- runs of elements ----------------------------------------------------------------------------
+// What bounds both operators is memory: the kernels below move 16 or 4 consecutive elements of one row
+// per thread, up to 16 bytes a load or store, at whatever address the row has (a global load takes
+// any).  Everything an element used to pay for by itself is gone:
 // the 64-bit division that finds its row (a multiplication by the reciprocal here, once per run), the
 // loads of scale and zero point (once per run where they don't vary along the row, else as a vector),
 // and arithmetic in double where float provably gives the same bits:
@@ -117,14 +117,15 @@ __global__ __launch_bounds__(PW_THREADS) void quantizelinear_kernel(
 //   rint + zp   whole numbers below 2^24, or saturated;
 //   (x - zp) s  the difference of two 8-bit values, fp8 e4m3fn's 2^-9 ... 896 included, is exact in
 //               float, so is the double product: one rounding to float either way.
+// The last run of a row ends where the row ends: it does again what the run before it did of it, and
+// writes the same values (one element at a time, what is left of a row was a chain of up to 15 loads and
+// divisions: [3, 1023] half with a scale per row to int8 3.1 us before the runs, 9.5 with the chain).
 // Left to the kernels of any strides: strides along the row other than 0 and 1, e5m2 (whose zero
 // points cost more than 24 bits), fp8 quantization with a zero point (the sum is rounded as a
-// double there), int32 and float32 inputs of dequantizelinear, 2^31 runs and beyond.
+// double there), int32 and float32 inputs of dequantizelinear, a single element, 2^31 runs and beyond.
 // Measured, [8192, 1024] bfloat16 with a scale per row: to uint8 14.3 -> 7.5 us, back
 // from uint8 with zero points 28 -> 7.0 us; [2048, 8192] bfloat16 to fp8
 // 30 -> 13 us (50 MB).
-
-constexpr int RUN = 16;
 
 struct run_params
 {
@@ -132,20 +133,21 @@ struct run_params
     void* out;
     qparams q;
     int64_t cols;
+    int run;           // elements
     uint32_t runs;     // in all
-    uint32_t per_row;  // runs of a row, the last of which may be short
+    uint32_t per_row;  // runs of a row, the last of which may overlap the one before it
     uint32_t magic;    // run / per_row = (run * magic) >> shift for run < 2^31
     uint32_t shift;
 };
 
 // consecutive elements at any address
-template <class T, int N = RUN>
+template <class T, int N>
 struct __attribute__((packed, aligned(1))) run_of
 {
     T v[N];
 };
 
-template <int N = RUN, class T>
+template <int N, class T>
 MI355_DEVINL run_of<T, N> load_run(const T* p)
 {
     return *reinterpret_cast<const run_of<T, N>*>(p);
@@ -327,51 +329,53 @@ MI355_DEVINL void dequantize_elements(const run_params& p, int64_t r, int64_t c)
 }
 
 // QUANTIZE: IN a float type, OUT a code's; else the other way
-template <bool QUANTIZE, int IN, int OUT>
+template <bool QUANTIZE, int IN, int OUT, int N>
 __global__ __launch_bounds__(PW_THREADS) void run_kernel(run_params p)
 {
     const uint32_t run = blockIdx.x * PW_THREADS + threadIdx.x;
     if(run >= p.runs)
         return;
     const uint32_t r = (uint32_t)(((uint64_t)run * p.magic) >> p.shift);
-    int64_t c        = (int64_t)(run - r * p.per_row) * RUN;
-    if(p.cols - c >= RUN)
-    {
-        if constexpr(QUANTIZE)
-            quantize_elements<IN, OUT, RUN>(p, r, c);
-        else
-            dequantize_elements<IN, OUT, RUN>(p, r, c);
-    }
+    const int64_t c  = min((int64_t)(run - r * p.per_row) * N, p.cols - N);
+    if constexpr(QUANTIZE)
+        quantize_elements<IN, OUT, N>(p, r, c);
     else
-        for(; c < p.cols; c++) // the end of a row
-        {
-            if constexpr(QUANTIZE)
-                quantize_elements<IN, OUT, 1>(p, r, c);
-            else
-                dequantize_elements<IN, OUT, 1>(p, r, c);
-        }
+        dequantize_elements<IN, OUT, N>(p, r, c);
 }
 
 // Strides along the row of 0 and 1 only; rows that are one vector for the parameters as well become
-// one long row.  False where the kernels of any strides have to take the call.
-bool run_plan(run_params& p, const void* x, const qparams& q, void* out, int64_t rows, int64_t cols)
+// one long row.  `wide`: runs of 16 may pay.  False where the kernels of any strides have to take the call.
+bool run_plan(run_params& p, const void* x, const qparams& q, void* out, int64_t rows, int64_t cols, bool wide)
 {
     const bool has_zp = q.zp != nullptr;
-    if(q.s_sc < 0 || q.s_sc > 1 || (has_zp && (q.z_sc < 0 || q.z_sc > 1)))
+    p.x   = x;
+    p.out = out;
+    p.q   = q;
+    if(cols == 1) // rows of one element: the stride along the rows is the one along a single row
+    {
+        p.q.s_sc = q.s_sr;
+        p.q.z_sc = q.z_sr;
+    }
+    if(p.q.s_sc < 0 || p.q.s_sc > 1 || (has_zp && (p.q.z_sc < 0 || p.q.z_sc > 1)))
         return false;
     // element i of the tensor has parameter i (a full tensor of them), or the one there is
     auto flat = [&](int64_t sr, int64_t sc) { return sr == sc * cols; };
-    if(flat(q.s_sr, q.s_sc) && (!has_zp || flat(q.z_sr, q.z_sc)))
+    if(flat(p.q.s_sr, p.q.s_sc) && (!has_zp || flat(p.q.z_sr, p.q.z_sc)))
     {
         cols *= rows;
         rows = 1;
     }
-    const int64_t per_row = (cols + RUN - 1) / RUN;
+    if(cols < 2)
+        return false;
+    // 16 elements a thread pay for their latency where there are many and one parameter serves them all, 4
+    // otherwise.  Over 2500 tensors, 4 against 16: below 2^21 elements 0.8 to 0.95 of the time, above
+    // 1.0 to 1.25; with parameters of their own 0.75 to 1.0 at any size; to float32 (64 bytes a
+    // thread side by side) 0.6 to 0.8.
+    const bool one = p.q.s_sc == 0 && (!has_zp || p.q.z_sc == 0);
+    p.run          = wide && one && cols >= 16 && rows * cols >= 1 << 21 ? 16 : cols >= 4 ? 4 : 2;
+    const int64_t per_row = (cols + p.run - 1) / p.run;
     if(per_row > 0x7fffffff || rows > 0x7fffffff / per_row)
         return false;
-    p.x       = x;
-    p.out     = out;
-    p.q       = q;
     p.cols    = cols;
     p.per_row = (uint32_t)per_row;
     p.runs    = (uint32_t)(rows * per_row);
@@ -382,6 +386,23 @@ bool run_plan(run_params& p, const void* x, const qparams& q, void* out, int64_t
     p.shift = 31 + l;
     p.magic = (uint32_t)((((uint64_t)1 << p.shift) + p.per_row - 1) / p.per_row);
     return true;
+}
+
+template <bool QUANTIZE, int IN, int OUT>
+int launch_runs(const run_params& p, hipStream_t s)
+{
+    const dim3 grid((p.runs + PW_THREADS - 1) / PW_THREADS), block(PW_THREADS);
+    if constexpr(QUANTIZE || OUT != MI355_F32)
+        if(p.run == 16)
+        {
+            hipLaunchKernelGGL((run_kernel<QUANTIZE, IN, OUT, 16>), grid, block, 0, s, p);
+            return mi355_launch_status();
+        }
+    if(p.run == 4)
+        hipLaunchKernelGGL((run_kernel<QUANTIZE, IN, OUT, 4>), grid, block, 0, s, p);
+    else
+        hipLaunchKernelGGL((run_kernel<QUANTIZE, IN, OUT, 2>), grid, block, 0, s, p);
+    return mi355_launch_status();
 }
 
 __global__ __launch_bounds__(PW_THREADS) void dequantizelinear_kernel(const void* x,
@@ -605,16 +626,13 @@ int launch_quantize(int out_type,
 {
     run_params p;
     if((out_type == MI355_I8 || out_type == MI355_U8 || (out_type == MI355_FP8 && q.zp == nullptr)) &&
-       run_plan(p, x, q, out, rows, cols))
+       run_plan(p, x, q, out, rows, cols, true))
     {
-        const dim3 grid(blocks_for(p.runs));
         if(out_type == MI355_I8)
-            hipLaunchKernelGGL((run_kernel<true, XT, MI355_I8>), grid, dim3(PW_THREADS), 0, s, p);
-        else if(out_type == MI355_U8)
-            hipLaunchKernelGGL((run_kernel<true, XT, MI355_U8>), grid, dim3(PW_THREADS), 0, s, p);
-        else
-            hipLaunchKernelGGL((run_kernel<true, XT, MI355_FP8>), grid, dim3(PW_THREADS), 0, s, p);
-        return mi355_launch_status();
+            return launch_runs<true, XT, MI355_I8>(p, s);
+        if(out_type == MI355_U8)
+            return launch_runs<true, XT, MI355_U8>(p, s);
+        return launch_runs<true, XT, MI355_FP8>(p, s);
     }
     const int64_t work = rows * ((cols + 3) / 4);
     switch(out_type)
@@ -641,15 +659,13 @@ int launch_quantize(int out_type,
 }
 
 template <int XT>
-void launch_dequantize_runs(int s_type, const run_params& p, hipStream_t s)
+int launch_dequantize_runs(int s_type, const run_params& p, hipStream_t s)
 {
-    const dim3 grid(blocks_for(p.runs));
     if(s_type == MI355_F32)
-        hipLaunchKernelGGL((run_kernel<false, XT, MI355_F32>), grid, dim3(PW_THREADS), 0, s, p);
-    else if(s_type == MI355_F16)
-        hipLaunchKernelGGL((run_kernel<false, XT, MI355_F16>), grid, dim3(PW_THREADS), 0, s, p);
-    else
-        hipLaunchKernelGGL((run_kernel<false, XT, MI355_BF16>), grid, dim3(PW_THREADS), 0, s, p);
+        return launch_runs<false, XT, MI355_F32>(p, s);
+    if(s_type == MI355_F16)
+        return launch_runs<false, XT, MI355_F16>(p, s);
+    return launch_runs<false, XT, MI355_BF16>(p, s);
 }
 
 } // namespace
@@ -710,16 +726,14 @@ extern "C" int mi355_dequantizelinear(const void* x,
         return MI355_OK;
     qparams q{scale, scale_stride_r, scale_stride_c, zp, zp_stride_r, zp_stride_c};
     run_params p;
-    if((x_type == MI355_I8 || x_type == MI355_U8 || x_type == MI355_FP8) && run_plan(p, x, q, out, rows, cols))
+    if((x_type == MI355_I8 || x_type == MI355_U8 || x_type == MI355_FP8) && run_plan(p, x, q, out, rows, cols, scale_type != MI355_F32))
     {
         hipStream_t s = static_cast<hipStream_t>(stream);
         if(x_type == MI355_I8)
-            launch_dequantize_runs<MI355_I8>(scale_type, p, s);
-        else if(x_type == MI355_U8)
-            launch_dequantize_runs<MI355_U8>(scale_type, p, s);
-        else
-            launch_dequantize_runs<MI355_FP8>(scale_type, p, s);
-        return mi355_launch_status();
+            return launch_dequantize_runs<MI355_I8>(scale_type, p, s);
+        if(x_type == MI355_U8)
+            return launch_dequantize_runs<MI355_U8>(scale_type, p, s);
+        return launch_dequantize_runs<MI355_FP8>(scale_type, p, s);
     }
     hipLaunchKernelGGL(dequantizelinear_kernel, dim3(blocks_for(rows * cols)), dim3(PW_THREADS), 0,
                        static_cast<hipStream_t>(stream), x, x_type, q, scale_type, out, rows, cols);

@@ -1,5 +1,5 @@
-"""the kernels that quantize, dequantize (16 elements a thread), pack and unpack (8 bytes), at the lengths
-and addresses where a run is short or misaligned, against the CPU oracle: all bit for bit."""
+"""the kernels that quantize, dequantize (16, 4 or 2 elements a thread), pack and unpack (8 bytes), at the
+lengths and addresses where runs overlap or are misaligned, against the CPU oracle: all bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -45,10 +45,23 @@ def _param(rng, place, rows, cols, make):
 
 
 @pytest.mark.parametrize("rows,cols,shift", [(1, 1, 0), (3, 7, 1), (5, 8, 0), (2, 9, 3), (37, 101, 1), (300, 15, 5),
-                                             (5, 16, 2), (2, 33, 0), (17, 4096, 0), (1, 70001, 1)])
+                                             (5, 16, 2), (2, 33, 0), (17, 4096, 0), (1, 70001, 1), (50, 1, 1), (40, 2, 0), (33, 3, 1),
+                                             (20, 4, 2), (21, 5, 0), (9, 17, 1), (700, 31, 0)])
 @pytest.mark.parametrize("place", ["tensor", "row", "col", "full"])
 @pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
 def test_runs_there_and_back(ops, kind, place, rows, cols, shift):
+    _there_and_back(ops, kind, place, rows, cols, shift)
+
+
+# 2^21 elements and more with one parameter for a row: 16 elements a thread
+@pytest.mark.parametrize("place,rows,cols,shift", [("tensor", 1, 2097157, 3), ("tensor", 3, 699053, 0), ("row", 131, 16111, 1),
+                                                   ("row", 116509, 18, 0), ("row", 131073, 16, 1)])
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+def test_long_runs_there_and_back(ops, kind, place, rows, cols, shift):
+    _there_and_back(ops, kind, place, rows, cols, shift)
+
+
+def _there_and_back(ops, kind, place, rows, cols, shift):
     rng = np.random.default_rng(rows * cols + shift)
     x = rng.standard_normal((rows, cols)) * rng.choice([0.01, 1.0, 30.0], (rows, cols))
     odd = np.array([0.0, -0.0, 0.5, -2.5, 1e9, -1e9, np.inf, -np.inf, np.nan, 1e-30, -1e-30])
