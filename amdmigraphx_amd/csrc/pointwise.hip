@@ -532,13 +532,12 @@ __global__ __launch_bounds__(PW_THREADS) void pack_fp4_kernel(const float* in, u
 }
 
 // two bytes -> one packed byte: 16 bytes per thread, one load and one 8-byte store at any address
-// ([8192, 1024] bytes: 7.9 -> 3.4 us)
+// ([8192, 1024] bytes: 7.9 -> 3.4 us).  The last thread's 8 end where the tensor ends and are in part
+// the ones before them again, with the same values; less than 8 are one a thread.
 __global__ __launch_bounds__(PW_THREADS) void pack_int4_kernel(
     const uint8_t* in, uint8_t* out, int is_signed, int64_t total_out)
 {
-    const int64_t i0 = ((int64_t)blockIdx.x * PW_THREADS + threadIdx.x) * 8;
-    if(i0 >= total_out)
-        return;
+    const int64_t i = (int64_t)blockIdx.x * PW_THREADS + threadIdx.x;
     auto packed = [&](uint32_t two) {
         int u1 = (int)(two & 0xff), u2 = (int)(two >> 8);
         if(is_signed)
@@ -553,18 +552,21 @@ __global__ __launch_bounds__(PW_THREADS) void pack_int4_kernel(
         }
         return (uint8_t)((u2 << 4) | (u1 & 0xf));
     };
-    if(total_out - i0 >= 8)
+    if(total_out < 8)
     {
-        const auto v = load_run<8>(reinterpret_cast<const uint16_t*>(in) + i0);
-        run_of<uint8_t, 8> res;
-#pragma unroll
-        for(int e = 0; e < 8; e++)
-            res.v[e] = packed(v.v[e]);
-        store_run(out + i0, res);
-    }
-    else
-        for(int64_t i = i0; i < total_out; i++)
+        if(i < total_out)
             out[i] = packed(in[2 * i] | ((uint32_t)in[2 * i + 1] << 8));
+        return;
+    }
+    if(8 * i >= total_out)
+        return;
+    const int64_t i0 = min(8 * i, total_out - 8);
+    const auto v     = load_run<8>(reinterpret_cast<const uint16_t*>(in) + i0);
+    run_of<uint8_t, 8> res;
+#pragma unroll
+    for(int e = 0; e < 8; e++)
+        res.v[e] = packed(v.v[e]);
+    store_run(out + i0, res);
 }
 
 __global__ __launch_bounds__(PW_THREADS) void convert_kernel(

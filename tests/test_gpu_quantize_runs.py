@@ -90,7 +90,7 @@ def _there_and_back(ops, kind, place, rows, cols, shift):
             assert np.array_equal(back, np.ascontiguousarray(want).view(raw)), (code, z is None)
 
 
-@pytest.mark.parametrize("count,shift", [(1, 0), (7, 1), (8, 0), (9, 3), (4099, 1)])
+@pytest.mark.parametrize("count,shift", [(1, 0), (7, 1), (8, 0), (9, 3), (15, 1), (2047, 0), (4099, 1)])
 @pytest.mark.parametrize("dtype", [np.uint8, np.int8])
 def test_int4_runs(ops, dtype, count, shift):
     rng = np.random.default_rng(count)
