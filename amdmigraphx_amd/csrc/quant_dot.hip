@@ -388,6 +388,20 @@ enum class kernel_id : int
     dma_atomic   = 7  // K in shares added into C
 };
 
+bool dma_takes(const mi355_quant_dot_desc* d, const void* a, const void* b, const float* bias)
+{
+    // int8 with N % 4 != 0 would take the DMA path's 32 x 32 kernel, which applies no bias
+    const bool fp8 = d->in_type == MI355_FP8;
+    return (fp8 || d->in_type == MI355_I8) && d->k > 0 && (bias == nullptr || fp8 || d->n % 4 == 0) &&
+           mi355_dma_gemm_supported(d, a, b);
+}
+
+bool mfma_takes(const mi355_quant_dot_desc* d, const void* a, const void* b, const void* c)
+{
+    return d->in_type != MI355_U8 && d->k > 0 && !(d->dequant && d->scale_b_mode == MI355_QP_PER_COL_BATCH) &&
+           mi355_mfma_gemm_supported(d, a, b, c);
+}
+
 // argument checks and the choice of the kernel; the pointers are looked at, not through
 int choose_kernel(const mi355_quant_dot_desc* d,
                   const void* a,
@@ -462,23 +476,21 @@ int choose_kernel(const mi355_quant_dot_desc* d,
     if(d->batch > 65535)
         return MI355_ERR_UNSUPPORTED;
 
-    // int8 with N % 4 != 0 would take the DMA path's 32 x 32 kernel, which applies no bias
-    const bool dma_has_bias = bias == nullptr || fp8 || d->n % 4 == 0;
-    if(!u8 && !bf8 && d->k > 0 && dma_has_bias && mi355_dma_gemm_supported(d, a, b))
+    if(dma_takes(d, a, b, bias))
     {
         // fp8: the sums of both are float
         bool atomic      = false;
         const int shares = mi355_dma_gemm_shares(d, c, workspace, workspace_bytes, &atomic);
-        *kernel          = ragged_is_faster(d, dma_us(d, shares, atomic), shares > 1 ? 0.1 : 0.07) ? kernel_id::ragged
-                           : shares == 1                                  ? kernel_id::dma
-                           : atomic                                       ? kernel_id::dma_atomic
-                                                                          : kernel_id::dma_shares;
+        if(ragged_is_faster(d, dma_us(d, shares, atomic), shares > 1 ? 0.1 : 0.07))
+            *kernel = kernel_id::ragged;
+        else
+            *kernel = shares == 1 ? kernel_id::dma : atomic ? kernel_id::dma_atomic : kernel_id::dma_shares;
         return MI355_OK;
     }
     // a vector of column scales per batch entry exists in the kernels above only
     if(d->dequant && d->scale_b_mode == MI355_QP_PER_COL_BATCH)
         return MI355_ERR_UNSUPPORTED;
-    if(!u8 && d->k > 0 && mi355_mfma_gemm_supported(d, a, b, c))
+    if(mfma_takes(d, a, b, c))
     {
         *kernel = !bf8 && ragged_is_faster(d, mfma_us(d), 0.07) ? kernel_id::ragged : kernel_id::mfma;
         return MI355_OK;
@@ -495,45 +507,22 @@ int choose_kernel(const mi355_quant_dot_desc* d,
 
 } // namespace
 
-// The kernel_id of a call, or its (negative) status.  Not part of the public interface: tests ask it,
-// without a GPU, which kernel their shapes reach.
-extern "C" int mi355_internal_quant_dot_kernel(const mi355_quant_dot_desc* d,
-                                               const void* a,
-                                               const void* b,
-                                               const void* c,
-                                               const float* scale_a,
-                                               const float* scale_b,
-                                               const int32_t* colsum_b,
-                                               const int32_t* rowsum_a,
-                                               const float* bias,
-                                               const void* workspace,
-                                               size_t workspace_bytes)
-{
-    kernel_id kernel = kernel_id::none;
-    const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
-                                     workspace_bytes, &kernel);
-    return status == MI355_OK ? (int)kernel : status;
-}
+namespace {
 
-extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
-                                  const void* a,
-                                  const void* b,
-                                  void* c,
-                                  const float* scale_a,
-                                  const float* scale_b,
-                                  const int32_t* colsum_b,
-                                  const int32_t* rowsum_a,
-                                  const float* bias,
-                                  void* workspace,
-                                  size_t workspace_bytes,
-                                  void* stream)
+int launch_kernel(kernel_id kernel,
+                  const mi355_quant_dot_desc* d,
+                  const void* a,
+                  const void* b,
+                  void* c,
+                  const float* scale_a,
+                  const float* scale_b,
+                  const int32_t* colsum_b,
+                  const int32_t* rowsum_a,
+                  const float* bias,
+                  void* workspace,
+                  size_t workspace_bytes,
+                  hipStream_t s)
 {
-    kernel_id kernel = kernel_id::none;
-    const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
-                                     workspace_bytes, &kernel);
-    if(status != MI355_OK)
-        return status;
-    hipStream_t s = static_cast<hipStream_t>(stream);
     switch(kernel)
     {
     case kernel_id::none: return MI355_OK;
@@ -583,6 +572,86 @@ extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
     dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)d->batch);
     hipLaunchKernelGGL(quant_dot_generic_kernel, grid, dim3(256), 0, s, p);
     return mi355_launch_status();
+}
+
+} // namespace
+
+extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
+                                  const void* a,
+                                  const void* b,
+                                  void* c,
+                                  const float* scale_a,
+                                  const float* scale_b,
+                                  const int32_t* colsum_b,
+                                  const int32_t* rowsum_a,
+                                  const float* bias,
+                                  void* workspace,
+                                  size_t workspace_bytes,
+                                  void* stream)
+{
+    kernel_id kernel = kernel_id::none;
+    const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
+                                     workspace_bytes, &kernel);
+    return status != MI355_OK ? status
+                              : launch_kernel(kernel, d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
+                                              workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+// The two below are not part of the public interface.  Tests ask the first, without a GPU, which kernel their
+// shapes reach (the kernel_id, or the call's negative status), and with the second run the edges of
+// a kernel at sizes that the rules leave to another (the product, or MI355_ERR_UNSUPPORTED where the
+// kernel does not take it).
+extern "C" int mi355_internal_quant_dot_kernel(const mi355_quant_dot_desc* d,
+                                               const void* a,
+                                               const void* b,
+                                               const void* c,
+                                               const float* scale_a,
+                                               const float* scale_b,
+                                               const int32_t* colsum_b,
+                                               const int32_t* rowsum_a,
+                                               const float* bias,
+                                               const void* workspace,
+                                               size_t workspace_bytes)
+{
+    kernel_id kernel = kernel_id::none;
+    const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
+                                     workspace_bytes, &kernel);
+    return status == MI355_OK ? (int)kernel : status;
+}
+
+extern "C" int mi355_internal_quant_dot_run(int32_t which,
+                                            const mi355_quant_dot_desc* d,
+                                            const void* a,
+                                            const void* b,
+                                            void* c,
+                                            const float* scale_a,
+                                            const float* scale_b,
+                                            const int32_t* colsum_b,
+                                            const int32_t* rowsum_a,
+                                            const float* bias,
+                                            void* workspace,
+                                            size_t workspace_bytes,
+                                            void* stream)
+{
+    kernel_id kernel = kernel_id::none;
+    const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
+                                     workspace_bytes, &kernel);
+    if(status != MI355_OK || kernel == kernel_id::none)
+        return status;
+    bool takes = false;
+    switch(static_cast<kernel_id>(which))
+    {
+    case kernel_id::dma: takes = dma_takes(d, a, b, bias); break;
+    case kernel_id::mfma: takes = mfma_takes(d, a, b, c); break;
+    case kernel_id::ragged:
+    case kernel_id::ragged_exact:
+        takes = mi355_ragged_gemm_supported(d) && !(d->dequant && d->scale_b_mode == MI355_QP_PER_COL_BATCH);
+        break;
+    default: break;
+    }
+    return !takes ? MI355_ERR_UNSUPPORTED
+                  : launch_kernel(static_cast<kernel_id>(which), d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias,
+                                  workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 // ---- quant_dot that allocates nothing and takes no workspace -------------------------------

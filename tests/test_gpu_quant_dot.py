@@ -62,8 +62,9 @@ def test_int8_accumulators_bit_exact(ops, m, n, k, trans_b):
     assert np.array_equal(got, want)
 
 
-# few output tiles and a long K: the split-K form of the kernel (shares of K added into C with
-# integer atomics) must still be bit-exact, for any split remainder and for rows past M
+# few output tiles and a long K: whichever kernel takes it, the product must be bit-exact, for any split
+# remainder and for rows past M (the split-K form, shares of K added into C with integer atomics, runs at all
+# these sizes in test_gpu_quant_dot_large_tiles.py)
 SKINNY = [(16, 8192, 8192), (128, 2048, 4096), (1, 256, 2048), (37, 512, 1088), (300, 260, 1024),
           (1024, 1024, 1024), (16, 768, 576)]
 
@@ -150,8 +151,8 @@ def test_int8_dequant_epilogue_bit_exact(ops, zp_a, zp_b, out):
 
 
 # ---- the four-wave kernel: one-pass int8 products with K >= 3072 --------------------------------
-# Bare products reach it when the tiles alone fill half the chip (here through the batch), products
-# with the dequantizing epilogue whenever no workspace is given.
+# The products below are those of its edges.  quant_dot itself leaves those of few 256 x 256 tiles, and [K, N]
+# with N % 16 != 0, to other kernels; test_gpu_quant_dot_large_tiles.py runs them with the kernel named.
 
 @pytest.mark.parametrize("m,n,k,batch,trans_b", [
     (300, 520, 3136, 32, False),      # ragged M and N tiles, an odd number of slabs (49)
@@ -178,8 +179,8 @@ def test_four_wave_kernel_bare_bit_exact(ops, m, n, k, batch, trans_b):
 # a K that is not a multiple of 128 (the last A step is half a step).
 @pytest.mark.parametrize("k", [3392, 3456, 3776, 3840, 4160, 7744])
 @pytest.mark.parametrize("trans_b", [False, True])
-def test_four_wave_kernels_trip_boundaries_bit_exact(ops, k, trans_b):
-    m, n, batch = 300, 520, 22   # 132 tiles: at least half the chip, so no K split (see above)
+def test_four_wave_kernels_trip_boundaries_bit_exact(ops, k, trans_b, n=520):
+    m, batch = 300, 22   # 132 tiles: at least half the chip, so no K split (see above)
     rng = np.random.default_rng(k + trans_b)
     a = rng.integers(-128, 128, (batch, m, k), dtype=np.int8)
     b = rng.integers(-128, 128, (batch, k, n), dtype=np.int8)
@@ -230,11 +231,11 @@ def test_four_wave_kernel_dequantizing_epilogue_bit_exact(ops, m, n, k, trans_b,
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-def test_four_wave_kernel_unaligned_column_arrays(ops, fp8):
+def test_four_wave_kernel_unaligned_column_arrays(ops, fp8, n=264):
     """Per-column scales, column sums and biases normally come four at a time; arrays that start
     off a 16-byte boundary are read one value at a time.  Both must give the same bits."""
     rng = np.random.default_rng(123 + fp8)
-    m, n, k = 260, 264, 3072
+    m, k = 260, 3072
     if fp8:
         a = orc.fp8_from_f32(rng.integers(-8, 9, (m, k)).astype(np.float32))
         b = orc.fp8_from_f32(rng.integers(-8, 9, (k, n)).astype(np.float32))
@@ -266,14 +267,14 @@ def test_four_wave_kernel_unaligned_column_arrays(ops, fp8):
 @pytest.mark.parametrize("k", [1024, 3072])
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("out", ["bare", "f32", "bf16"])
-def test_results_through_the_lds_copy_into_strided_batched_views(ops, k, fp8, out):
+def test_results_through_the_lds_copy_into_strided_batched_views(ops, k, fp8, out, n=264):
     """The kernels write C from a row-major copy in the LDS, whole rows of a wave's part per store.
     C here is a view with a row pitch beyond N and a batch stride beyond M x pitch, ragged in M and
     N: every element inside must carry the oracle's bits (operands are small integers, so fp8 sums
     are exact too) and everything around the view must stay untouched.  K = 1024 runs on the
     eight-wave kernels, K = 3072 on the four-wave ones."""
     rng = np.random.default_rng(k + 7 * fp8 + len(out))
-    bt, m, n, pitch, rows = 2, 300, 264, 280, 310
+    bt, m, pitch, rows = 2, 300, 280, 310
     if fp8:
         a = orc.fp8_from_f32(rng.integers(-8, 9, (bt, m, k)).astype(np.float32))
         b = orc.fp8_from_f32(rng.integers(-8, 9, (bt, k, n)).astype(np.float32))
@@ -308,9 +309,9 @@ def test_results_through_the_lds_copy_into_strided_batched_views(ops, k, fp8, ou
     assert bool((outside == 7).all())
 
 
-def test_four_wave_kernel_per_row_scales(ops):
+def test_four_wave_kernel_per_row_scales(ops, n=260):
     rng = np.random.default_rng(77)
-    m, n, k = 300, 260, 3072
+    m, k = 300, 3072
     a = rng.integers(-128, 128, (m, k), dtype=np.int8)
     b = rng.integers(-128, 128, (k, n), dtype=np.int8)
     sa = rng.uniform(0.01, 0.05, m).astype(np.float32)

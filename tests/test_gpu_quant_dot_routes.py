@@ -1,9 +1,10 @@
 """quant_dot on both sides of the line between the kernels with 256 x 256 tiles and the register-staged
 one: the shapes that stay with the large tiles, and those beside them that do not, against the same
-product in float64 (exact for int8; the fp8 sums are float)."""
-import numpy as np
+product in float64 (exact for int8; the fp8 sums are float).  Each test says which kernel its calls run."""
 import pytest
 import torch
+
+from tests.quant_dot_kernel import kernel_of
 
 pytestmark = pytest.mark.gpu
 
@@ -50,18 +51,44 @@ def _check(ops, batch, m, n, k, trans_b, fp8, workspace=None):
             assert bool(((t[i].double() - want).abs() <= torch.maximum(want.abs() * 1e-3, most * 2.0**-15)).all())
 
 
+def _kernels(batch, m, n, k, trans_b, fp8):
+    """of the bare product, with scales, and with a workspace as well"""
+    room = dict(out="f32", workspace=1 << 30) if batch == 1 else dict(out="f32")
+    return {kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, batch=batch, **kw) for kw in (dict(), dict(out="f32"), room)}
+
+
 # K on both sides of the four-wave kernels' first length; edges of the 256 tiles
-@pytest.mark.parametrize("batch,m,n,k", [(1, 4100, 4112, 1600), (1, 2050, 8208, 3136), (1, 16, 512, 8192),
-                                         (1, 2050, 8208, 784), (1, 300, 8208, 3136)])
+@pytest.mark.parametrize("batch,m,n,k", [(1, 4100, 4112, 1600), (1, 2050, 8208, 3136), (2, 4100, 2064, 3136)])
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_large_tiles(ops, batch, m, n, k, trans_b, fp8):
+    assert _kernels(batch, m, n, k, trans_b, fp8) == {"dma"}
     _check(ops, batch, m, n, k, trans_b, fp8)
 
 
+# K that is no multiple of 64
+@pytest.mark.parametrize("batch,m,n,k", [(1, 4100, 8240, 2064), (2, 4100, 4112, 2096)])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_large_register_staged_tiles(ops, batch, m, n, k, trans_b, fp8):
+    assert _kernels(batch, m, n, k, trans_b, fp8) == {"mfma"}
+    _check(ops, batch, m, n, k, trans_b, fp8)
+
+
+# few tiles of a long K: in shares where there is room or the product is bare, register-staged without
+@pytest.mark.parametrize("batch,m,n,k", [(1, 16, 512, 8192), (1, 16, 16, 3072), (1, 37, 272, 25600)])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_long_k_of_few_tiles(ops, batch, m, n, k, trans_b, fp8):
+    assert _kernels(batch, m, n, k, trans_b, fp8) == {"ragged" if fp8 else "dma_atomic", "ragged", "dma_shares"}
+    _check(ops, batch, m, n, k, trans_b, fp8)
+
+
+# tiles of 64 x 64, and of 128 x 128 where those fill the chip (2060 x 2064)
 @pytest.mark.parametrize("batch,m,n,k", [(5, 64, 64, 64), (3, 197, 208, 128), (2, 130, 80, 272), (40, 384, 64, 384),
-                                         (1, 1030, 1040, 1024), (1, 16, 16, 3072)])
+                                         (1, 2060, 2064, 784), (1, 1030, 1040, 1024), (1, 300, 2064, 1088)])
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_small_tiles(ops, batch, m, n, k, trans_b, fp8):
+    assert _kernels(batch, m, n, k, trans_b, fp8) == {"ragged"}
     _check(ops, batch, m, n, k, trans_b, fp8)
