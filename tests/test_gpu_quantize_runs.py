@@ -107,3 +107,44 @@ def test_fp8_zeros_and_extremes_keep_their_signs(ops):
         want = orc.quantizelinear(x, np.float32(s), None, orc.F32, orc.FP8)
         got = ops.quantizelinear(_put(x), torch.tensor([s], device="cuda"), None, ops.DT.FP8)
         assert np.array_equal(got.cpu().numpy(), want), s
+
+
+def _near_ties(rng, scale, kind):
+    """values around scale * (whole + 1/2), where the last bit of the quotient decides, and at the bounds of the range
+    in which the quotient is made from the reciprocal"""
+    whole = np.arange(-130, 260)
+    with np.errstate(over="ignore", invalid="ignore"):
+        t = (np.float64(scale) * (whole + 0.5)).astype(np.float32)
+        x = [np.nextafter(t, np.float32(-np.inf)), t, np.nextafter(t, np.float32(np.inf))]
+        x.append((np.float64(scale) * rng.uniform(-500, 500, 300)).astype(np.float32))
+        x.append((np.float64(scale) * 2.0**rng.uniform(-40, 10, 300)).astype(np.float32))
+        x.append(np.float32([2.0**60, np.nextafter(np.float32(2**60), np.float32(0)), -2.0**60, 2.0**-149, -2.0**-126, 0, -0.0]))
+        x = np.concatenate(x)
+    return _bits(np.where(np.isfinite(x), x, np.float32(1)), kind)
+
+
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16"])
+def test_quotients_by_the_reciprocal(ops, kind):
+    """One scale for a tensor: the quotient is the corrected product with the reciprocal for scales of 2^-60 to 2^60 and
+    values up to 2^60, else a division, and has to be the division's in every case."""
+    rng = np.random.default_rng(11)
+    lo, hi = np.float32(2.0**-60), np.float32(2.0**60)
+    scales = [lo, np.nextafter(lo, np.float32(0)), np.nextafter(lo, hi), hi, np.nextafter(hi, lo),
+              np.nextafter(hi, np.float32(np.inf)), 2.0**-140, 2.0**100, 1.0, np.nextafter(np.float32(1), lo),
+              np.nextafter(np.float32(2), lo), -0.37]
+    scales += [m * 2.0**e for m, e in zip(rng.uniform(1, 2, 60), rng.integers(-14, 15, 60))]
+    if kind == "f32":
+        scales += [m * 2.0**e for m, e in zip(rng.uniform(1, 2, 60), rng.integers(-62, 62, 60))]
+    for s in scales:
+        sb = _bits(np.float32([s]), kind)
+        if kind == "f16" and not 6e-8 <= abs(float(orc.half_to_f32(sb)[0])) <= 65504:
+            continue
+        x = _near_ties(rng, np.float32(s), kind).reshape(1, -1)
+        # once in runs of 4, and once in runs of 16 (2^21 elements and more)
+        for repeat in (1, (1 << 21) // x.size + 1) if s in (lo, hi, 1.0, -0.37) else (1,):
+            y = np.ascontiguousarray(np.tile(x, (1, repeat)))
+            dx, ds = _put_float(y, kind), _put_float(sb, kind)
+            for code, (ct, np_code) in _CODES.items():
+                want = orc.quantizelinear(x, sb, None, _FLOATS[kind][0], ct)
+                got = ops.quantizelinear(dx, ds, None, ct).cpu().numpy().view(np_code)
+                assert np.array_equal(got, np.tile(want, (1, repeat))), (float(s), code, repeat)

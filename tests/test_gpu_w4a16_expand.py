@@ -70,3 +70,46 @@ def test_a_workspace_one_byte_short_is_left_alone(ops):
     dense = (dense * scales.float()[:, :, None]).reshape(n, k).abs().double()
     bound = 2 * (x.double().abs() @ dense.t()) * (k * 2.0**-24) + whole.double().abs() * 2.0**-9 + 2.0**-23
     assert bool(((short.double() - whole.double()).abs() <= bound).all())
+
+
+def test_infinities_nan_and_results_beyond_half(ops):
+    """In activations and scales, and sums outside the half range: as the definition has them, and as the call
+    without a workspace, whose kernel dequantizes for itself."""
+    m, n, k, group = 970, 15744, 1664, 128
+    need = ops.w4a16_gemm_workspace_size(m, n, k, group)
+    assert need == 2 * n * k
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.randn(m, k, generator=g, device="cuda").half()
+    w = torch.randint(0, 256, (n, k // 2), generator=g, dtype=torch.uint8, device="cuda")
+    w[:, 0] = 0x88  # the first two weights are zero
+    w[1, 5] = 0x8f
+    scales = (torch.rand(n, k // group, generator=g, device="cuda") * 0.015 + 0.005).half()
+    x[3, 10], x[5, k - 1], x[7, 0], x[8, 11] = float("inf"), float("-inf"), float("inf"), float("nan")
+    x[20:40] *= 3000
+    scales[100, 2], scales[101, 0], scales[102, 3], scales[200, 1] = float("inf"), float("inf"), float("nan"), 65504.0
+    scales[300:310] *= 4000
+    dense = torch.stack([w & 15, w >> 4], dim=2).reshape(n, -1, group).double() - 8
+    dense = (dense * scales.double()[:, :, None]).reshape(n, k)
+    # a weight beyond half's range is cut to its largest value
+    dense = torch.where(dense.isfinite(), dense.clamp(-65504, 65504), dense)
+    # rounded toward zero, as dequantizelinear rounds it
+    near = dense.half()
+    away = near.double().abs() > dense.abs()
+    near = torch.where(away, (near.view(torch.int16) - 1).view(torch.float16), near)
+    want = x.double() @ near.double().t()
+    got = ops.w4a16_gemm(x, w, scales, group, workspace=torch.empty(need, dtype=torch.uint8, device="cuda")).double()
+    tiles = ops.w4a16_gemm(x, w, scales, group).double()
+    for result in (got, tiles):
+        assert bool((result.isnan() == want.isnan()).all())
+        assert bool((result == want)[want.isinf()].all())
+    assert bool(want.isnan().any()) and bool(want.isinf().any())
+    fin = want.isfinite()
+    # of the sums that leave the range for certain both make the same
+    over = fin & (want.abs() > 66000)
+    assert bool(over.any()) and bool((got == tiles)[over].all())
+    size = torch.where(x.isfinite(), x, torch.zeros_like(x)).double().abs() @ \
+        torch.where(near.isfinite(), near, torch.zeros_like(near)).double().abs().t()
+    bound = size * (k * 2.0**-24) + want.abs() * 2.0**-10 + 2.0**-24
+    within = fin & (want.abs() + bound < 65504)
+    for result in (got, tiles):
+        assert bool(((result - want).abs() <= bound)[within].all())
