@@ -7,7 +7,8 @@
 // a lane's fragment is one scale block.  The operator (ref_quant_gemm::compute, four inputs,
 // src/targets/ref/lowering.cpp:221-242) is more general: its scales are float tensors of the
 // operands' own shape, any value per element.  Three kernels keep every input right without a
-// host-side decision:
+// host-side decision (a fourth, mx_tile_kernel, stands for the first two where the result is small and
+// its scales are one float per block):
 //   mx_prepare_kernel   walks the scale tensors once: a block whose 32 scales are one normal power
 //                       of two becomes its exponent byte in a compact [rows, K/32] array; anything
 //                       else raises a flag in device memory (by writing the call's number there:
@@ -526,10 +527,12 @@ int64_t mx_small_tiles(const mx_params& p, int64_t batch)
     return batch * ((p.m + 63) / 64) * ((p.n + 63) / 64);
 }
 
-// Up to two workgroups a CU: the last size at which the small tiles are the faster ones whatever K is
-// (512 of them: 512 x 4096 fp4 with K = 512 / 4096 / 14336 16.2 -> 8.3, 40.0 -> 27.6, 104 -> 76 us; at
-// 1024 a second wave of them costs what the 256 x 256 kernels' whole call does).  One type, scales of one
-// float per block side by side, whole runs of 4 blocks.
+// Up to two workgroups a CU, where the small tiles were the faster ones in each of 1374 products of K = 128 to
+// 14336 (fp4 at most 0.63 of the time of the 256 x 256 kernels' whole call, fp8 0.71; 512 x 4096 fp4 with
+// K = 512 / 4096 / 14336 16.2 -> 8.3, 40.0 -> 27.6, 104 -> 76 us).  Beyond, a third and fourth of
+// them share a CU: of 513 to 767 tiles fp8 takes up to 0.99, of 768 and more up to 1.39, fp4 up to 0.84
+// and 1.17, the long K the most.  One type, scales of one float per block side by side, whole runs
+// of 4 blocks.
 bool mx_tiles_pay(const mx_params& p, int64_t batch)
 {
     const bool compact = p.sa_elem == 0 && p.sb_elem == 0 && p.sa_block == 1 && p.sb_block == 1;

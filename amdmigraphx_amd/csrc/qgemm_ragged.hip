@@ -20,9 +20,12 @@
 // code has no digits: rows of A and columns of B that hold one are noted while they are loaded.
 //
 // What bounds it: 500 x 30522 x 768 int8 -> float is 1810 us in the scalar kernel and 48 us here, of which
-// the 61 MB of C are 12 us at this card's copy rate; the rest is the transposition of B (4-byte loads and
-// the v_perm work of every 128 rows of A again).  fp8 of that size: 150 us, bound by the making of digits.
-// 197 x 197 x 64 in 96 batches: 50 -> 7 us (16 KiB of loads a workgroup and nothing to hide them behind).
+// the 61 MB of C are 12 us at this card's copy rate.  Matrix cores are busy 13 % of it.  190 MB are read
+// behind the L2s, B (23 MB) eight times: a tile's 128 columns of an unaligned row lie in two lines, and
+// the four tiles that share them run on different XCDs (956 tiles, no multiple of 8).  A fifth of
+// the waves' time is vector work (the transposition of B, for every 128 rows of A again), a quarter waits.  fp8 of that size: 150 us, bound by the making
+// of digits.  96 batches of 197 x 197 x 64 (B as [N, K]) 23.7 -> 11.9 us, of 197 x 64 x 197
+// 7.7 us: 16 KiB of loads a workgroup and nothing to hide them behind, matrix cores busy 4 %.
 // Loads without branches and a barrier that leaves them in flight took 128 x 4096 x 4096 from 18.5 to 12.5.
 #include "common.h"
 

@@ -407,7 +407,7 @@ def main():
                 continue
             t2a, _ = _time_launches(skinny, 18, 6, settle_ms=60)
             if not args.no_check:
-                checks[f"int8_quant_dot_M{m2}_atomics"] = sampled_rows_equal(
+                checks[f"int8_quant_dot_M{m2}_no_workspace"] = sampled_rows_equal(
                     c2, a2, bs[(it[0] - 1) % 6].cpu().numpy(), [0, m2 - 1])
             t2, _ = _time_launches(skinny_ws, 18, 6, settle_ms=60)
             if not args.no_check:

@@ -199,10 +199,11 @@ int mi355_convolution_f32(const mi355_quant_conv3d_desc* desc, const float* x, c
                           void* stream);
 
 /* The same with a workspace.  A quant_dot that launches fewer workgroups than the chip has CUs
- * (a skinny or mid-size A against a large B, one image of a convolution) is split along K.
- * Without a workspace only the bare int8 product is split (the shares are added into C with
- * integer atomics); with one, the shares write partial tiles and a second kernel adds them up and
- * applies the dequantizing epilogue (no atomics, no clearing of C).  int8: the same bits as the
+ * (a skinny or mid-size A against a large B, one image of a convolution) can be split along K, and
+ * is where that is the fastest of the kernels that take the call.  Without a workspace only the bare
+ * int8 product can be split (the shares are added into C with integer atomics); with one, the shares
+ * write partial tiles and a second kernel adds them up and applies the dequantizing epilogue (no
+ * atomics, no clearing of C).  int8: the same bits as the
  * unsplit kernel, any N when B is [N, K].  fp8 (one batch, N % 4 == 0): float partial sums added
  * in a fixed order, the same bits on every call, within the fp8 tolerance of the unsplit
  * kernel's.  mi355_quant_dot_workspace_size gives the bytes that description can use (0: none);
