@@ -31,6 +31,12 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
+def _dense(t):
+    """scales, zero points and sums are read as vectors without a stride; the caller keeps a name for the copy until
+    the launch"""
+    return t if t is None or t.is_contiguous() else t.contiguous()
+
+
 def _require_cuda(*ts):
     for t in ts:
         if t is not None and not t.is_cuda:
@@ -127,6 +133,12 @@ def quant_dot(a, b, fp8=False, scale_a=None, scale_b=None, zp_a=0, zp_b=0,
         if bias.dtype != torch.float32 or bias.numel() != (nb * n if cols_per_batch else n) or \
                 not bias.is_contiguous():
             raise Mi355Error("bias must be a dense float32 vector of N elements (batch x N with such scales)")
+    if d.scale_a_mode == QP.PER_ROW:
+        scale_a = _dense(scale_a)
+    if d.scale_b_mode == QP.PER_COL:
+        scale_b = _dense(scale_b)
+    if zp_a or zp_b:
+        colsum_b, rowsum_a = _dense(colsum_b), _dense(rowsum_a)
     if isinstance(workspace, str):
         if workspace != "static":
             raise Mi355Error("workspace must be a device tensor or the word 'static'")
@@ -193,6 +205,14 @@ def quant_dot_prepacked(a, b_prepacked, n, fp8=False, scale_a=None, scale_b=None
                      scale_b_mode=QP.NONE if scale_b is None else
                      (QP.PER_TENSOR if scale_b.numel() == 1 else QP.PER_COL),
                      zp_a=int(zp_a), zp_b=int(zp_b))
+    if d.scale_a_mode == QP.PER_ROW:
+        scale_a = _dense(scale_a)
+    if d.scale_b_mode == QP.PER_COL:
+        scale_b = _dense(scale_b)
+    if zp_a or zp_b:
+        colsum_b, rowsum_a = _dense(colsum_b), _dense(rowsum_a)
+    if bias is not None and not bias.is_contiguous():
+        bias = bias.contiguous()
     check(lib().mi355_quant_dot_prepacked(ctypes.byref(d), _ptr(a), _ptr(b_prepacked), _ptr(out), _ptr(scale_a),
                                           _ptr(scale_b), _ptr(colsum_b), _ptr(rowsum_a), _ptr(bias), _stream()),
           "mi355_quant_dot_prepacked")
@@ -328,6 +348,7 @@ def quant_convolution(x, w, padding=None, stride=None, dilation=None, group=1, f
         if len(_CONV_PLANS) < 256:
             _CONV_PLANS[key] = plan
     d, out_spatial, need_bytes, run, what = plan
+    scale_w = _dense(scale_w)
     shape = (n, o, *out_spatial)
     if out is None:
         out = torch.empty(shape, dtype=odt, device=x.device)
@@ -420,8 +441,7 @@ def quantizelinear(x, scale, zp=None, out_type=DT.I8):
     out = torch.empty(x.shape, dtype=_DT2TORCH[out_type], device=x.device)
     ssr, ssc = _qparam_strides(scale, rows, cols)
     zsr, zsc = _qparam_strides(zp, rows, cols)
-    # named: a dense copy of a strided parameter has to live until the launch
-    scale, zp = scale.contiguous(), None if zp is None else zp.contiguous()
+    scale, zp = _dense(scale), _dense(zp)
     st = lib().mi355_quantizelinear(_ptr(x), _TORCH2DT[x.dtype], _ptr(scale), ssr, ssc, _ptr(zp), zsr, zsc,
                                     _ptr(out), out_type, rows, cols, _stream())
     check(st, "mi355_quantizelinear")
@@ -437,7 +457,7 @@ def dequantizelinear(x, scale, zp=None, x_type=None):
     out = torch.empty(x.shape, dtype=scale.dtype, device=x.device)
     ssr, ssc = _qparam_strides(scale, rows, cols)
     zsr, zsc = _qparam_strides(zp, rows, cols)
-    scale, zp = scale.contiguous(), None if zp is None else zp.contiguous()
+    scale, zp = _dense(scale), _dense(zp)
     st = lib().mi355_dequantizelinear(_ptr(x), xt, _ptr(scale), _TORCH2DT[scale.dtype], ssr, ssc, _ptr(zp), zsr, zsc,
                                       _ptr(out), rows, cols, _stream())
     check(st, "mi355_dequantizelinear")
@@ -536,9 +556,11 @@ def w4a16_gemm(a, w_packed, scales, group, zp=8, zp_mode=None, out=None, workspa
         raise Mi355Error("packed weight does not match K")
     if out is None:
         out = torch.empty((m, n), dtype=torch.float16, device=a.device)
+    w_packed, scales = _dense(w_packed), _dense(scales)
     if isinstance(zp, int):
         zptr, mode, zs = None, W4ZP.SCALAR, zp
     else:
+        zp = _dense(zp)
         zptr, zs = _ptr(zp), 0
         mode = zp_mode if zp_mode is not None else W4ZP.GROUP
     if workspace is not None:
