@@ -213,6 +213,7 @@ def native():
     """The module of plain calls (csrc/torch_calls.cpp), built beside the library; raises if only the library is there."""
     if not os.path.exists(_LIB):
         return _NothingNative()
+    import torch  # noqa: F401  (its libraries are found because they are loaded: the module names no path to them)
     try:
         from . import _torch_calls
     except ImportError as e:
