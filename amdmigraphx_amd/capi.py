@@ -5,6 +5,7 @@ There is no fallback: if the library cannot be loaded every use raises
 import ctypes
 import os
 import subprocess
+import warnings
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 _LIB = os.path.join(_PKG, "lib", "libmi355_qgemm.so")
@@ -202,22 +203,26 @@ def lib():
 
 
 class _NothingNative:
-    """stands for the module of plain calls where nothing is built: every call is left to the Python function, whose
-    first use of the library then says what is missing"""
+    """stands for the module of plain calls where it is not built or cannot be loaded: every call is left to the Python
+    function, which works through ctypes, or whose first use of the library says what is missing"""
 
     def __getattr__(self, name):
         return lambda *args: None
 
 
 def native():
-    """The module of plain calls (csrc/torch_calls.cpp), built beside the library; raises if only the library is there."""
+    """The module of plain calls (csrc/torch_calls.cpp), built beside the library.  It saves host time and nothing
+    else, so a library without it, or a torch that it was not built for, leaves the calls to Python."""
     if not os.path.exists(_LIB):
         return _NothingNative()
     import torch  # noqa: F401  (its libraries are found because they are loaded: the module names no path to them)
     try:
         from . import _torch_calls
     except ImportError as e:
-        raise Mi355Error(f"the library is built, amdmigraphx_amd/_torch_calls is not: run __graft_entry__.build() ({e})") from e
+        if any(name.startswith("_torch_calls.") for name in os.listdir(_PKG)):
+            warnings.warn(f"amdmigraphx_amd/_torch_calls cannot be loaded, calls go through ctypes: {e}", RuntimeWarning,
+                          stacklevel=2)
+        return _NothingNative()
     return _torch_calls
 
 

@@ -23,3 +23,21 @@ def test_loads_where_torch_is_not(first):
                  "print(capi.native().__name__)", cwd=ROOT)
     assert got.returncode == 0, got.stderr
     assert got.stdout.split() == ["amdmigraphx_amd._torch_calls"]
+
+
+@pytest.mark.parametrize("module", ["missing", "broken"])
+def test_the_functions_need_the_library_alone(tmp_path, module):
+    """a library made by its own target, or a torch that the module was not built for: calls go through ctypes"""
+    package = tmp_path / "amdmigraphx_amd"
+    package.mkdir()
+    source = os.path.join(ROOT, "amdmigraphx_amd")
+    for name in ("__init__.py", "capi.py", "ops.py", "lib"):
+        os.symlink(os.path.join(source, name), package / name)
+    if module == "broken":
+        suffix = next(n for n in os.listdir(source) if n.startswith("_torch_calls.")).split(".", 1)[1]
+        (package / f"_torch_calls.{suffix}").write_bytes(b"\x7fELF")
+    got = _child("from amdmigraphx_amd import capi, ops; assert isinstance(ops._native, capi._NothingNative); "
+                 "print(ops.quant_dot_workspace_size(16, 512, 8192) > 0)", cwd=tmp_path)
+    assert got.returncode == 0, got.stderr
+    assert got.stdout.split() == ["True"]
+    assert ("cannot be loaded" in got.stderr) == (module == "broken")
