@@ -174,7 +174,9 @@ def build_library(force=True):
     cmd = ["make", "-C", os.path.join(_PKG, "csrc"), "-j8"]
     if force:
         cmd.append("-B")
-    subprocess.check_call(cmd, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    made = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if made.returncode != 0:
+        raise Mi355Error(f"{' '.join(cmd)} failed ({made.returncode}):\n{made.stdout}")
 
 
 _handle = None

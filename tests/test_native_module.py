@@ -41,3 +41,11 @@ def test_the_functions_need_the_library_alone(tmp_path, module):
     assert got.returncode == 0, got.stderr
     assert got.stdout.split() == ["True"]
     assert ("cannot be loaded" in got.stderr) == (module == "broken")
+
+
+def test_a_failed_build_shows_what_the_compiler_said(tmp_path, monkeypatch):
+    (tmp_path / "csrc").mkdir()
+    (tmp_path / "csrc" / "Makefile").write_text("all:\n\t@echo 'x.hip:7: error: no such builtin' >&2; exit 1\n")
+    monkeypatch.setattr(capi, "_PKG", str(tmp_path))
+    with pytest.raises(capi.Mi355Error, match="x.hip:7: error: no such builtin"):
+        capi.build_library()
