@@ -49,3 +49,40 @@ def test_gather_rows(words, kind, shift):
                                   torch.cuda.current_stream().cuda_stream), "gather")
     at = torch.where((ids >= rows) | (ids < -rows), torch.zeros_like(ids), torch.where(ids < 0, ids + rows, ids)).long()
     assert torch.equal(out[:n], table[at]) and bool((out[n] == -1).all())
+
+
+def _gather(table, ids, out):
+    check(lib().mi355_gather_rows(_ptr(table), _ptr(ids), int(ids.dtype == torch.int64), _ptr(out), len(ids), len(table),
+                                  table.shape[1] * 4, torch.cuda.current_stream().cuda_stream), "gather")
+
+
+@pytest.mark.parametrize("n,words", [(1, 294912), (3, 100000), (3, 100001), (2, 1023), (5, 1024), (1, 1028), (70000, 64),
+                                     (20000, 255), (20000, 1024 + 4)])
+def test_gather_of_few_long_rows_and_many_short_ones(n, words):
+    """a row in many pieces (whole and begun), and more pieces than there are waves"""
+    rows = 40
+    g = torch.Generator(device="cuda").manual_seed(words)
+    table = torch.randn(rows, words, generator=g, device="cuda")
+    ids = torch.randint(0, rows, (n,), generator=g, device="cuda")
+    out = torch.full((n + 1, words), -1.0, device="cuda")
+    _gather(table, ids, out)
+    assert torch.equal(out[:n], table[ids]) and bool((out[n] == -1).all())
+
+
+def test_one_long_row_is_copied_by_the_whole_chip():
+    """A row of 5 MB takes about what a copy of it does; one wave by itself would take some hundred times that."""
+    table, out = torch.ones(3, 1310720, device="cuda"), torch.empty(1, 1310720, device="cuda")
+    ids = torch.tensor([1], device="cuda")
+
+    def best(call):
+        times = []
+        for _ in range(20):
+            start, stop = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            call()
+            stop.record()
+            stop.synchronize()
+            times.append(start.elapsed_time(stop))
+        return min(times)
+
+    assert best(lambda: _gather(table, ids, out)) < 20 * best(lambda: out.copy_(table[1:2]))
