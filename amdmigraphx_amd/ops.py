@@ -15,7 +15,8 @@ from .capi import DT, QP, W4ZP, QuantDotDesc, QuantConv3dDesc, QuantConvDesc, Mx
 
 # The plain calls in native code (csrc/torch_calls.cpp): ordinary dense device tensors, nothing to convert, copy or
 # refuse.  None means that the function below has to look at the call itself, which then does what it always
-# did; so it does where something stands in for the library (`lib`), which is to see every call.  Host time of a call,
+# did, 0.2 us later; an output of the caller's goes there at once.  So does every call where something stands in for
+# the library (`lib`), which is to see them all.  Host time of a call,
 # Python and ctypes -> native (us): quantizelinear 7.4 -> 3.7, pack_int4 6.3 -> 3.7, quant_dot with epilogue and bias
 # 11.2 -> 3.9, prepacked 8.2 -> 3.8, quant_dot_mx 17.3 -> 7.2 (two launches), convolution 13.2 -> 7.3 (two), w4a16_gemm
 # 7.4 -> 3.8; a torch.empty is 1.7 of each and a launch about 2.
@@ -80,10 +81,11 @@ def quant_dot(a, b, fp8=False, scale_a=None, scale_b=None, zp_a=0, zp_b=0,
     product, bare or with the epilogue, split K over the chip without atomics; the word
     ``"static"`` takes the library's own static device buffer instead (nothing is allocated,
     shapes that need more than it holds are refused)."""
-    done = None if lib is not _library else _native.quant_dot(a, b, fp8, scale_a, scale_b, zp_a, zp_b, colsum_b,
-        rowsum_a, out_dtype, out, bias, workspace)
-    if done is not None:
-        return done
+    if out is None and lib is _library:
+        done = _native.quant_dot(a, b, fp8, scale_a, scale_b, zp_a, zp_b, colsum_b, rowsum_a, out_dtype, out, bias,
+                                 workspace)
+        if done is not None:
+            return done
     _require_cuda(a, b, scale_a, scale_b, bias, None if isinstance(workspace, str) else workspace)
     if a.dim() != b.dim() or a.dim() < 2:
         raise Mi355Error("QUANT_DOT: dot only accepts >= 2D operands of equal rank")
@@ -204,10 +206,11 @@ def quant_dot_prepacked(a, b_prepacked, n, fp8=False, scale_a=None, scale_b=None
                         colsum_b=None, rowsum_a=None, out_dtype=None, out=None, bias=None):
     """quant_dot of a [M <= 16, K] against a B reordered by quant_dot_prepack, with the epilogue
     arguments of quant_dot; one launch, no workspace."""
-    done = None if lib is not _library else _native.quant_dot_prepacked(a, b_prepacked, n, fp8, scale_a, scale_b, zp_a,
-        zp_b, colsum_b, rowsum_a, out_dtype, out, bias)
-    if done is not None:
-        return done
+    if out is None and lib is _library:
+        done = _native.quant_dot_prepacked(a, b_prepacked, n, fp8, scale_a, scale_b, zp_a, zp_b, colsum_b, rowsum_a,
+                                           out_dtype, out, bias)
+        if done is not None:
+            return done
     _require_cuda(a, b_prepacked, scale_a, scale_b, bias)
     if a.dim() != 2 or a.stride(1) != 1:
         raise Mi355Error("quant_dot_prepacked: A is a row-major matrix")
@@ -247,10 +250,10 @@ def quant_dot_mx(a, b_nk, scale_a, scale_b, a_fp4=False, b_fp4=False, out=None, 
     float32, either of the operand's logical shape ([..., M, K], the operator's form) or compact
     ([..., M, K/32], one per block).  Returns float32 [..., M, N].  ``workspace``: a dense uint8
     device tensor to use (and keep between calls) instead of a fresh allocation."""
-    done = None if lib is not _library else _native.quant_dot_mx(a, b_nk, scale_a, scale_b, a_fp4, b_fp4, out,
-        workspace)
-    if done is not None:
-        return done
+    if out is None and lib is _library:
+        done = _native.quant_dot_mx(a, b_nk, scale_a, scale_b, a_fp4, b_fp4, out, workspace)
+        if done is not None:
+            return done
     _require_cuda(a, b_nk, scale_a, scale_b)
     if a.dtype != torch.uint8 or b_nk.dtype != torch.uint8:
         raise Mi355Error("quant_dot_mx: operands are uint8 tensors of fp8 codes or packed fp4 pairs")
@@ -337,10 +340,11 @@ def quant_convolution(x, w, padding=None, stride=None, dilation=None, group=1, f
     or the low values followed by the high ones.  ``out`` (dense, of the result's shape and type)
     and ``workspace`` (a uint8 tensor of at least the size the library asks for) are allocated
     here unless the caller brings them, e.g. to reuse them from call to call."""
-    done = None if lib is not _library else _native.quant_convolution(x, w, padding, stride, dilation, group, fp8,
-        scale_x, scale_w, out_dtype, out, workspace)
-    if done is not None:
-        return done
+    if out is None and workspace is None and lib is _library:
+        done = _native.quant_convolution(x, w, padding, stride, dilation, group, fp8, scale_x, scale_w, out_dtype,
+                                         out, workspace)
+        if done is not None:
+            return done
     _require_cuda(x, w, scale_x, scale_w)
     nd = x.dim() - 2
     if nd < 1 or nd > 3 or w.dim() != x.dim():
@@ -460,9 +464,10 @@ def _qparam_strides(p, rows, cols):
 def quantizelinear(x, scale, zp=None, out_type=DT.I8):
     """quantizelinear of a dense tensor (last dim = columns).  ``scale`` has
     x's dtype; ``zp`` the output's (uint8 bits for fp8)."""
-    done = None if lib is not _library else _native.quantizelinear(x, scale, zp, out_type)
-    if done is not None:
-        return done
+    if lib is _library:
+        done = _native.quantizelinear(x, scale, zp, out_type)
+        if done is not None:
+            return done
     _require_cuda(x, scale, zp)
     x = x.contiguous()
     cols = x.shape[-1]
@@ -480,9 +485,10 @@ def quantizelinear(x, scale, zp=None, out_type=DT.I8):
 
 
 def dequantizelinear(x, scale, zp=None, x_type=None):
-    done = None if lib is not _library else _native.dequantizelinear(x, scale, zp, x_type)
-    if done is not None:
-        return done
+    if lib is _library:
+        done = _native.dequantizelinear(x, scale, zp, x_type)
+        if done is not None:
+            return done
     _require_cuda(x, scale, zp)
     x = x.contiguous()
     cols = x.shape[-1]
@@ -538,9 +544,10 @@ def _int4_nd(fn_name, x, axis, out_shape):
 
 def unpack_int4(x, axis=-1):
     """unpack_int4 along ``axis`` of any strided view (transposed, expanded): the result is dense."""
-    done = None if lib is not _library else _native.unpack_int4(x, axis)
-    if done is not None:
-        return done
+    if lib is _library:
+        done = _native.unpack_int4(x, axis)
+        if done is not None:
+            return done
     _require_cuda(x)
     ax = axis % x.dim()
     shp = list(x.shape)
@@ -556,9 +563,10 @@ def unpack_int4(x, axis=-1):
 
 
 def pack_int4(x, axis=-1):
-    done = None if lib is not _library else _native.pack_int4(x, axis)
-    if done is not None:
-        return done
+    if lib is _library:
+        done = _native.pack_int4(x, axis)
+        if done is not None:
+            return done
     _require_cuda(x)
     ax = axis % x.dim()
     shp = list(x.shape)
@@ -589,9 +597,10 @@ def w4a16_gemm(a, w_packed, scales, group, zp=8, zp_mode=None, out=None, workspa
     group scales [N, K/group]; zp is an int (per tensor) or a uint8 tensor.
     ``workspace`` (a dense device tensor, see w4a16_gemm_workspace_size) lets many rows multiply
     weights dequantized once, and shapes whose column tiles do not fill the chip split K."""
-    done = None if lib is not _library else _native.w4a16_gemm(a, w_packed, scales, group, zp, zp_mode, out, workspace)
-    if done is not None:
-        return done
+    if out is None and lib is _library:
+        done = _native.w4a16_gemm(a, w_packed, scales, group, zp, zp_mode, out, workspace)
+        if done is not None:
+            return done
     _require_cuda(a, w_packed, scales, workspace)
     m, k = a.shape
     n = w_packed.shape[0]
@@ -639,9 +648,10 @@ def w4a16_prepack(w_packed, scales, group, zp=8):
 
 def w4a16_gemm_prepacked(a, prepacked, n, out=None):
     """fp16 activations [M, K] times weights reordered by w4a16_prepack (N rows)."""
-    done = None if lib is not _library else _native.w4a16_gemm_prepacked(a, prepacked, n, out)
-    if done is not None:
-        return done
+    if out is None and lib is _library:
+        done = _native.w4a16_gemm_prepacked(a, prepacked, n, out)
+        if done is not None:
+            return done
     _require_cuda(a, prepacked)
     m, k = a.shape
     if out is None:
