@@ -118,8 +118,8 @@ def quant_dot(a, b, fp8=False, scale_a=None, scale_b=None, zp_a=0, zp_b=0,
     if out is None:
         out = torch.empty(batch_shape + (m, n), dtype=odt, device=a.device)
     # the kernels store elements of odt: into narrower ones they would write past the end
-    elif out.dtype.itemsize != odt.itemsize:
-        raise Mi355Error("quant_dot: the output's elements are not those of the result's type")
+    elif out.dtype.itemsize < odt.itemsize:
+        raise Mi355Error("quant_dot: the output's elements are narrower than those of the result's type")
     # C may be a row-strided view (columns contiguous, batches evenly spaced)
     if out.stride(-1) != 1 and n > 1:
         raise Mi355Error("quant_dot: the output's last dimension must be contiguous")
