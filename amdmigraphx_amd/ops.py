@@ -53,6 +53,29 @@ def _require_cuda(*ts):
             raise Mi355Error("operands must be device tensors")
 
 
+def _require_room(what, out, itemsize, rows, ld, cols, batch=1, batch_stride=0):
+    """The kernels store `batch` matrices of `rows` rows, `ld` elements apart, of `cols` elements side by side, whatever
+    the caller's tensor is like: one that does not hold them would have the memory behind it overwritten."""
+    if not out.is_cuda and not out.is_pinned():
+        raise Mi355Error(f"{what}: the output must be a device tensor")
+    if rows * cols * batch == 0:
+        return
+    need = ((batch - 1) * batch_stride + (rows - 1) * ld + cols) * itemsize
+    if out.is_contiguous():
+        have = out.nbytes
+    else:
+        have = out.element_size() * (1 + sum((n - 1) * s for n, s in zip(out.shape, out.stride()))) if out.numel() else 0
+    if need > have:
+        raise Mi355Error(f"{what}: the output does not hold the result")
+
+
+def _require_rows(what, out, itemsize, m, n):
+    """the same for one matrix in the rows of `out`"""
+    if out.stride(-1) != 1 and n > 1:
+        raise Mi355Error(f"{what}: the output's last dimension must be contiguous")
+    _require_room(what, out, itemsize, m, out.stride(0), n)
+
+
 def _mat_layout(t):
     """(trans, ld, batch_stride) of a [..., R, C] view that is row-major or a
     transpose of row-major storage in its last two dims."""
@@ -115,7 +138,8 @@ def quant_dot(a, b, fp8=False, scale_a=None, scale_b=None, zp_a=0, zp_b=0,
         odt = out_dtype or torch.float32
     else:
         odt = torch.float32 if fp8 else torch.int32
-    if out is None:
+    own = out is not None
+    if not own:
         out = torch.empty(batch_shape + (m, n), dtype=odt, device=a.device)
     # the kernels store elements of odt: into narrower ones they would write past the end
     elif out.dtype.itemsize < odt.itemsize:
@@ -129,6 +153,8 @@ def quant_dot(a, b, fp8=False, scale_a=None, scale_b=None, zp_a=0, zp_b=0,
         if out.dim() > 3 and not out.flatten(0, -3).is_contiguous():
             raise Mi355Error("quant_dot: batch dimensions of the output must be dense")
         stride_c = out.stride(-3)
+    if own:
+        _require_room("quant_dot", out, odt.itemsize, m, ldc, n, nb, stride_c)
     # one vector of column scales (and one bias) per batch entry: scale_b dense [batch, N]
     cols_per_batch = (scale_b is not None and nb > 1 and scale_b.dim() >= 2 and scale_b.numel() == nb * n and
                       scale_b.is_contiguous())
@@ -219,6 +245,8 @@ def quant_dot_prepacked(a, b_prepacked, n, fp8=False, scale_a=None, scale_b=None
     odt = (out_dtype or torch.float32) if dequant else (torch.float32 if fp8 else torch.int32)
     if out is None:
         out = torch.empty((m, n), dtype=odt, device=a.device)
+    else:
+        _require_rows("quant_dot_prepacked", out, out.dtype.itemsize, m, n)
     d = QuantDotDesc(m=m, n=n, k=k, lda=a.stride(0) if m > 1 else max(k, a.stride(0)), ldb=n,
                      ldc=out.stride(0) if m > 1 else max(n, out.stride(0)), batch=1, stride_a=0, stride_b=0,
                      stride_c=0, trans_a=0, trans_b=0, in_type=_fp8_dt(fp8, a), out_type=_TORCH2DT[out.dtype],
@@ -282,10 +310,18 @@ def quant_dot_mx(a, b_nk, scale_a, scale_b, a_fp4=False, b_fp4=False, out=None, 
 
     sab, sar, sak, sae = scale_strides(scale_a, m)
     sbb, sbr, sbk, sbe = scale_strides(scale_b, n)
+    ldc, stride_c = n, m * n
     if out is None:
         out = torch.empty(batch_shape + (m, n), dtype=torch.float32, device=a.device)
-    d = MxDotDesc(m=m, n=n, k=k, batch=nb, lda=a.shape[-1], ldb=b_nk.shape[-1], ldc=n,
-                  stride_a=m * a.shape[-1], stride_b=n * b_nk.shape[-1], stride_c=m * n,
+    else:
+        if not out.is_contiguous():  # rows (and batches) of a wider tensor
+            if (out.stride(-1) != 1 and n > 1) or out.dim() != 2 + (nb > 1):
+                raise Mi355Error("quant_dot_mx: the output must be dense, or evenly spaced rows of one")
+            ldc = out.stride(-2) if m > 1 else max(n, out.stride(-2))
+            stride_c = out.stride(0) if nb > 1 else m * ldc
+        _require_room("quant_dot_mx", out, 4, m, ldc, n, nb, stride_c)
+    d = MxDotDesc(m=m, n=n, k=k, batch=nb, lda=a.shape[-1], ldb=b_nk.shape[-1], ldc=ldc,
+                  stride_a=m * a.shape[-1], stride_b=n * b_nk.shape[-1], stride_c=stride_c,
                   sa_batch=sab, sa_row=sar, sa_block=sak, sa_elem=sae,
                   sb_batch=sbb, sb_row=sbr, sb_block=sbk, sb_elem=sbe,
                   a_type=DT.FP4X2 if a_fp4 else DT.FP8, b_type=DT.FP4X2 if b_fp4 else DT.FP8)
@@ -608,6 +644,8 @@ def w4a16_gemm(a, w_packed, scales, group, zp=8, zp_mode=None, out=None, workspa
         raise Mi355Error("packed weight does not match K")
     if out is None:
         out = torch.empty((m, n), dtype=torch.float16, device=a.device)
+    else:
+        _require_rows("w4a16_gemm", out, 2, m, n)
     w_packed, scales = _dense(w_packed), _dense(scales)
     if isinstance(zp, int):
         zptr, mode, zs = None, W4ZP.SCALAR, zp
@@ -656,6 +694,8 @@ def w4a16_gemm_prepacked(a, prepacked, n, out=None):
     m, k = a.shape
     if out is None:
         out = torch.empty((m, n), dtype=torch.float16, device=a.device)
+    else:
+        _require_rows("w4a16_gemm_prepacked", out, 2, m, n)
     check(lib().mi355_w4a16_gemm_prepacked(_ptr(a), a.stride(0), _ptr(prepacked), _ptr(out), out.stride(0),
                                            m, n, k, _stream()), "mi355_w4a16_gemm_prepacked")
     return out

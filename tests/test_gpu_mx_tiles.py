@@ -89,3 +89,17 @@ def test_a_scale_of_any_quarter_and_chunk_raises_the_flag(ops, fp4):
         x = (va[0] * sa[0].double().repeat_interleave(32, dim=1)).float().double()
         w = (vb[0] * sb[0].double().repeat_interleave(32, dim=1)).float().double()
         assert torch.equal(got[0], (x @ w.t()).float()), (is_b, row, block)
+
+
+@pytest.mark.parametrize("batch,m,n,k", [(1, 40, 70, 512), (3, 33, 20, 256), (1, 2100, 4104, 4096)])
+def test_rows_of_a_wider_output(ops, batch, m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m)
+    a, _, sa = _operands(g, m, k, False, batch)
+    b, _, sb = _operands(g, n, k, False, batch)
+    room = torch.full((batch, m + 1, n + 8), -1.0, device="cuda")
+    out = room[:, :m, 4:4 + n]
+    args = (a, b, sa, sb) if batch > 1 else (a[0], b[0], sa[0], sb[0])
+    ops.quant_dot_mx(*args, out=out if batch > 1 else out[0])
+    want = ops.quant_dot_mx(*args)
+    assert torch.equal(out, want.view(batch, m, n))
+    assert bool((room[:, m] == -1).all()) and bool((room[:, :, :4] == -1).all()) and bool((room[:, :, 4 + n:] == -1).all())
