@@ -347,8 +347,9 @@ size_t small_tile_bytes(const mi355_quant_dot_desc* d, int shares)
 // costs a workgroup alone on its CU, the partial sums' way, and a start that grows with the workgroups, fitted to 40
 // products of 20 to 1000 rows (within 10 %), against the fits above.  Not beyond one workgroup a CU; from 65
 // tiles on two or three shares gain nothing (512 x 4096 x 4096 28.0 us in one pass of 64 x 64 tiles).  Not beyond
-// the 32 MiB that callers without an allocator have.  A function of the shape and the operands' types
-// alone, so that the size asked for ahead of a call is that of the call.
+// the 32 MiB that callers without an allocator have.  A function of the shape, B's order and the operands' types
+// alone (the fits look at dense matrices, whatever the distance of the rows), so that the size asked for ahead of a call
+// is that of the call.
 int small_tile_shares(const mi355_quant_dot_desc* d0)
 {
     if((d0->in_type != MI355_I8 && d0->in_type != MI355_FP8) || d0->batch != 1 || d0->trans_a || d0->m <= 0 ||
@@ -357,6 +358,9 @@ int small_tile_shares(const mi355_quant_dot_desc* d0)
         return 1;
     mi355_quant_dot_desc d = *d0;
     d.dequant              = 0;
+    d.lda                  = d.k;
+    d.ldb                  = d.trans_b ? d.k : d.n;
+    d.ldc                  = d.n;
     const double tiles     = tiles_of(&d, 128);
     if(tiles > 64)
         return 1;

@@ -58,6 +58,20 @@ def test_a_workspace_is_used_where_the_shares_are_faster(m, n, k, trans_b, kerne
     assert kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, out=out, workspace=1 << 10) in ("ragged", "dma_atomic")
 
 
+@pytest.mark.parametrize("m,n,k,trans_b,fp8", [
+    (640, 1520, 6656, False, True), (897, 400, 6016, False, True), (142, 2128, 5504, False, True),
+    (543, 1376, 4224, False, False), (291, 912, 2752, False, False), (127, 6304, 3776, False, False),
+    (16, 512, 4096, False, True), (16, 512, 4096, False, False), (1, 16, 4160, True, True), (1, 16, 4160, True, False)])
+def test_the_size_asked_for_serves_any_distance_of_the_rows(m, n, k, trans_b, fp8):
+    """rows of B that lie a multiple of 1 KiB apart take another time, yet the size is asked for without it"""
+    from amdmigraphx_amd import ops
+    need = ops.quant_dot_workspace_size(m, n, k, trans_b=trans_b, fp8=fp8)
+    kernel = kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, workspace=need)
+    for ldb in ((k if trans_b else n) + 1023) // 1024 * 1024, ((k if trans_b else n) + 1039) // 16 * 16:
+        for lda in (k, k + 64):
+            assert kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, lda=lda, ldb=ldb, workspace=need) == kernel
+
+
 def test_large_and_small_grids():
     for fp8 in (False, True):
         for out in (None, "bf16", "f32"):
