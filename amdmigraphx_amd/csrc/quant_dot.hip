@@ -781,8 +781,8 @@ extern "C" int mi355_quant_dot_static(const mi355_quant_dot_desc* d,
 {
     if(d == nullptr)
         return MI355_ERR_BAD_ARG;
-    // by the need of the 256 x 256 tiles, whatever the smaller ones ask for: what is refused, and what shares
-    // nothing with a call on another stream, is the same for both
+    // By the need of the 256 x 256 tiles, whatever the smaller ones ask for: callers rely on what is refused, and on
+    // what shares nothing with a call on another stream, and neither follows the choice of a tile.
     const size_t large = mi355_dma_gemm_workspace(d);
     if(large > MI355_QUANT_DOT_STATIC_SCRATCH_BYTES)
         return MI355_ERR_SCRATCH_TOO_SMALL;

@@ -204,7 +204,7 @@ int mi355_convolution_f32(const mi355_quant_conv3d_desc* desc, const float* x, c
  * int8 product can be split (the shares are added into C with integer atomics); with one, the shares
  * write partial tiles and a second kernel adds them up and applies the dequantizing epilogue (no
  * atomics, no clearing of C).  int8: the same bits as the
- * unsplit kernel, any N when B is [N, K].  fp8 (one batch, N % 4 == 0): float partial sums added
+ * unsplit kernel, any N when B is [N, K].  fp8 (one batch): float partial sums added
  * in a fixed order, the same bits on every call, within the fp8 tolerance of the unsplit
  * kernel's.  mi355_quant_dot_workspace_size gives the bytes that description can use (0: none);
  * a NULL or smaller workspace is not an error, the call then behaves like mi355_quant_dot_bias.
@@ -222,11 +222,14 @@ int mi355_quant_dot_ws(const mi355_quant_dot_desc* desc, const void* a, const vo
  * result as mi355_quant_dot_ws; the split-K partial sums go to a buffer of
  * MI355_QUANT_DOT_STATIC_SCRATCH_BYTES that is part of the library's device code (one copy per
  * GPU, held from module load until the process ends).  The call itself allocates and frees
- * nothing; the first call on a device looks the buffer's address up once.  A description whose
- * mi355_quant_dot_workspace_size exceeds the buffer is refused with MI355_ERR_SCRATCH_TOO_SMALL
- * (nothing is launched).  All calls on one GPU share the buffer: calls that may run at the same
- * time on one GPU (different streams, different threads) race on it and must be ordered by the
- * caller.  The buffer keeps the last call's partial sums; no call depends on its contents. */
+ * nothing; the first call on a device looks the buffer's address up once.  A description is refused
+ * with MI355_ERR_SCRATCH_TOO_SMALL (nothing is launched) by what its split in 256 x 256 tiles needs:
+ * always where mi355_quant_dot_workspace_size exceeds the buffer, and also where only the smaller
+ * tiles that mi355_quant_dot_ws would take there stay below it.  Where the 256 x 256 tiles would
+ * not split, the call runs as without a workspace and leaves the buffer alone (fp8 sums are then
+ * added in another order than mi355_quant_dot_ws adds them with room for small tiles).  All calls on
+ * one GPU share the buffer: calls that may run at the same time on one GPU (different streams,
+ * different threads) race on it and must be ordered by the caller.  The buffer keeps the last call's partial sums; no call depends on its contents. */
 #define MI355_QUANT_DOT_STATIC_SCRATCH_BYTES (32u << 20)
 int mi355_quant_dot_static(const mi355_quant_dot_desc* desc, const void* a, const void* b, void* c,
                            const float* scale_a, const float* scale_b, const int32_t* colsum_b,

@@ -72,6 +72,19 @@ def test_the_size_asked_for_serves_any_distance_of_the_rows(m, n, k, trans_b, fp
             assert kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, lda=lda, ldb=ldb, workspace=need) == kernel
 
 
+@pytest.mark.parametrize("m,n,k,trans_b,fp8", [(318, 1664, 12672, True, False), (750, 880, 12480, True, True),
+                                               (255, 8192, 8192, False, False)])
+def test_the_static_entry_refuses_by_the_large_tiles(m, n, k, trans_b, fp8):
+    """two products that would split in small tiles with less than the buffer, and one that would not"""
+    import ctypes
+    from amdmigraphx_amd import ops
+    d = capi.QuantDotDesc(m=m, n=n, k=k, lda=k, ldb=k if trans_b else n, ldc=n, batch=1, trans_b=int(trans_b),
+                          in_type=capi.DT.FP8 if fp8 else capi.DT.I8, out_type=capi.DT.F32 if fp8 else capi.DT.I32)
+    status = capi.lib().mi355_quant_dot_static(ctypes.byref(d), *[ctypes.c_void_p(1 << 20)] * 3, *[None] * 6)
+    assert status == -4  # MI355_ERR_SCRATCH_TOO_SMALL
+    assert (ops.quant_dot_workspace_size(m, n, k, trans_b=trans_b, fp8=fp8) > 32 << 20) == (m == 255)
+
+
 def test_large_and_small_grids():
     for fp8 in (False, True):
         for out in (None, "bf16", "f32"):

@@ -27,9 +27,12 @@ def _operands(m, n, k, trans_b, seed):
 
 
 def test_two_calls_in_a_row_second_one_smaller(ops):
-    # (128, 8192, 8192) fills the static buffer to its last byte; (16, 1024, 4096) then reuses
-    # its first quarter MiB with the larger call's partial sums still in it
-    for m, n, k, trans_b in ((128, 8192, 8192, False), (16, 1024, 4096, True)):
+    # (128, 16384, 4096) fills the static buffer to its last byte, (128, 8192, 8192) in small tiles half of it;
+    # (16, 1024, 4096) then reuses its first MiB with the larger calls' partial sums still in it
+    needs = [ops.quant_dot_workspace_size(m, n, k, 1, t) for m, n, k, t in
+             ((128, 16384, 4096, False), (128, 8192, 8192, False), (16, 1024, 4096, True))]
+    assert needs[0] == STATIC_BYTES and needs[1] == STATIC_BYTES // 2 and needs[2] <= 1 << 20
+    for m, n, k, trans_b in ((128, 16384, 4096, False), (128, 8192, 8192, False), (16, 1024, 4096, True)):
         print("static scratch", m, n, k, trans_b, flush=True)
         a, b = _operands(m, n, k, trans_b, m + n)
         need = ops.quant_dot_workspace_size(m, n, k, 1, trans_b)
