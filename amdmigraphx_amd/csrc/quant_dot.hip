@@ -470,7 +470,8 @@ bool mfma_takes(const mi355_quant_dot_desc* d, const void* a, const void* b, con
            mi355_mfma_gemm_supported(d, a, b, c);
 }
 
-// argument checks and the choice of the kernel; the pointers are looked at, not through
+// argument checks and the choice of the kernel, and for dma_shares of the tiles: *small shares in those of 128 x 128
+// (1: 256 x 256); the pointers are looked at, not through
 int choose_kernel(const mi355_quant_dot_desc* d,
                   const void* a,
                   const void* b,
@@ -482,7 +483,8 @@ int choose_kernel(const mi355_quant_dot_desc* d,
                   const float* bias,
                   const void* workspace,
                   size_t workspace_bytes,
-                  kernel_id* kernel)
+                  kernel_id* kernel,
+                  int* small)
 {
     if(d == nullptr)
         return MI355_ERR_BAD_ARG;
@@ -535,6 +537,7 @@ int choose_kernel(const mi355_quant_dot_desc* d,
             return MI355_ERR_BAD_ARG;
     }
     *kernel = kernel_id::none;
+    *small  = 1;
     if(empty)
         return MI355_OK;
     if(d->ldc < d->n)
@@ -547,7 +550,8 @@ int choose_kernel(const mi355_quant_dot_desc* d,
     if(dma_takes(d, a, b, bias))
     {
         // fp8: the sums of all are float
-        if(small_tile_shares(d, workspace, workspace_bytes) > 1)
+        *small = small_tile_shares(d, workspace, workspace_bytes);
+        if(*small > 1)
         {
             *kernel = kernel_id::dma_shares;
             return MI355_OK;
@@ -583,6 +587,7 @@ int choose_kernel(const mi355_quant_dot_desc* d,
 namespace {
 
 int launch_kernel(kernel_id kernel,
+                  int small, // as choose_kernel gives it
                   const mi355_quant_dot_desc* d,
                   const void* a,
                   const void* b,
@@ -608,9 +613,8 @@ int launch_kernel(kernel_id kernel,
     case kernel_id::dma:
     case kernel_id::dma_shares:
     case kernel_id::dma_atomic:
-        return mi355_dma_gemm_launch(
-            d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace, workspace_bytes,
-            kernel == kernel_id::dma_shares ? small_tile_shares(d, workspace, workspace_bytes) : 1, s);
+        return mi355_dma_gemm_launch(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
+                                     workspace_bytes, small, s);
     case kernel_id::generic: break;
     }
 
@@ -664,15 +668,17 @@ extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
                                   void* stream)
 {
     kernel_id kernel = kernel_id::none;
+    int small        = 1;
     const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
-                                     workspace_bytes, &kernel);
+                                     workspace_bytes, &kernel, &small);
     return status != MI355_OK ? status
-                              : launch_kernel(kernel, d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
-                                              workspace_bytes, static_cast<hipStream_t>(stream));
+                              : launch_kernel(kernel, small, d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias,
+                                              workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
-// The two below are not part of the public interface.  Tests ask the first, without a GPU, which kernel their
-// shapes reach (the kernel_id, or the call's negative status), and with the second run the edges of
+// The three below are not part of the public interface.  Tests ask the first, without a GPU, which kernel their
+// shapes reach (the kernel_id, or the call's negative status), the second how many shares a workspace of those bytes
+// has in 128 x 128 tiles (1: none), and with the third run the edges of
 // a kernel at sizes that the rules leave to another (the product, or MI355_ERR_UNSUPPORTED where the
 // kernel does not take it).
 extern "C" int mi355_internal_quant_dot_kernel(const mi355_quant_dot_desc* d,
@@ -688,9 +694,16 @@ extern "C" int mi355_internal_quant_dot_kernel(const mi355_quant_dot_desc* d,
                                                size_t workspace_bytes)
 {
     kernel_id kernel = kernel_id::none;
+    int small        = 1;
     const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
-                                     workspace_bytes, &kernel);
+                                     workspace_bytes, &kernel, &small);
     return status == MI355_OK ? (int)kernel : status;
+}
+
+extern "C" int mi355_internal_quant_dot_small_shares(const mi355_quant_dot_desc* d, size_t workspace_bytes)
+{
+    const int shares = small_tile_shares(d);
+    return shares > 1 && small_tile_bytes(d, shares) <= workspace_bytes ? shares : 1;
 }
 
 extern "C" int mi355_internal_quant_dot_run(int32_t which,
@@ -708,8 +721,9 @@ extern "C" int mi355_internal_quant_dot_run(int32_t which,
                                             void* stream)
 {
     kernel_id kernel = kernel_id::none;
+    int small        = 1;
     const int status = choose_kernel(d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias, workspace,
-                                     workspace_bytes, &kernel);
+                                     workspace_bytes, &kernel, &small);
     if(status != MI355_OK || kernel == kernel_id::none)
         return status;
     bool takes = false;
@@ -724,8 +738,8 @@ extern "C" int mi355_internal_quant_dot_run(int32_t which,
     default: break;
     }
     return !takes ? MI355_ERR_UNSUPPORTED
-                  : launch_kernel(static_cast<kernel_id>(which), d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a, bias,
-                                  workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+                  : launch_kernel(static_cast<kernel_id>(which), 1, d, a, b, c, scale_a, scale_b, colsum_b, rowsum_a,
+                                  bias, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 // ---- quant_dot that allocates nothing and takes no workspace -------------------------------
