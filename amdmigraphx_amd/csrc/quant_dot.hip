@@ -345,11 +345,11 @@ size_t small_tile_bytes(const mi355_quant_dot_desc* d, int shares)
 
 // Shares of K in 128 x 128 tiles (qgemm_shares.h), 1 where another kernel is the faster one: what a slab of 128
 // costs a workgroup alone on its CU, the partial sums' way, and a start that grows with the workgroups, fitted to 40
-// products of 20 to 1000 rows (within 10 %), against the fits above.  Not beyond one workgroup a CU; from 65
-// tiles on two or three shares gain nothing (512 x 4096 x 4096 28.0 us in one pass of 64 x 64 tiles).  Not beyond
-// the 32 MiB that callers without an allocator have.  A function of the shape, B's order and the operands' types
-// alone (the fits look at dense matrices, whatever the distance of the rows), so that the size asked for ahead of a call
-// is that of the call.
+// products of 20 to 1000 rows (within 10 %), against the fits above.  Not beyond one workgroup a CU, whose partial
+// sums are 16 MiB at most; from 65 tiles on two or three shares gain nothing (512 x 4096 x 4096 28.0 us in one pass of
+// 64 x 64 tiles).  Any count that leaves every share a slab, the last one fewer than the others.
+// A function of the shape, B's order and the operands' types alone (the fits look at dense matrices, whatever the
+// distance of the rows), so that the size asked for ahead of a call is that of the call.
 int small_tile_shares(const mi355_quant_dot_desc* d0)
 {
     if((d0->in_type != MI355_I8 && d0->in_type != MI355_FP8) || d0->batch != 1 || d0->trans_a || d0->m <= 0 ||
@@ -371,7 +371,7 @@ int small_tile_shares(const mi355_quant_dot_desc* d0)
     for(int s = 2; s * tiles <= 256 && s <= slabs / 2; s++)
     {
         const int per = (slabs + s - 1) / s;
-        if((slabs + per - 1) / per != s || (d.in_type == MI355_FP8 && d.k / 64 % s != 0) || small_tile_bytes(&d, s) > MI355_QUANT_DOT_STATIC_SCRATCH_BYTES)
+        if((slabs + per - 1) / per != s)
             continue;
         const double us = 5.6 + 0.011 * s * tiles + per * (0.6 + 0.0004 * s * tiles) + 0.38 * s * mb;
         if(shares == 1 || us < best)

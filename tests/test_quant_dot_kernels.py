@@ -4,7 +4,7 @@ import os
 import pytest
 
 from amdmigraphx_amd import capi
-from tests.quant_dot_kernel import kernel_of
+from tests.quant_dot_kernel import kernel_of, small_shares
 
 pytestmark = pytest.mark.skipif(not os.path.exists(capi.lib_path()), reason="library not built in this checkout")
 
@@ -70,6 +70,12 @@ def test_the_size_asked_for_serves_any_distance_of_the_rows(m, n, k, trans_b, fp
     for ldb in ((k if trans_b else n) + 1023) // 1024 * 1024, ((k if trans_b else n) + 1039) // 16 * 16:
         for lda in (k, k + 64):
             assert kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, lda=lda, ldb=ldb, workspace=need) == kernel
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 4096, 8128), (128, 4096, 14272), (64, 4096, 4288), (128, 2048, 8128), (32, 4096, 4160)])
+def test_fp8_shares_need_no_divisor_of_k(m, n, k):
+    """slabs of K are dealt to the shares in small tiles, whose last one may be the shorter, for either type"""
+    assert small_shares(m, n, k, fp8=True) == small_shares(m, n, k) > 1
 
 
 @pytest.mark.parametrize("m,n,k,trans_b,fp8", [(318, 1664, 12672, True, False), (750, 880, 12480, True, True),
