@@ -35,7 +35,9 @@ __global__ __launch_bounds__(512) void qgemm_shares_kernel(dma_params p, int per
     const int wave_m = wave >> 2, wave_n = wave & 3;
     const int i = lane & 15, g = lane >> 4;
 
-    // a contiguous run of (share, column) pairs per XCD, the row tiles that share a panel of B one after the other
+    // A contiguous run of (share, column) pairs per XCD, the row tiles that share a panel of B one after the other, where
+    // the workgroups are a multiple of 8; any other number is dealt in turn.  (xcd_run for those too: 70 products 0.83 to
+    // 1.06 of the time, 1.006 in the mean: these few workgroups share less than its divisions cost.)
     const int total = (int)gridDim.x;
     int v           = blockIdx.x;
     if(total % 8 == 0)
