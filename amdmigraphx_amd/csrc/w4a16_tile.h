@@ -415,9 +415,10 @@ bool tile_gemm_supported(const w4_params& p)
 // 64 rows per workgroup
 int launch_tile_gemm(const w4_params& p0, hipStream_t s)
 {
-    w4_params p       = p0;
-    const bool simple = p.zp_mode == MI355_W4_ZP_SCALAR && (p.group & 127) == 0;
-    dim3 grid((unsigned)((p.n + TL_BN - 1) / TL_BN), (unsigned)((p.m + 63) / 64));
+    constexpr int most = 65535 * 64; // rows of a launch: its grid has no more workgroups along y
+    w4_params p        = p0;
+    const bool simple  = p.zp_mode == MI355_W4_ZP_SCALAR && (p.group & 127) == 0;
+    dim3 grid((unsigned)((p.n + TL_BN - 1) / TL_BN));
     const int shares = tile_gemm_shares(p.m, p.n, p.k);
     float* room      = p0.partial;
     p.partial        = nullptr;
@@ -425,19 +426,26 @@ int launch_tile_gemm(const w4_params& p0, hipStream_t s)
     {
         const int nchunks  = (p.k + TL_CK - 1) / TL_CK;
         p.chunks_per_share = (nchunks + shares - 1) / shares;
-        p.partial          = room;
+        p.partial          = room; // (there are at most 128 tiles then: one launch)
         grid.z             = (unsigned)((nchunks + p.chunks_per_share - 1) / p.chunks_per_share);
     }
     // up to 48 rows a tile of 48: a quarter of the activations' way into the CU and of the products less
     const bool low = p.m <= 48;
-    if(simple && low)
-        hipLaunchKernelGGL((w4a16_tile_kernel<3, true>), grid, dim3(WL_THREADS), 0, s, p);
-    else if(simple)
-        hipLaunchKernelGGL((w4a16_tile_kernel<4, true>), grid, dim3(WL_THREADS), 0, s, p);
-    else if(low)
-        hipLaunchKernelGGL((w4a16_tile_kernel<3, false>), grid, dim3(WL_THREADS), 0, s, p);
-    else
-        hipLaunchKernelGGL((w4a16_tile_kernel<4, false>), grid, dim3(WL_THREADS), 0, s, p);
+    for(int64_t m0 = 0; m0 < p0.m; m0 += most)
+    {
+        p.a    = p0.a + m0 * p0.lda;
+        p.out  = p0.out + m0 * p0.ldc;
+        p.m    = (int)min((int64_t)most, p0.m - m0);
+        grid.y = (unsigned)((p.m + 63) / 64);
+        if(simple && low)
+            hipLaunchKernelGGL((w4a16_tile_kernel<3, true>), grid, dim3(WL_THREADS), 0, s, p);
+        else if(simple)
+            hipLaunchKernelGGL((w4a16_tile_kernel<4, true>), grid, dim3(WL_THREADS), 0, s, p);
+        else if(low)
+            hipLaunchKernelGGL((w4a16_tile_kernel<3, false>), grid, dim3(WL_THREADS), 0, s, p);
+        else
+            hipLaunchKernelGGL((w4a16_tile_kernel<4, false>), grid, dim3(WL_THREADS), 0, s, p);
+    }
     if(p.partial != nullptr)
         return launch_w4a16_reduce(p, (int)grid.z, s);
     return mi355_launch_status();

@@ -433,3 +433,24 @@ def test_w4a16_tile_kernel_of_a_part_of_its_columns(ops, m, n, k, g, zeros, room
     assert bool((out[:, n:] == -1).all())
     wdq = orc.dequantizelinear(wq, np.repeat(scales, g, axis=1), np.repeat(z, g, axis=1), orc.U8, orc.F16)
     _check(half_bits(out[:, :n].contiguous())[rows], want, a[rows], wdq)
+
+
+@pytest.mark.parametrize("n", [128, 144])
+def test_w4a16_rows_beyond_one_grid(ops, n):
+    """65535 tiles of 64 rows are the most of one launch: the rows behind them, and the last of the first launch"""
+    m, k, g = 65535 * 64 + 70, 128, 128
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    a = torch.randn(m, k, generator=gen, device="cuda", dtype=torch.float16)
+    w = torch.randint(0, 256, (n, k // 2), generator=gen, device="cuda", dtype=torch.uint8)
+    scales = (torch.rand(n, 1, generator=gen, device="cuda") * 0.02).half()
+    print("w4a16 rows", m, n, flush=True)
+    got = ops.w4a16_gemm(a, w, scales, g)
+    # weights in half as the kernel has them; sums in float, cut to half: 2^-10 of the value, 128 roundings of the sum
+    q = torch.stack([w & 15, w >> 4], dim=2).view(n, k).cpu().numpy()
+    half = orc.dequantizelinear(q, np.repeat(scales.cpu().numpy().view(np.uint16), g, axis=1), np.full((n, k), 8, dtype=np.uint8),
+                                orc.U8, orc.F16)
+    wd = torch.from_numpy(orc.half_to_f32(half)).cuda().double().t()
+    for first, last in ((0, 100), (65535 * 64 - 100, 65535 * 64), (65535 * 64 - 30, m), (m - 64, m)):
+        x = a[first:last].double()
+        bound = (x @ wd).abs() * 2.0**-10 + (x.abs() @ wd.abs()) * (128 * 2.0**-24) + 2.0**-24
+        assert bool(((got[first:last].double() - x @ wd).abs() <= bound).all()), (first, last)
