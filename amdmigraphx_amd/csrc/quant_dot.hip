@@ -347,7 +347,10 @@ size_t small_tile_bytes(const mi355_quant_dot_desc* d, int shares)
 // costs a workgroup alone on its CU, the partial sums' way, and a start that grows with the workgroups, fitted to 40
 // products of 20 to 1000 rows (within 10 %), against the fits above.  Not beyond one workgroup a CU, whose partial
 // sums are 16 MiB at most; from 65 tiles on two or three shares gain nothing (512 x 4096 x 4096 28.0 us in one pass of
-// 64 x 64 tiles).  Any count that leaves every share a slab, the last one fewer than the others.
+// 64 x 64 tiles).  Any count that leaves every share a slab, the last one fewer than the others; fp8 sums, whose bits
+// depend on the slices, keep equal ones as the 256 x 256 kernels cut them (a count that divides K / 64), or none,
+// unless that takes a third longer: 344 x 400 x 6016 in 2 16.4 us, in 8 13.1; 8 x 32 x 9664 (151 halves of a slab)
+// unsplit 30.5, in shares 7.0.
 // A function of the shape, B's order and the operands' types alone (the fits look at dense matrices, whatever the
 // distance of the rows), so that the size asked for ahead of a call is that of the call.
 int small_tile_shares(const mi355_quant_dot_desc* d0)
@@ -366,26 +369,36 @@ int small_tile_shares(const mi355_quant_dot_desc* d0)
         return 1;
     const int slabs = (int)((d.k + 127) / 128);
     const double mb = (double)d.m * (double)d.n * 4e-6;
-    double best     = 0;
-    int shares      = 1;
+    double any_us = 0, equal_us = 0;
+    int any = 1, equal = 1;
     for(int s = 2; s * tiles <= 256 && s <= slabs / 2; s++)
     {
         const int per = (slabs + s - 1) / s;
         if((slabs + per - 1) / per != s)
             continue;
         const double us = 5.6 + 0.011 * s * tiles + per * (0.6 + 0.0004 * s * tiles) + 0.38 * s * mb;
-        if(shares == 1 || us < best)
+        if(any == 1 || us < any_us)
         {
-            best   = us;
-            shares = s;
+            any_us = us;
+            any    = s;
+        }
+        if(d.k / 64 % s == 0 && (equal == 1 || us < equal_us))
+        {
+            equal_us = us;
+            equal    = s;
         }
     }
-    if(shares == 1)
+    if(any == 1)
         return 1;
     double other = dma_us(&d, mi355_dma_gemm_shares_with_room(&d), false);
     if(mi355_ragged_gemm_supported(&d))
         other = __builtin_fmin(other, ragged_us(&d));
-    return best < 0.9 * other ? shares : 1;
+    if(d.in_type == MI355_FP8 && any_us >= 0.75 * (equal > 1 ? __builtin_fmin(equal_us, other) : other))
+    {
+        any    = equal;
+        any_us = equal_us;
+    }
+    return any > 1 && any_us < 0.9 * other ? any : 1;
 }
 
 // the same for a call, whose workspace has to hold them

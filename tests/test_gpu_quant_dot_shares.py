@@ -16,13 +16,14 @@ def ops():
 
 # one row and one 16-column tile; tiles begun in both directions; K an odd number of 64 (a prime one, 8128); shares of
 # unequal length; the most tiles
-@pytest.mark.parametrize("m,n,k,trans_b", [(1, 16, 4160, False), (20, 512, 4096, True), (130, 144, 4160, False), (127, 129, 4160, True),
+@pytest.mark.parametrize("m,n,k,trans_b", [(1, 16, 4160, False), (1, 16, 8128, False), (20, 512, 4096, True), (130, 144, 4160, False), (127, 129, 4160, True),
                                            (257, 272, 4160, False), (33, 51, 4160, True), (40, 272, 8128, False), (128, 8192, 8256, False), (1000, 1008, 8256, False)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_against_the_product_in_double(ops, m, n, k, trans_b, fp8):
     need = ops.quant_dot_workspace_size(m, n, k, trans_b=trans_b, fp8=fp8)
     assert need > 0 and kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, workspace=need) == "dma_shares"
-    assert small_shares(m, n, k, trans_b=trans_b, fp8=fp8, workspace=need) > 1
+    # (fp8 of 1 x 16 x 4160 goes to equal slices in 256 x 256 tiles)
+    assert small_shares(m, n, k, trans_b=trans_b, fp8=fp8, workspace=need) > 1 or (fp8 and (m, n, k) == (1, 16, 4160))
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
 
     def codes(*shape):

@@ -72,10 +72,17 @@ def test_the_size_asked_for_serves_any_distance_of_the_rows(m, n, k, trans_b, fp
             assert kernel_of(m, n, k, trans_b=trans_b, fp8=fp8, lda=lda, ldb=ldb, workspace=need) == kernel
 
 
-@pytest.mark.parametrize("m,n,k", [(128, 4096, 8128), (128, 4096, 14272), (64, 4096, 4288), (128, 2048, 8128), (32, 4096, 4160)])
+@pytest.mark.parametrize("m,n,k", [(128, 4096, 8128), (128, 4096, 14272), (64, 4096, 4288), (128, 2048, 8128), (344, 400, 6016)])
 def test_fp8_shares_need_no_divisor_of_k(m, n, k):
     """slabs of K are dealt to the shares in small tiles, whose last one may be the shorter, for either type"""
     assert small_shares(m, n, k, fp8=True) == small_shares(m, n, k) > 1
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 256, 2112), (606, 288, 4160), (128, 4096, 8192)])
+def test_fp8_shares_are_equal_where_that_costs_little(m, n, k):
+    from amdmigraphx_amd import ops
+    shares = ops.quant_dot_workspace_size(m, n, k, fp8=True) // (4 * m * n)
+    assert shares > 1 and shares != small_shares(m, n, k) and k // 64 % shares == 0
 
 
 @pytest.mark.parametrize("m,n,k,trans_b,fp8", [(318, 1664, 12672, True, False), (750, 880, 12480, True, True),
