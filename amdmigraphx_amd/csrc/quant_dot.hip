@@ -689,9 +689,9 @@ extern "C" int mi355_quant_dot_ws(const mi355_quant_dot_desc* d,
                                               workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
-// The three below are not part of the public interface.  Tests ask the first, without a GPU, which kernel their
+// The four below are not part of the public interface.  Tests ask the first, without a GPU, which kernel their
 // shapes reach (the kernel_id, or the call's negative status), the second how many shares a workspace of those bytes
-// has in 128 x 128 tiles (1: none), and with the third run the edges of
+// has in 128 x 128 tiles (1: none), the third what 256 x 256 tiles would ask for, and with the fourth run the edges of
 // a kernel at sizes that the rules leave to another (the product, or MI355_ERR_UNSUPPORTED where the
 // kernel does not take it).
 extern "C" int mi355_internal_quant_dot_kernel(const mi355_quant_dot_desc* d,
@@ -717,6 +717,11 @@ extern "C" int mi355_internal_quant_dot_small_shares(const mi355_quant_dot_desc*
 {
     const int shares = small_tile_shares(d);
     return shares > 1 && small_tile_bytes(d, shares) <= workspace_bytes ? shares : 1;
+}
+
+extern "C" size_t mi355_internal_quant_dot_large_workspace(const mi355_quant_dot_desc* d)
+{
+    return mi355_dma_gemm_workspace(d);
 }
 
 extern "C" int mi355_internal_quant_dot_run(int32_t which,

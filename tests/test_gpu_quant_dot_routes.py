@@ -4,7 +4,7 @@ product in float64 (exact for int8; the fp8 sums are float).  Each test says whi
 import pytest
 import torch
 
-from tests.quant_dot_kernel import kernel_of
+from tests.quant_dot_kernel import Forced, kernel_of
 
 pytestmark = pytest.mark.gpu
 
@@ -100,7 +100,42 @@ def test_small_tiles(ops, batch, m, n, k, trans_b, fp8):
                                          (40, 33, 191, 128), (96, 197, 197, 64), (2, 70, 66, 129)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_one_slab(ops, batch, m, n, k, fp8):
-    # one instruction cuts each of up to 128 products 20 bits below the largest of them, which is at most the sum of
-    # the magnitudes: 2^-13 of that.  (Among the millions of sums of 96 x 197 x 197 some reach 2^-14, the same bits
-    # as the 256 x 256 kernels'.)
-    _check(ops, batch, m, n, k, True, fp8, cut=2.0**-13)
+    # (3 x 65 x 63 x 17 and the like are there for what lies beside the kernel: see below for the calls that reach it)
+    _check(ops, batch, m, n, k, True, fp8, cut=_cut(batch, m, n, k, fp8))
+
+
+def _cut(batch, m, n, k, fp8):
+    """One instruction cuts each of up to 128 products 20 bits below the largest of them, which is at most the sum of
+    the magnitudes: 2^-13 of that.  (Among the millions of sums of 96 x 197 x 197 some reach 2^-14, the same bits as
+    the 256 x 256 kernels'.)  The other kernels' sums keep the narrower bound, those in digits are exact."""
+    return 2.0**-13 if fp8 and "ragged" in _kernels(batch, m, n, k, True, fp8) else 2.0**-15
+
+
+# the kernel itself: int8 whatever K is, e4m3fn in float where rows are whole 16-byte pieces and N whole groups of 4
+@pytest.mark.parametrize("batch,m,n,k", [(20, 129, 132, 16), (9, 131, 192, 48), (5, 300, 500, 64), (9, 131, 188, 80),
+                                         (12, 197, 196, 112), (3, 70, 64, 128)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_one_slab_of_whole_pieces(ops, batch, m, n, k, fp8):
+    assert _kernels(batch, m, n, k, True, fp8) == {"ragged"}
+    _check(ops, batch, m, n, k, True, fp8, cut=_cut(batch, m, n, k, fp8))
+
+
+@pytest.mark.parametrize("batch,m,n,k", [(5, 300, 500, 17), (5, 300, 501, 33), (9, 131, 190, 63), (5, 300, 499, 65),
+                                         (12, 197, 197, 111), (2, 130, 70, 127)])
+def test_one_slab_of_any_bytes(ops, batch, m, n, k):
+    assert _kernels(batch, m, n, k, True, False) == {"ragged_exact"}
+    _check(ops, batch, m, n, k, True, False)
+
+
+@pytest.mark.parametrize("batch,m,n,k", [(96, 197, 197, 64), (3, 300, 260, 128), (1, 500, 1030, 128)])
+@pytest.mark.parametrize("out", [None, torch.float32, torch.bfloat16])
+def test_one_slab_gives_the_bits_of_the_large_tiles(ops, monkeypatch, batch, m, n, k, out):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, b = (_codes(g, (batch, rows, k), True).view(torch.uint8) for rows in (m, n))
+    kw = dict(fp8=True, out_dtype=out, **(dict(scale_a=torch.rand(1, generator=g, device="cuda")) if out else {}))
+    assert kernel_of(m, n, k, trans_b=True, fp8=True, batch=batch, out="f32" if out else None) == "ragged"
+    got = ops.quant_dot(a, b.transpose(1, 2), **kw)
+    large = Forced("dma")
+    monkeypatch.setattr(ops, "lib", lambda: large)
+    want = ops.quant_dot(a, b.transpose(1, 2), **kw)
+    assert large.taken == 1 and torch.equal(got, want)

@@ -15,9 +15,11 @@ def ops():
     return ops
 
 
-# rows and columns that fill no 256 x 256 tile, K of 12 * 4 slabs, one more trip of slabs and a remainder
+# rows and columns that fill no 256 x 256 tile, K of 12 * 4 slabs, one more trip of slabs and a remainder; N no
+# multiple of 128: 16, 144 and 240 columns of the last tile, one part of K and four
 @pytest.mark.parametrize("m,n,k,pad", [(1999, 7296, 1536, 0), (970, 15744, 1664, 8), (2048, 8192, 2688, 0),
-                                       (1000, 3968, 9216, 8)])
+                                       (1000, 3968, 9216, 8), (1999, 7184, 1536, 8), (970, 15760, 1664, 0),
+                                       (512, 4112, 8192, 8), (700, 4080, 8192, 0)])
 @pytest.mark.parametrize("group,zeros", [(128, "scalar"), (64, "group"), (32, "packed")])
 def test_many_rows(ops, m, n, k, pad, group, zeros):
     need = ops.w4a16_gemm_workspace_size(m, n, k, group)
