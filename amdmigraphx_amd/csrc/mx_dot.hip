@@ -292,10 +292,11 @@ __global__ __launch_bounds__(256) void mx_gemm_kernel(mx_params p)
 // lines: a wave that read its own scales touched 64 lines a slab for 2 KiB of them, twice what the
 // operands take.  The scales of four slabs are now fetched together, a line a row, once for the workgroup, and
 // staged as exponent bytes.
-// Measured, all launches of a call, fp4 / fp8, 256 x 256 kernels -> scales by the wave -> staged: 512 x 4096 x 4096
-// 40.0 -> 27.6 -> 19.7 / 59.5 -> 43.5 -> 29.8 us, 16 x 4096 x 4096 35.6 -> 13.2 -> 11.9 / 51.2 -> 17.9 -> 18.4, 128 x 4096 x 14336
-// 101 -> 41 -> 34 / 154 -> 71 -> 56.  (Slabs of 256 bytes need more
-// registers than two workgroups on a CU have and spill; 128 x 128 tiles as well.)
+// Measured, all launches of a call over operands in the caches, fp4 / fp8, 256 x 256 kernels -> scales by the wave ->
+// staged: 512 x 4096 x 4096 40.0 -> 27.8 -> 19.8 / 59.5 -> 44.8 -> 29.9 us, 16 x 4096 x 4096 35.6 -> 13.5 -> 12.2 /
+// 51.2 -> 18.0 -> 18.6, 128 x 4096 x 14336 101 -> 40 -> 32 / 154 -> 71 -> 55; over weights from memory the last two
+// 14.0 -> 12.2 / 22.7 -> 21.1 and 47 -> 36 / 85 -> 61 (and none of 60 fp8 products of up to 300 tiles slower).
+// (Slabs of 256 bytes need more registers than two workgroups on a CU have and spill; 128 x 128 tiles as well.)
 //
 // Both operands have one type, K bytes are K / 2 (fp4) or K (fp8).  The product does not care which K
 // positions meet as long as A and B agree, so the blocks of a slab are dealt to the instruction's
@@ -547,9 +548,10 @@ int64_t mx_small_tiles(const mx_params& p, int64_t batch)
     return batch * ((p.m + 63) / 64) * ((p.n + 63) / 64);
 }
 
-// Up to four workgroups a CU, where the small tiles are the faster ones at any K from 128 to 14336 (the 256 x 256
+// Up to 1024 tiles, where the small ones are the faster ones at any K from 128 to 14336 (the 256 x 256
 // kernels' whole call against theirs, fp4 / fp8: 1024 x 4096 with K = 1024 20.9 -> 13.2 / 27.2 -> 17.1 us, 14336
-// 104.6 -> 81.9 / 159.4 -> 138.7; 16 x 65536 x 512 16.4 -> 9.1 / 22.9 -> 12.2).  At 1280 tiles fp8 of a long K loses
+// 104.6 -> 81.9 / 159.4 -> 138.7; 16 x 65536 x 512 16.4 -> 9.1 / 22.9 -> 12.2).  Three share a CU (155 to 168
+// registers, 41 to 46 KiB of LDS), so that 768 run at once and the others behind them.  At 1280 fp8 of a long K loses
 // (160 -> 177).  One type, scales of one float per block side by side, whole runs of 4 blocks.
 bool mx_tiles_pay(const mx_params& p, int64_t batch)
 {

@@ -20,7 +20,7 @@
 // code has no digits: rows of A and columns of B that hold one are noted while they are loaded.
 //
 // What bounds it: 500 x 30522 x 768 int8 -> float is 1810 us in the scalar kernel and 38 us here, of which
-// the 61 MB of C are 12 us at this card's copy rate: matrix cores are busy 13 % of it, a fifth of the waves' time
+// the 61 MB of C are 12 us at this card's copy rate: matrix cores are busy 15 % of it, a quarter of the waves' time
 // is vector work (the transposition of B, for every 128 rows of A again), a quarter waits.  A tile's 128 columns
 // of an unaligned row lie in two lines; while the four tiles that share them ran on different XCDs (956 tiles, no
 // multiple of 8, dealt in turn) B came in eight times from behind the L2s and the call took 46 us.
