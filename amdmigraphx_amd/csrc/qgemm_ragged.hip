@@ -563,10 +563,17 @@ __global__ __launch_bounds__(THREADS) void qgemm_ragged_kernel(ragged_params p)
         }
 }
 
-// B as [N, K], K in one slab of 128 at most; a grid holds less than 2^32 threads along x
-bool one_slab(bool trans_b, int64_t m, int64_t n, int64_t k)
+// B as [N, K], K in one slab of 128 at most, in 64 x 64 tiles; a grid holds less than 2^32 threads along x.  Up to 16384
+// of them (bare results: 4096) the slab is the faster one nearly everywhere (1370 random products of both types: at
+// most 1.06 of what the call took before, 0.86 in the mean): 96 x 197 x 197 x 64 int8 11.3 -> 9.3 us, 104 x 475 x 475 x 64
+// 36.4 -> 27.4, 64 x 1000 x 1000 x 64 67 -> 48 (all to float32).  Beyond, the memory's writes bound both, and tiles of
+// 128 x 128 read half as much: 11707 x 16424 x 128 fp8 bare 241 us against 278, 10874 x 13531 x 32 int8 230 against 266;
+// the slab stays where those would be padding for two fifths and more (1910 x 828 x 64 x 114 243 -> 139).
+bool one_slab(bool trans_b, bool bare, int64_t batch, int64_t m, int64_t n, int64_t k)
 {
-    return trans_b && k <= 128 && ((m + 63) / 64) * ((n + 63) / 64) < ((int64_t)1 << 32) / THREADS;
+    const int64_t tiles = ((m + 63) / 64) * ((n + 63) / 64), big = ((m + 127) / 128) * ((n + 127) / 128);
+    return trans_b && k <= 128 && tiles < ((int64_t)1 << 32) / THREADS &&
+           (batch * tiles <= (bare ? 4096 : 16384) || 20 * big >= 7 * tiles);
 }
 
 template <int FORM, bool TRANS_B, int OUT, bool BIG, int ONE = 0>
@@ -583,11 +590,9 @@ int launch_tile(ragged_params& p, int batch, hipStream_t s)
 template <int FORM, bool TRANS_B, int OUT>
 int launch_out(ragged_params& p, int batch, hipStream_t s)
 {
-    // K in one slab, whatever the size: 96 x 197 x 197 x 64 int8 11.3 -> 9.3 us, 104 x 475 x 475 x 64 36.4 -> 27.4,
-    // 64 x 1000 x 1000 x 64 67 -> 48, 2048 x 30000 x 128 57.9 -> 44.9 (all to float32)
     if constexpr(TRANS_B && FORM != FP8_DIGITS)
     {
-        if(one_slab(TRANS_B, p.m, p.n, p.k))
+        if(one_slab(TRANS_B, OUT == -1, batch, p.m, p.n, p.k))
         {
             if constexpr(FORM == INT8)
             {
@@ -653,7 +658,10 @@ bool mi355_ragged_gemm_supported(const mi355_quant_dot_desc* d)
 }
 
 // not for the exact sums of e4m3fn
-bool mi355_ragged_gemm_one_slab(const mi355_quant_dot_desc* d) { return one_slab(d->trans_b, d->m, d->n, d->k); }
+bool mi355_ragged_gemm_one_slab(const mi355_quant_dot_desc* d)
+{
+    return one_slab(d->trans_b, !d->dequant, d->batch, d->m, d->n, d->k);
+}
 
 int mi355_ragged_gemm_launch(const mi355_quant_dot_desc* d,
                              const void* a,

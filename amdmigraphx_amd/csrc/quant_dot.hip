@@ -248,13 +248,10 @@ double part(int64_t dim, double side) { return __builtin_fmin((double)dim, side)
 //   1024 x 1024 x 1024 int8 -> bfloat16          23.5 -> 6.5         512 x 4096 x 4096 (split)   30.9 -> 21.3
 //   48 x 1024 x 1024 x 128                       49.8 against 53.7 (stays)
 // It never splits K: few tiles of a long K stay with shares (5 x 192 x 25472 int8: 79.9 against 16.4 us).
-double ragged_us(const mi355_quant_dot_desc* d)
+double two_slab_us(const mi355_quant_dot_desc* d)
 {
     const int deq = d->dequant != 0, tb = d->trans_b != 0;
     const double k = (double)d->k;
-    // K in one slab: by the tile, for 64 to 16384 of them and every type of result (int8 and fp8 within 10 %)
-    if(mi355_ragged_gemm_one_slab(d))
-        return 4.6 + tiles_of(d, 64) * (d->k <= 64 ? 0.0029 : 0.0037);
     // (the kernel's own choice of the tile; two of the large ones share a CU)
     if(const double big = tiles_of(d, 128); big >= 256)
     {
@@ -276,6 +273,20 @@ double ragged_us(const mi355_quant_dot_desc* d)
     f.b_mb             = tb ? 0.080 : fill > 1.0 ? 0.170 : 0.100;
     const double first = tb ? 0.0020 : pitched ? 0.0036 : 0.0030;
     return fitted_us(f, d, fill, part(d->m, 64.0), k) + (first - f.k_wave) * k;
+}
+
+// The same kernel with K in one slab where it has one: a start, the tiles, the results, and what of those no cache
+// takes (750 random products of up to 128 of K: nine in ten take 0.85 to 1.3 times that).  It is hardly ever the
+// slower one, so what two slabs would win stays won.
+double ragged_us(const mi355_quant_dot_desc* d)
+{
+    const double two = two_slab_us(d);
+    if(!mi355_ragged_gemm_one_slab(d))
+        return two;
+    const double out = (double)d->batch * (double)d->m * (double)d->n * 1e-6;
+    const double mb  = out * (d->dequant && d->out_type != MI355_F32 ? 2.0 : 4.0);
+    return __builtin_fmin(two, (d->dequant ? 3.8 : 3.0) + 0.0016 * tiles_of(d, 64) + 0.25 * out +
+                                   (mb > 200.0 ? 0.17 * (mb - 200.0) : 0.0));
 }
 
 // direct-to-LDS kernels; `shares` of K through a workspace, or added into C

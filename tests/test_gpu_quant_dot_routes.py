@@ -127,6 +127,13 @@ def test_one_slab_of_any_bytes(ops, batch, m, n, k):
     _check(ops, batch, m, n, k, True, False)
 
 
+# more tiles than the one-slab kernel takes (of bare results, of any), and so many that are mostly padding otherwise
+@pytest.mark.parametrize("batch,m,n,k", [(1, 4200, 4304, 80), (1, 8200, 8208, 48), (300, 64, 1000, 64), (2, 2900, 2880, 128)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_short_k_of_many_tiles(ops, batch, m, n, k, fp8):
+    _check(ops, batch, m, n, k, True, fp8, cut=_cut(batch, m, n, k, fp8))
+
+
 @pytest.mark.parametrize("batch,m,n,k", [(96, 197, 197, 64), (3, 300, 260, 128), (1, 500, 1030, 128)])
 @pytest.mark.parametrize("out", [None, torch.float32, torch.bfloat16])
 def test_one_slab_gives_the_bits_of_the_large_tiles(ops, monkeypatch, batch, m, n, k, out):

@@ -98,6 +98,15 @@ def test_the_static_entry_refuses_by_the_large_tiles(m, n, k, trans_b, fp8):
     assert (ops.quant_dot_workspace_size(m, n, k, trans_b=trans_b, fp8=fp8) > 32 << 20) == (m == 255)
 
 
+@pytest.mark.parametrize("batch,m,n,k,fp8,out", [
+    (1, 10, 58608, 128, False, None), (1, 1, 2896, 16, True, None), (1, 8, 4996, 32, True, None), (3, 26, 16, 16, True, None),
+    (1, 2, 23956, 32, True, "f32"), (18, 282, 16, 64, True, None), (1, 26278, 16, 64, True, None), (477, 18, 236, 32, True, "f32")])
+def test_one_slab_of_few_rows(batch, m, n, k, fp8, out):
+    """Measured, one slab against the kernel of 256 x 256 tiles that a fit without the small start of bare results had
+    chosen: 3.7 / 7.4 us, 2.8 / 5.1, 3.0 / 5.3, 3.0 / 5.0, 3.4 / 5.7, 3.3 / 4.8, 3.6 / 5.0, 8.0 / 12.4."""
+    assert kernel_of(m, n, k, trans_b=True, fp8=fp8, out=out, batch=batch) == "ragged"
+
+
 def test_large_and_small_grids():
     for fp8 in (False, True):
         for out in (None, "bf16", "f32"):
