@@ -21,6 +21,16 @@ MI355_DEVINL int xcd_run(int wg, int total)
     return x * (total / 8) + (x < more ? x : more) + wg / 8;
 }
 
+// The same where it pays.  A run meets its panels of B in one L2; with a number that is no multiple of 8 it also ends
+// in the middle of them, and the XCDs write far from each other.  Measured over 2000 products (tiles dealt in turn ->
+// runs): wide results of K beyond 128 0.95 of the time in the register-staged kernel (500 x 30522 x 768 45.8 -> 37.8 us)
+// and 0.98 in up to 1024 tiles of 256 x 256 (3351 x 26672 x 384 fp8 bare has 1470: 128 -> 144), a few up to 1.08; tall
+// or square ones and short K 1.00, up to 1.22 (11728 x 288 x 1344 fp8 20.4 -> 23.5, 6799 x 23152 x 64 140 -> 171).
+MI355_DEVINL int xcd_place(int wg, int total, int tiles_m, int tiles_n, int k, int most)
+{
+    return total % 8 == 0 || (k > 128 && tiles_n >= 2 * tiles_m && total <= most) ? xcd_run(wg, total) : wg;
+}
+
 static inline int mi355_launch_status()
 {
     return hipGetLastError() == hipSuccess ? MI355_OK : MI355_ERR_LAUNCH;

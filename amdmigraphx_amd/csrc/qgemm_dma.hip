@@ -123,13 +123,13 @@ MI355_DEVINL v2i read_tr8(const uint8_t* l)
 }
 
 // XCD-aware tile order.  Workgroup ids are dealt round-robin to the 8 XCDs,
-// each with its own L2.  Give every XCD a contiguous run of the tile order, and
+// each with its own L2.  Give every XCD a contiguous run of the tile order (xcd_place says where), and
 // walk that order in column-major bands of 8 tile rows, so the ~32 tiles an
 // XCD works on at one time share A row panels and B column panels in its L2.
-MI355_DEVINL void tile_coords(int wg, int tiles_m, int tiles_n, int& tm, int& tn)
+MI355_DEVINL void tile_coords(int wg, int tiles_m, int tiles_n, int k, int& tm, int& tn)
 {
     const int total = tiles_m * tiles_n;
-    const int v     = xcd_run(wg, total);
+    const int v     = xcd_place(wg, total, tiles_m, tiles_n, k, 1024);
     constexpr int band = 8;
     int per_band       = band * tiles_n;
     int b              = v / per_band;
@@ -233,7 +233,7 @@ __global__ __launch_bounds__(NTHREADS) void qgemm_dma_kernel(dma_params p)
     const int wave_n = wave & 3;  // 0..3
 
     int tm, tn;
-    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, p.k, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * BN;
 
@@ -928,7 +928,7 @@ __global__ __launch_bounds__(NTHREADS) void qgemm_dma_i8_kernel(dma_params p)
     const int wave_n = wave & 3;  // 0..3
 
     int tm, tn;
-    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, p.k, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * BN;
 
@@ -1476,7 +1476,7 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_i8_kernel(dma_params p)
     const int wave_n = wave & 1;  // 0..1
 
     int tm, tn;
-    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, p.k, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * BN;
 
@@ -2474,7 +2474,7 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_f8_kernel(dma_params p)
     const int wave_n = wave & 1;  // 0..1
 
     int tm, tn;
-    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, p.k, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * BN;
 
@@ -3303,7 +3303,7 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_mx4_kernel(dma_params p)
     const int wave_n = wave & 1;  // 0..1
 
     int tm, tn;
-    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, p.k, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * BN;
 
@@ -3870,7 +3870,7 @@ __global__ __launch_bounds__(W4_THREADS) void qgemm_w4_mx8_kernel(dma_params p)
     const int wave_n = wave & 1;  // 0..1
 
     int tm, tn;
-    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, p.k, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * BN;
 

@@ -76,10 +76,10 @@ MI355_DEVINL void transpose4x4(uint32_t r0, uint32_t r1, uint32_t r2, uint32_t r
 // each with its own L2.  Give every XCD a contiguous run of the tile order, and
 // walk that order in column-major bands of 8 tile rows, so the ~32 tiles an
 // XCD works on at one time share A row panels and B column panels in its L2.
-MI355_DEVINL void tile_coords(int wg, int tiles_m, int tiles_n, int& tm, int& tn)
+MI355_DEVINL void tile_coords(int wg, int tiles_m, int tiles_n, int k, int& tm, int& tn)
 {
     const int total = tiles_m * tiles_n;
-    const int v     = xcd_run(wg, total);
+    const int v     = xcd_place(wg, total, tiles_m, tiles_n, k, 1024);
     constexpr int band = 8;
     int per_band       = band * tiles_n;
     int b              = v / per_band;
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(NTHREADS) void qgemm_mfma_kernel(gemm_params p)
     const int wave_n = wave & 3;  // 0..3
 
     int tm, tn;
-    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, p.k, tm, tn);
     const int m0 = tm * BM;
     const int n0 = tn * BN;
 

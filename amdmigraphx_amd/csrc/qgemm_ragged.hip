@@ -210,7 +210,9 @@ __global__ __launch_bounds__(THREADS) void qgemm_ragged_kernel(ragged_params p)
 
     // a contiguous run of tiles per XCD (workgroups are dealt to the 8 of them in turn), rows first: the
     // tiles that share a panel of B follow each other in one L2
-    const int v  = xcd_run(blockIdx.x, p.tiles_m * p.tiles_n);
+    const int total = p.tiles_m * p.tiles_n;
+    // (one slab: runs everywhere; in turn 1.01 of their time over 350 products, up to 1.14)
+    const int v     = ONE != 0 ? xcd_run(blockIdx.x, total) : xcd_place(blockIdx.x, total, p.tiles_m, p.tiles_n, p.k, total);
     const int m0 = (v % p.tiles_m) * BT;
     const int n0 = (v / p.tiles_m) * BT;
 
