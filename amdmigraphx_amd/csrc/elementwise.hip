@@ -796,6 +796,46 @@ __global__ __launch_bounds__(256) void gather_wide_rows_kernel(
     }
 }
 
+// The product as [rows, cols]: leading dimensions merge into one row index when, for both operands, each stride
+// continues the next one (or both are broadcast there); with `join`, dimensions that continue the columns in
+// both operands are columns too.  False where that leaves dimensions, or columns that are no whole aligned vectors.
+bool rows_and_cols(const bcast_params& p, bool join, binary2d_params& q)
+{
+    int last = p.ndim - 1;
+    while(last > 0 && p.lens[last] == 1)
+        last--;
+    int64_t cols       = p.lens[last];
+    const int64_t a_sc = cols == 1 ? 0 : p.a_strides[last];
+    const int64_t b_sc = cols == 1 ? 0 : p.b_strides[last];
+    while(join && last > 0 && cols > 1 && cols * p.lens[last - 1] <= (1 << 30) &&
+          (p.lens[last - 1] == 1 || (p.a_strides[last - 1] == a_sc * cols && p.b_strides[last - 1] == b_sc * cols)))
+    {
+        last--;
+        cols *= p.lens[last];
+    }
+    int64_t rows = 1, a_sr = 0, b_sr = 0;
+    bool first = true;
+    for(int d = last - 1; d >= 0; d--)
+    {
+        if(p.lens[d] == 1)
+            continue;
+        if(first)
+        {
+            a_sr  = p.a_strides[d];
+            b_sr  = p.b_strides[d];
+            first = false;
+        }
+        else if(p.a_strides[d] != a_sr * rows || p.b_strides[d] != b_sr * rows)
+            return false;
+        rows *= p.lens[d];
+    }
+    auto vec_ok = [](const float* x, int64_t sr, int64_t sc) {
+        return sc == 0 || (sc == 1 && sr % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0);
+    };
+    q = binary2d_params{p.a, p.b, p.out, rows, cols, a_sr, b_sr, (int)a_sc, (int)b_sc, p.op};
+    return cols % 4 == 0 && reinterpret_cast<uintptr_t>(p.out) % 16 == 0 && vec_ok(p.a, a_sr, a_sc) && vec_ok(p.b, b_sr, b_sc);
+}
+
 unsigned blocks_for_n(int64_t n)
 {
     int64_t b = (n + 255) / 256;
@@ -837,58 +877,18 @@ extern "C" int mi355_binary_f32(int32_t op,
     p.out  = out;
     p.ndim = ndim;
     p.op   = op;
-    // collapse to [rows, cols]: leading dimensions merge into one row index when, for both
-    // operands, each stride continues the next one (or both are broadcast there)
+    // A position table [384, 768] added to [32, 384, 768] is 32 rows of 294912 (35 -> 14 us; element by element with
+    // divisions before).  Dimensions that join the columns leave fewer and longer rows; where they alone make rows
+    // of the product, those are worth a workgroup each from 128 columns on (10^6 elements in rows of 8 / 64 / 128 /
+    // 1024: 30.3 / 9.0 / 5.8 / 3.4 us, element by element 6.9).
+    binary2d_params q{}, plain{};
+    if(rows_and_cols(p, true, q) && (q.cols >= 128 || rows_and_cols(p, false, plain)))
     {
-        int last = ndim - 1;
-        while(last > 0 && lens[last] == 1)
-            last--;
-        int64_t cols       = lens[last];
-        const int64_t a_sc = cols == 1 ? 0 : a_strides[last];
-        const int64_t b_sc = cols == 1 ? 0 : b_strides[last];
-        // dimensions that continue the columns in both operands are columns too: a position table [384, 768]
-        // added to [32, 384, 768] is 32 rows of 294912 (35 -> 14 us; element by element with divisions before)
-        while(last > 0 && cols > 1 && cols * lens[last - 1] <= (1 << 30) &&
-              (lens[last - 1] == 1 || (a_strides[last - 1] == a_sc * cols && b_strides[last - 1] == b_sc * cols)))
-        {
-            last--;
-            cols *= lens[last];
-        }
-        int64_t rows = 1;
-        int64_t a_sr = 0, b_sr = 0;
-        bool ok      = true;
-        bool first   = true;
-        for(int d = last - 1; d >= 0 && ok; d--)
-        {
-            if(lens[d] == 1)
-                continue;
-            if(first)
-            {
-                a_sr  = a_strides[d];
-                b_sr  = b_strides[d];
-                first = false;
-            }
-            else
-            {
-                ok = a_strides[d] == a_sr * rows && b_strides[d] == b_sr * rows;
-            }
-            rows *= lens[d];
-        }
-        auto vec_ok        = [&](const float* q, int64_t sr, int64_t sc) {
-            if(sc == 0)
-                return true;
-            return sc == 1 && sr % 4 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0;
-        };
-        if(ok && cols % 4 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 && vec_ok(a, a_sr, a_sc) &&
-           vec_ok(b, b_sr, b_sc))
-        {
-            binary2d_params q{a, b, out, rows, cols, a_sr, b_sr, (int)a_sc, (int)b_sc, op};
-            const int64_t gx = (cols / 4 + 255) / 256;
-            const int64_t gy = rows < 65535 ? rows : 65535;
-            hipLaunchKernelGGL(binary2d_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0,
-                               static_cast<hipStream_t>(stream), q);
-            return mi355_launch_status();
-        }
+        const int64_t gx = (q.cols / 4 + 255) / 256;
+        const int64_t gy = q.rows < 65535 ? q.rows : 65535;
+        hipLaunchKernelGGL(binary2d_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0,
+                           static_cast<hipStream_t>(stream), q);
+        return mi355_launch_status();
     }
     hipLaunchKernelGGL(binary_kernel, dim3(blocks_for_n(p.total)), dim3(256), 0,
                        static_cast<hipStream_t>(stream), p);
