@@ -764,9 +764,10 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(
 // of W words a lane of one row, so that many rows and few long ones both spread over the chip.  Rows that are
 // whole 16-byte pieces move in those.  Word by word, a wave a row, now: one row of 112163 words 2.5, 183, 2.7 us, 137 of
 // 363319 152, 2429, 82; 12491 of 755 19.4 word by word, 14.7 now (calls in a graph).
+// (61 of 1644: 2.5 word by word, 2.8 with four pieces a lane, 2.5 with one, which few rows take)
 constexpr int GATHER_TURNS = 4;
 
-template <class I, int W>
+template <class I, int W, int TURNS>
 __global__ __launch_bounds__(256) void gather_wide_rows_kernel(
     const uint32_t* table, const I* ids, uint32_t* out, uint32_t units, uint32_t units_of_row, int64_t table_rows, int64_t row_words)
 {
@@ -783,14 +784,14 @@ __global__ __launch_bounds__(256) void gather_wide_rows_kernel(
             id = 0;
         const piece* src = reinterpret_cast<const piece*>(table + id * row_words);
         piece* dst       = reinterpret_cast<piece*>(out + (int64_t)r * row_words);
-        const int64_t c  = (int64_t)(u - r * units_of_row) * (64 * GATHER_TURNS) + lane;
-        piece v[GATHER_TURNS];
+        const int64_t c  = (int64_t)(u - r * units_of_row) * (64 * TURNS) + lane;
+        piece v[TURNS];
 #pragma unroll
-        for(int t = 0; t < GATHER_TURNS; t++)
+        for(int t = 0; t < TURNS; t++)
             if(c + 64 * t < pieces)
                 v[t] = src[c + 64 * t];
 #pragma unroll
-        for(int t = 0; t < GATHER_TURNS; t++)
+        for(int t = 0; t < TURNS; t++)
             if(c + 64 * t < pieces)
                 dst[c + 64 * t] = v[t];
     }
@@ -1315,15 +1316,20 @@ extern "C" int mi355_softmax_f32(const float* in, float* out, int64_t rows, int6
 }
 
 namespace {
-template <class I, int W>
+template <class I, int W, int TURNS = GATHER_TURNS>
 void launch_gather_wide_rows(const uint32_t* table, const I* ids, uint32_t* out, int64_t n_ids, int64_t table_rows,
                              int64_t words, hipStream_t s)
 {
     // a unit is 256 bytes of the result at least, so that their number fits 32 bits with any memory
-    const int64_t of_row = (words / W + 64 * GATHER_TURNS - 1) / (64 * GATHER_TURNS);
+    const int64_t of_row = (words / W + 64 * TURNS - 1) / (64 * TURNS);
     const int64_t units  = n_ids * of_row;
-    hipLaunchKernelGGL((gather_wide_rows_kernel<I, W>), dim3((unsigned)std::min<int64_t>((units + 3) / 4, 4096)), dim3(256), 0,
-                       s, table, ids, out, (uint32_t)units, (uint32_t)of_row, table_rows, words);
+    if constexpr(TURNS > 1)
+    {
+        if(units < 1024)
+            return launch_gather_wide_rows<I, W, 1>(table, ids, out, n_ids, table_rows, words, s);
+    }
+    hipLaunchKernelGGL((gather_wide_rows_kernel<I, W, TURNS>), dim3((unsigned)std::min<int64_t>((units + 3) / 4, 4096)),
+                       dim3(256), 0, s, table, ids, out, (uint32_t)units, (uint32_t)of_row, table_rows, words);
 }
 
 template <class I>
