@@ -565,17 +565,19 @@ __global__ __launch_bounds__(THREADS) void qgemm_ragged_kernel(ragged_params p)
         }
 }
 
-// B as [N, K], K in one slab of 128 at most, in 64 x 64 tiles; a grid holds less than 2^32 threads along x.  Up to 16384
-// of them (bare results: 4096) the slab is the faster one nearly everywhere (1370 random products of both types: at
-// most 1.06 of what the call took before, 0.86 in the mean): 96 x 197 x 197 x 64 int8 11.3 -> 9.3 us, 104 x 475 x 475 x 64
-// 36.4 -> 27.4, 64 x 1000 x 1000 x 64 67 -> 48 (all to float32).  Beyond, the memory's writes bound both, and tiles of
-// 128 x 128 read half as much: 11707 x 16424 x 128 fp8 bare 241 us against 278, 10874 x 13531 x 32 int8 230 against 266;
-// the slab stays where those would be padding for two fifths and more (1910 x 828 x 64 x 114 243 -> 139).
-bool one_slab(bool trans_b, bool bare, int64_t batch, int64_t m, int64_t n, int64_t k)
+// B as [N, K], K in one slab of 128 at most, in 64 x 64 tiles; a grid holds less than 2^32 threads along x.  The slab is
+// the faster one while the result stays within 1.4 times the last-level cache (1360 random products of both types:
+// 0.80 of the two-slab tiles' time): 96 x 197 x 197 x 64 int8 11.3 -> 9.3 us, 104 x 475 x 475 x 64 36.4 -> 27.4, 64 x 1000 x
+// 1000 x 64 67 -> 48 (all to float32).  Larger ones leave at the memory's rate, which rows that end inside a line of
+// 128 bytes hold up, less so from tiles of 128 x 128: 11707 x 16424 x 128 fp8 bare 241 us against 278, 10874 x 13531 x 32
+// int8 230 against 266.  The slab stays where those would be padding for a third and more (1910 x 828 x 64 x 114
+// 243 -> 139), and for scaled results of many matrices (312 x 975 x 975 x 64 fp8 to half 359 -> 302).
+bool one_slab(bool trans_b, int64_t batch, int64_t m, int64_t n, int64_t k, int64_t elem_bytes, bool scaled)
 {
     const int64_t tiles = ((m + 63) / 64) * ((n + 63) / 64), big = ((m + 127) / 128) * ((n + 127) / 128);
     return trans_b && k <= 128 && tiles < ((int64_t)1 << 32) / THREADS &&
-           (batch * tiles <= (bare ? 4096 : 16384) || 20 * big >= 7 * tiles);
+           (batch * m * n * elem_bytes <= 350000000 || n * elem_bytes % 128 == 0 || 8 * big >= 3 * tiles ||
+            (scaled && batch > 1));
 }
 
 template <int FORM, bool TRANS_B, int OUT, bool BIG, int ONE = 0>
@@ -594,7 +596,7 @@ int launch_out(ragged_params& p, int batch, hipStream_t s)
 {
     if constexpr(TRANS_B && FORM != FP8_DIGITS)
     {
-        if(one_slab(TRANS_B, OUT == -1, batch, p.m, p.n, p.k))
+        if(one_slab(TRANS_B, batch, p.m, p.n, p.k, OUT == MI355_F16 || OUT == MI355_BF16 ? 2 : 4, OUT != -1))
         {
             if constexpr(FORM == INT8)
             {
@@ -662,7 +664,8 @@ bool mi355_ragged_gemm_supported(const mi355_quant_dot_desc* d)
 // not for the exact sums of e4m3fn
 bool mi355_ragged_gemm_one_slab(const mi355_quant_dot_desc* d)
 {
-    return one_slab(d->trans_b, !d->dequant, d->batch, d->m, d->n, d->k);
+    return one_slab(d->trans_b, d->batch, d->m, d->n, d->k, d->dequant ? (int64_t)mi355_dtype_size(d->out_type) : 4,
+                    d->dequant != 0);
 }
 
 int mi355_ragged_gemm_launch(const mi355_quant_dot_desc* d,

@@ -276,17 +276,20 @@ double two_slab_us(const mi355_quant_dot_desc* d)
 }
 
 // The same kernel with K in one slab where it has one: a start, the tiles, the results, and what of those no cache
-// takes (750 random products of up to 128 of K: nine in ten take 0.85 to 1.3 times that).  It is hardly ever the
-// slower one, so what two slabs would win stays won.
+// takes; many tiles of bare results take longer (1300 random products of up to 128 of K: nine in ten take 0.85 to 1.25
+// times that).  It is hardly ever the slower one, so what two slabs would win stays won.
 double ragged_us(const mi355_quant_dot_desc* d)
 {
     const double two = two_slab_us(d);
     if(!mi355_ragged_gemm_one_slab(d))
         return two;
-    const double out = (double)d->batch * (double)d->m * (double)d->n * 1e-6;
-    const double mb  = out * (d->dequant && d->out_type != MI355_F32 ? 2.0 : 4.0);
-    return __builtin_fmin(two, (d->dequant ? 3.8 : 3.0) + 0.0016 * tiles_of(d, 64) + 0.25 * out +
-                                   (mb > 200.0 ? 0.17 * (mb - 200.0) : 0.0));
+    const double tiles = tiles_of(d, 64);
+    const double out   = (double)d->batch * (double)d->m * (double)d->n * 1e-6;
+    const double mb    = out * (d->dequant && d->out_type != MI355_F32 ? 2.0 : 4.0);
+    double one = (d->dequant ? 3.8 : 3.0) + 0.0016 * tiles + 0.25 * out + (mb > 200.0 ? 0.17 * (mb - 200.0) : 0.0);
+    if(!d->dequant && tiles > 4096.0)
+        one = __builtin_fmax(one, 4.6 + tiles * (d->k <= 64 ? 0.0029 : 0.0037));
+    return __builtin_fmin(two, one);
 }
 
 // direct-to-LDS kernels; `shares` of K through a workspace, or added into C
@@ -582,7 +585,10 @@ int choose_kernel(const mi355_quant_dot_desc* d,
         }
         bool atomic      = false;
         const int shares = mi355_dma_gemm_shares(d, c, workspace, workspace_bytes, &atomic);
-        if(ragged_is_faster(d, dma_us(d, shares, atomic), shares > 1 ? 0.1 : 0.07))
+        // results of a short K whose rows are no whole groups of 4 leave these kernels element by element: 2 to 5 times
+        // the register-staged kernel's time (7187 x 24363 x 64 int8 519 us against 254, 14 x 882 x 882 x 64 fp8 46 against 12)
+        const bool broken_rows = d->trans_b && d->k <= 128 && d->n % 4 != 0;
+        if(ragged_is_faster(d, broken_rows ? HUGE_VAL : dma_us(d, shares, atomic), shares > 1 ? 0.1 : 0.07))
             *kernel = kernel_id::ragged;
         else
             *kernel = shares == 1 ? kernel_id::dma : atomic ? kernel_id::dma_atomic : kernel_id::dma_shares;

@@ -127,8 +127,10 @@ def test_one_slab_of_any_bytes(ops, batch, m, n, k):
     _check(ops, batch, m, n, k, True, False)
 
 
-# more tiles than the one-slab kernel takes (of bare results, of any), and so many that are mostly padding otherwise
-@pytest.mark.parametrize("batch,m,n,k", [(1, 4200, 4304, 80), (1, 8200, 8208, 48), (300, 64, 1000, 64), (2, 2900, 2880, 128)])
+# results within one and a half of the last-level cache and beyond (one slab and not; whole lines; mostly padding
+# otherwise; several matrices), rows that are no whole groups of 4
+@pytest.mark.parametrize("batch,m,n,k", [(1, 4200, 4304, 80), (1, 9400, 9500, 48), (1, 9400, 9504, 64), (300, 64, 1000, 64),
+                                         (5, 4300, 4204, 128), (3, 882, 881, 64), (1, 700, 1503, 128)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_short_k_of_many_tiles(ops, batch, m, n, k, fp8):
     _check(ops, batch, m, n, k, True, fp8, cut=_cut(batch, m, n, k, fp8))

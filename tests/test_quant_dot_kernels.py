@@ -107,6 +107,15 @@ def test_one_slab_of_few_rows(batch, m, n, k, fp8, out):
     assert kernel_of(m, n, k, trans_b=True, fp8=fp8, out=out, batch=batch) == "ragged"
 
 
+@pytest.mark.parametrize("batch,m,n,k,out", [(14, 882, 882, 64, "f32"), (1, 3058, 38471, 64, "bf16"), (1, 7187, 24363, 64, None),
+                                             (451, 963, 527, 128, "bf16"), (1, 4447, 29009, 64, None)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_rows_that_are_no_whole_groups_of_4(batch, m, n, k, out, fp8):
+    """Short K: the large tiles store such rows element by element (46 us against 12, 328 / 105, 519 / 254, 654 / 245,
+    398 / 174)"""
+    assert kernel_of(m, n, k, trans_b=True, fp8=fp8, out=out, batch=batch) == "ragged"
+
+
 def test_large_and_small_grids():
     for fp8 in (False, True):
         for out in (None, "bf16", "f32"):
